@@ -47,12 +47,12 @@ struct FactorOut {
   int32_t* info;
 };
 
-// 1 / sqrt(p) in FP64: hardware estimate refined by two Newton steps
-// r <- r (3 - p r^2) / 2 (each step doubles the correct bits).
+// 1 / sqrt(p) in FP64: hardware estimate and one third-order step
+// r <- r (1 + e / 2 + 3 e^2 / 8), e = 1 - p r^2.
 __device__ __forceinline__ double rsqrt_f64(double p) {
-  double r = __builtin_amdgcn_rsq(p);
-  r = r * (1.5 - 0.5 * p * r * r);
-  return r * (1.5 - 0.5 * p * r * r);
+  const double r = __builtin_amdgcn_rsq(p);
+  const double e = fma(-p * r, r, 1.0);
+  return fma(r * e, fma(e, 0.375, 0.5), r);
 }
 
 // Broadcast lane `lane`'s double to the whole wave (through scalar registers).
@@ -62,195 +62,222 @@ __device__ __forceinline__ double bcast(double v, int lane) {
   return __hiloint2double(hi, lo);
 }
 
-// 16x16x16 FP64 MFMA product on LDS operands ([row][65] arrays), one wave:
-// acc(i, j) += sum_k A(ar + i, ac + k) * B(k, j), with B(k, j) = Bm(br + k, bc + j)
-// (bt = 0) or Bm(br + j, bc + k) (bt = 1).  acc[r] holds D(row (l >> 4) + 4r,
-// col l & 15) (lane l).
-__device__ __forceinline__ void mma16(const double (*A)[TILE + 1], int ar, int ac,
-                                      const double (*Bm)[TILE + 1], int br, int bc, int bt,
-                                      doublex4& acc) {
-  const int l = threadIdx.x & 63;
-  const int lr = l & 15, lk = l >> 4;
-#pragma unroll
-  for (int kk = 0; kk < 16; kk += 4) {
-    const double a = A[ar + lr][ac + kk + lk];
-    const double b = bt ? Bm[br + lr][bc + kk + lk] : Bm[br + kk + lk][bc + lr];
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-  }
-}
-// mma16 on row-major LDS arrays of row pitch PA (A) and PB (Bm).
-template <int PA, int PB>
-__device__ __forceinline__ void mma16p(const double* A, int ar, int ac, const double* Bm, int br,
-                                       int bc, int bt, doublex4& acc) {
-  const int l = threadIdx.x & 63;
-  const int lr = l & 15, lk = l >> 4;
-#pragma unroll
-  for (int kk = 0; kk < 16; kk += 4) {
-    const double a = A[(ar + lr) * PA + ac + kk + lk];
-    const double b = bt ? Bm[(br + lr) * PB + bc + kk + lk] : Bm[(br + kk + lk) * PB + bc + lr];
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-  }
-}
-
 // LDS of the diagonal-block factor: the block A ([64][65] doubles) and the
-// four 16x16 diagonal blocks of its inverse ([4][16][17]); the inverse's
-// off-diagonal blocks live, transposed, in A's upper triangle.
-constexpr int XD_PITCH = 17;
-constexpr int XD_BLK = 16 * XD_PITCH;
-constexpr int FACTOR_LDS = (TILE * (TILE + 1) + 4 * XD_BLK) * 8;
+// exchange area of its waves: the finished 16x16 blocks of three row blocks
+// and the next diagonal sub-block, as register images.
+constexpr int FX_BLOCK = 4 * 64;
+constexpr int FX_DOUBLES = 7 * FX_BLOCK;  // two panels' blocks, one sub-block
+constexpr int FACTOR_LDS = (TILE * (TILE + 1) + FX_DOUBLES) * 8;
 
-// Factor the 16-column panel A(o.., o..o+15) of a 64x64 block in place: one
-// wave, lane l holds row o + l (16 values in registers; lanes past the
-// block's last row idle).  Values another row needs travel through scalar
-// registers (readlane), never through LDS; the pivot chain stays short
-// because row j+1's diagonal entry only needs its own row.  The rows below
-// the diagonal sub-block are finished here too, so no inverse is needed on
-// the way.  dval / rinv receive L(o+j, o+j) and its reciprocal square root.
-__device__ __forceinline__ void panel16(double (*A)[TILE + 1], int o, double* dval,
-                                        double* rinv, int32_t* info) {
-  const int l = threadIdx.x & 63;
-  const bool valid = l < TILE - o;
-  double a[16];
-#pragma unroll
-  for (int m = 0; m < 16; ++m) a[m] = valid ? A[o + l][o + m] : 0.0;
-  double myri = 0.0;
-  bool bad = false;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const double p = bcast(a[j], j);
-    const double ri = rsqrt_f64(p);
-    bad |= !(p > 0.0);
-    myri = (l == j) ? ri : myri;
-    const double lj = (l > j) ? a[j] * ri : (l == j ? p * ri : 0.0);
-    a[j] = lj;
-    // a(l, m) -= l(l, j) l(m, j) for the later columns m, the next pivot's
-    // column first
-#pragma unroll
-    for (int m = j + 1; m < 16; ++m) a[m] -= lj * bcast(lj, m);
-  }
-  if (l == 0 && bad && info) atomicOr(info, PGP_INFO_NOT_PD);
-  if (valid) {
-#pragma unroll
-    for (int m = 0; m < 16; ++m)
-      if (m <= l) A[o + l][o + m] = a[m];
-  }
-  if (l < 16) {
-    dval[o + l] = a[l];
-    rinv[o + l] = myri;
-  }
+// 1 / d in FP64: hardware estimate and one third-order step
+// r <- r (1 + e + e^2), e = 1 - d r (three dependent operations, where two
+// Newton steps take four).
+__device__ __forceinline__ double rcp_f64(double d) {
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = fma(-d, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 
-// X(o.., o..) = inverse of the factored 16x16 diagonal sub-block at (o, o)
-// (zero above the diagonal).  One wave; lane c runs forward substitution on
-// column c of I, reading L from LDS (one address per step: a broadcast).
-__device__ __forceinline__ void invert16(const double (*A)[TILE + 1], double* Xb, int o,
-                                         const double* rinv) {
-  const int c = threadIdx.x & 15;
-  double x[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    double acc0 = (r == c) ? 1.0 : 0.0, acc1 = 0.0;
-#pragma unroll
-    for (int k = 0; k + 1 < r; k += 2) {
-      acc0 -= A[o + r][o + k] * x[k];
-      acc1 -= A[o + r][o + k + 1] * x[k + 1];
-    }
-    if (r & 1) acc0 -= A[o + r][o + r - 1] * x[r - 1];
-    x[r] = (acc0 + acc1) * rinv[o + r];
-  }
-  if ((threadIdx.x & 63) < 16) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) Xb[r * XD_PITCH + c] = (r >= c) ? x[r] : 0.0;
-  }
+// v[k]
+__device__ __forceinline__ double pick4(const double (&v)[4], int k) {
+  const double a = (k & 1) ? v[1] : v[0], b = (k & 1) ? v[3] : v[2];
+  return (k & 2) ? b : a;
 }
 
-// Blocked factor + inverse of a 64x64 SPD block held in LDS (`A`, [row][65]).
-// Per 16-wide panel s: one wave factors the panel (panel16), then FP64 MFMA
-// products apply it to the trailing blocks, A_rc -= L_rs L_cs^T.  Then each
-// wave inverts one diagonal sub-block, and the off-diagonal blocks of
-// X = L^-1 follow by block distance: X_rs = -X_rr sum_{k=s}^{r-1} L_rk X_ks.
-// X's diagonal blocks go to Xd ([4][16][17]); X_rs (r > s) is kept
-// transposed in A's upper block (s, r), free once the factor is done, after
-// serving as the scratch of T_rs = sum_k L_rk X_ks.
-// L (lower) goes to global storage as T, X to o.dinv (FP64).
-// `published(...)` runs (all threads) once the inverse's stores are issued,
-// before L's: a caller that hands DINV to other workgroups publishes there.
+// Factor + inverse of a 64x64 SPD block held in LDS (`A`, [row][65], lower
+// triangle read), blocked by 16 columns and, inside, by 4.
+//
+// The 64 rows of L and the 64 rows of Y = L^-T = I L^-T go through the same
+// elimination, 16 rows per wave: in panel s (columns 16 s ..), wave w > s
+// finishes block L_ws and wave w <= s finishes block Y_ws, so every panel
+// gives each of the four waves one 16x16 block, and the inverse comes along
+// with the factor.  A wave's row block stays in registers (R[c]: its block
+// column c) in the transposed MFMA D layout, whose register r holds, at lane
+// l, row l & 15 and column 4 r + (l >> 4): for the symmetric diagonal
+// sub-block that is both D's layout and the layout of a four-column MFMA
+// operand, so a rank-4 update needs no data movement.  Every wave eliminates
+// the panel's diagonal sub-block S itself (redundantly: the pivots never
+// cross waves), four columns at a time: the 4x4 pivot block is read through
+// readlane and eliminated as L4 D L4^T in every lane (one reciprocal per
+// pivot on the chain; square roots after it), an MFMA each applies L4^-T to
+// the four columns of S and of the wave's block, and one each updates the
+// rest.  After a panel the waves
+// swap their finished blocks through LDS and update the next panel's columns;
+// the later columns' update runs inside the next panel, beside its chain.
+//
+// Bound: the serial chain of 64 pivots in one workgroup.  A 16-column panel
+// by one wave with the pivots and column values through readlane (about 125
+// ns per pivot), then the inverse after the factor, took 14.1-14.6 us per
+// block; this form takes 8.9 us, 8.2 to the inverse's stores (one workgroup
+// alone; a four-column step is about 0.32 us).
+//
+// L (lower) goes to global storage as T, the inverse to o.dinv (FP64).  In
+// LDS, L takes A's strict lower triangle and Y its strict upper one (the
+// diagonals are dval and rinv).  `published(...)` runs (all threads) once
+// the inverse's stores are issued, before L's: a caller that hands DINV to
+// other workgroups publishes there.
 struct NoPublish {
   __device__ void operator()() const {}
 };
 template <typename T, typename Pub = NoPublish>
-__device__ __forceinline__ void factor_block_blocked(double (*A)[TILE + 1], double* Xd, int64_t r0,
+__device__ __forceinline__ void factor_block_blocked(double (*A)[TILE + 1], double* fx, int64_t r0,
                                      const FactorOut& o, Pub published = Pub()) {
   __shared__ double dval[TILE], rinv[TILE];
   const int t = threadIdx.x;
-  const int wv = t >> 6, l = t & 63;
-  const int orow = l >> 4, ocol = l & 15;  // D layout: row orow + 4r, col ocol
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const unsigned ul = t & 63;
+  const int l = (int)ul;
+  const int row = l & 15, kq = l >> 4;
+  double* sbuf = fx + 6 * FX_BLOCK;
   __builtin_amdgcn_s_setprio(3);
+  // entries above the diagonal of S reach only its finished rows and columns
+  doublex4 R[4], S;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) S[r] = A[row][4 * r + kq];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) R[c][r] = c <= w ? A[16 * w + row][16 * c + 4 * r + kq] : 0.0;
+  double e[4];  // column kq of the 4x4 identity
+#pragma unroll
+  for (int q = 0; q < 4; ++q) e[q] = q == kq ? 1.0 : 0.0;
+  __syncthreads();  // A is in registers: L and Y take its place
+  double lp[4], fp[4][4];  // the previous panel's block and L blocks
+#pragma unroll
   for (int s = 0; s < 4; ++s) {
     const int o16 = 16 * s;
-    if (wv == 0) panel16(A, o16, dval, rinv, o.info);
+    double* fs = fx + 3 * FX_BLOCK * (s & 1);
+    if (s > 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[r] = sbuf[64 * r + l];
+    }
+    doublex4 B = R[s];
+    if (w == s) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) B[r] = row == 4 * r + kq ? 1.0 : 0.0;
+    }
+    // the wave's finished block and the diagonal one, operand layout; 1 / sqrt(d)
+    double lb[4], ls[4], rs[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int p0 = 4 * r;
+      // the 4x4 pivot block (lane 16 b + p0 + a: row p0 + a, column p0 + b)
+      auto piv = [&](int a, int b) { return bcast(S[r], 16 * b + p0 + a); };
+      const double s10 = piv(1, 0), s20 = piv(2, 0), s30 = piv(3, 0);
+      double s21 = piv(2, 1), s31 = piv(3, 1), s32 = piv(3, 2);
+      double d[4] = {piv(0, 0), piv(1, 1), piv(2, 2), piv(3, 3)};
+      // the previous panel's update of the columns after the next panel runs
+      // beside the pivots' chain
+#pragma unroll
+      for (int c = s + 1; c < 4; ++c)
+        if (s > 0) R[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(fp[c][r], lp[r], R[c], 0, 0, 0);
+      // (products of column entries are formed beside the reciprocals)
+      const double r0 = rcp_f64(d[0]);
+      d[1] = fma(-(s10 * s10), r0, d[1]);
+      d[2] = fma(-(s20 * s20), r0, d[2]);
+      d[3] = fma(-(s30 * s30), r0, d[3]);
+      s21 = fma(-(s20 * s10), r0, s21);
+      s31 = fma(-(s30 * s10), r0, s31);
+      s32 = fma(-(s30 * s20), r0, s32);
+      const double r1 = rcp_f64(d[1]);
+      d[2] = fma(-(s21 * s21), r1, d[2]);
+      d[3] = fma(-(s31 * s31), r1, d[3]);
+      s32 = fma(-(s31 * s21), r1, s32);
+      const double r2 = rcp_f64(d[2]);
+      d[3] = fma(-(s32 * s32), r2, d[3]);
+      const double l10 = s10 * r0, l20 = s20 * r0, l30 = s30 * r0;
+      const double l21 = s21 * r1, l31 = s31 * r1, l32 = s32 * r2;
+      // X = (the four columns) L4^-T = L D, as X^T = L4^-1 (columns)^T: one
+      // 4x4x4 MFMA for the four blocks of four rows, whose result is in the
+      // operand layout again.  Lane l brings L4^-1(l & 3, l >> 4).
+      double y[4];
+      y[0] = e[0];
+      y[1] = fma(-l10, e[0], e[1]);
+      y[2] = fma(-l21, y[1], fma(-l20, e[0], e[2]));
+      y[3] = fma(-l32, y[2], fma(-l31, y[1], fma(-l30, e[0], e[3])));
+      const double inv4 = pick4(y, l & 3);
+      const double xs = __builtin_amdgcn_mfma_f64_4x4x4f64(inv4, S[r], 0.0, 0, 0, 0);
+      const double xb = __builtin_amdgcn_mfma_f64_4x4x4f64(inv4, B[r], 0.0, 0, 0, 0);
+      rs[r] = rsqrt_f64(pick4(d, kq));
+      ls[r] = xs * rs[r];
+      lb[r] = xb * rs[r];
+      if (r < 3) {
+        S = __builtin_amdgcn_mfma_f64_16x16x4f64(-ls[r], ls[r], S, 0, 0, 0);
+        B = __builtin_amdgcn_mfma_f64_16x16x4f64(-ls[r], lb[r], B, 0, 0, 0);
+        // both in flight before the next step: B's would otherwise be
+        // scheduled late and hold up that step's MFMAs
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (w > s) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) fs[(w - 1) * FX_BLOCK + 64 * r + l] = -lb[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int cl = 4 * r + kq;  // column inside the panel
+      if (w != s) {
+        A[16 * w + row][o16 + cl] = lb[r];
+      } else {
+        A[o16 + row][o16 + cl] = cl > row ? lb[r] : ls[r];
+        if (row == cl) {
+          dval[o16 + row] = ls[r];
+          rinv[o16 + row] = rs[r];
+        }
+      }
+    }
     __syncthreads();
     if (s == 3) break;
-    const int nrb = 3 - s;
-    // trailing blocks (r, c), s < c <= r: A_rc -= L_rs L_cs^T
-    for (int b = wv; b < nrb * (nrb + 1) / 2; b += 4) {
-      int rr = 0;
-      while ((rr + 1) * (rr + 2) / 2 <= b) ++rr;
-      const int cc = b - rr * (rr + 1) / 2;
-      const int r = s + 1 + rr, c = s + 1 + cc;
-      doublex4 acc = {0.0, 0.0, 0.0, 0.0};
-      mma16(A, 16 * r, o16, A, 16 * c, o16, 1, acc);
+    // the wave's later block columns, R_wc -= (its block) L_cs^T: the next
+    // panel's at once, the others beside that panel (in rows of L only
+    // columns up to the wave's own exist; L_cs = 0 keeps the others zero)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) A[16 * r + orow + 4 * q][16 * c + ocol] -= acc[q];
+    for (int c = s + 1; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        fp[c][r] = (w <= s || c <= w) ? fs[(c - 1) * FX_BLOCK + 64 * r + l] : 0.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      lp[r] = lb[r];
+      R[s + 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(fp[s + 1][r], lb[r], R[s + 1], 0, 0, 0);
+    }
+    if (w == s + 1) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sbuf[64 * r + l] = R[s + 1][r];
     }
     __syncthreads();
   }
-  invert16(A, Xd + wv * XD_BLK, 16 * wv, rinv);
-  __syncthreads();
-  // off-diagonal blocks of X by distance d; T goes to A's upper block (s, r)
-  // and is replaced there by X_rs transposed: X_ks (k > s) is read back as
-  // B(kk, j) = A(16 s + j, 16 k + kk)
-  const double* Af = &A[0][0];
-  for (int d = 1; d < 4; ++d) {
-    const int nblk = 4 - d;
-    if (wv < nblk) {
-      const int r = d + wv, s = wv;
-      doublex4 acc = {0.0, 0.0, 0.0, 0.0};
-      mma16p<TILE + 1, XD_PITCH>(Af, 16 * r, 16 * s, Xd + s * XD_BLK, 0, 0, 0, acc);
-      for (int k = s + 1; k < r; ++k)
-        mma16p<TILE + 1, TILE + 1>(Af, 16 * r, 16 * k, Af, 16 * s, 16 * k, 1, acc);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) A[16 * s + orow + 4 * q][16 * r + ocol] = acc[q];
-    }
-    __syncthreads();
-    if (wv < nblk) {
-      const int r = d + wv, s = wv;
-      doublex4 acc = {0.0, 0.0, 0.0, 0.0};
-      mma16p<XD_PITCH, TILE + 1>(Xd + r * XD_BLK, 0, 0, Af, 16 * s, 16 * r, 0, acc);
-      // (the product has read all of T_rs before its result exists)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) A[16 * s + ocol][16 * r + orow + 4 * q] = -acc[q];
-    }
-    __syncthreads();
-  }
+  // a pivot that was not positive left no positive sqrt(d) (NaN)
+  if (t < TILE && !(dval[t] > 0.0) && o.info) atomicOr(o.info, PGP_INFO_NOT_PD);
   __builtin_amdgcn_s_setprio(0);
-  for (int e = t; e < TILE * TILE; e += NTHREADS) {
-    const int c = e / TILE, r = e % TILE;  // column-major walk: coalesced stores
-    double v = 0.0;
-    if (c <= r)
-      v = (r >> 4) == (c >> 4) ? Xd[(r >> 4) * XD_BLK + (r & 15) * XD_PITCH + (c & 15)] : A[c][r];
-    // coherent: the column kernels hand DINV to other workgroups
-    st_coherent(&o.dinv[r + c * TILE], v);
+  // columns w + 4q, one row per lane: whole columns per store
+  {
+    double v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = A[w + 4 * q][l];
+    const double dg = rinv[l];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int c = w + 4 * q;
+      // coherent: the column kernels hand DINV to other workgroups
+      __hip_atomic_store(gbl(o.dinv) + c * TILE + ul, c < l ? v[q] : c == l ? dg : 0.0,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   published();
   if (t < TILE) {
     if (o.logdiag) o.logdiag[t] = log(dval[t]);
     if (o.diagval) o.diagval[t] = dval[t];
   }
-  T* L = (T*)o.L;
-  for (int e = t; e < TILE * TILE; e += NTHREADS) {
-    const int c = e / TILE, r = e % TILE;
-    if (c <= r) L[(size_t)(r0 + r) + (size_t)(r0 + c) * o.ld] = (T)A[r][c];
+  const auto L = gbl((T*)o.L) + r0 + r0 * o.ld;
+  double v[16];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) v[q] = A[l][w + 4 * q];
+  const double dg = dval[l];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int c = w + 4 * q;
+    if (c <= l) (L + c * o.ld)[ul] = (T)(c == l ? dg : v[q]);
   }
 }
 
@@ -258,7 +285,7 @@ __device__ __forceinline__ void factor_block_blocked(double (*A)[TILE + 1], doub
 template <typename T>
 __device__ void factor_first(const T* A, int64_t ld, const FactorOut& o) {
   __shared__ double blk[TILE][TILE + 1];
-  __shared__ double xd[4 * XD_BLK];
+  __shared__ double xd[FX_DOUBLES];
   const int m = threadIdx.x & 63, kb = threadIdx.x >> 6;
   for (int q = 0; q < 16; ++q) {
     const int c = kb + 4 * q;
@@ -836,68 +863,65 @@ __global__ __launch_bounds__(NTHREADS) void k_column(Prob* const* probs, Sched r
         L[(size_t)(ri + acc_row<T>(bm, r)) + (size_t)(c0 + acc_col(bn)) * P.Np] = acc[bm][bn][r];
 }
 
-// ---- column-form super-step in two launches ----------------------------------
-// Phase A (k_superstep): the tiles (i, j) of the super-step's columns
-// [s0, s1) with row block i < rlim (the super-step's diagonal block of
-// tiles when rlim = s0 + G) in one launch, each tile one workgroup, in
-// lookahead ticket order (StepSched).  A workgroup applies the left-looking
-// update by the columns s0..j-1 as k_column does, fetching those columns'
-// tiles -- written in this launch -- with coherent loads once their flags
-// show them final; a diagonal workgroup then factors and inverts block j, a
-// row workgroup waits for that and forms L_ij = C_ij DINV_j^T.  Each tile's
-// flag is published after its stores complete.  The chain from one column to
-// the next is tile (j+1, j) -> block j+1, so a column's factor overlaps the
-// previous column's remaining rows, and the G - 1 launch gaps of the
-// per-column form go away.  Phase B (k_panel_rows) takes the rows below,
-// i >= rlim: one workgroup per row block, which forms its tiles (i, s0),
-// (i, s0 + 1), ... in order from its own earlier tiles and phase A's
-// (launch-ordered, so plain cached loads and no waits).  Same operations in
-// the same order on every tile as k_column: the factor is bitwise the same.
+// ---- column-form super-step in one launch ------------------------------------
+// The tiles (i, j), j <= i < rlim, of the super-step's columns [s0, s1) in one
+// launch: one workgroup per row block i of every member, which forms its
+// tiles (i, s0), (i, s0 + 1), ... from left to right and, for a row block of
+// the super-step itself, then factors and inverts its diagonal block.  For a
+// tile it accumulates sum_{c in [s0, j)} L_ic L_jc^T from its own earlier
+// tiles and row block j's (published in this launch: coherent loads once
+// their flags show them final), waits for block j's inverse and multiplies:
+// L_ij = C_ij DINV_j^T.  A row block of the super-step also accumulates its
+// diagonal tile's update on the way, so the chain from one block column to
+// the next is DINV_{i-1} -> L_{i,i-1} (in LDS) -> update of tile (i, i) ->
+// factor -> DINV_i: one hand-off between workgroups per column.  With the
+// super-step's rows s0..s1-1 cut off by rlim = s1 the rows below are left to
+// k_panel_rows.  Same operations in the same order on every tile as
+// k_column: the factor is bitwise the same.
+//
+// Bound: that chain.  With a workgroup per tile a block column took two
+// hand-offs through memory and 33 us (FP64) / 29 us (FP32) of a lone N = 512
+// factor; with one per row block 14.3 us (FP32) and 18 us (FP64, to 29 us in
+// the last columns of 8, where the left-looking products are the longer
+// side): 287 -> 164 us and 217 -> 114 us for the eight columns.
 //
 // Member sync words (Prob::csync, zeroed when the descriptor is written with
-// reset): flag (i, c) at csync[(c - s0) nb + i] holds the launch's epoch
-// once tile (i, c) is final; csync[16 nb] counts the member's finished
-// workgroups.  The member's last workgroup resets the count and clears the
-// flags, so no flag outlives its launch (a replayed graph of the launch,
-// whose epoch is the captured one, starts from cleared flags).
+// reset): flag (i, c) at csync[(c - s0) MAXG + i - s0] holds the launch's
+// epoch once tile (i, c), i < s1, is final (c = i: DINV_i); csync[16 nb]
+// counts the member's finished workgroups.  The member's last workgroup
+// resets the count and clears the flags, so no flag outlives its launch (a
+// replayed graph of the launch, whose epoch is the captured one, starts from
+// cleared flags).
 constexpr int MAXG = 16;
-// Tickets run in groups k = s0 .. s1 (lookahead order): group k holds the
-// diagonal workgroups D(k) of every member, then the rows i >= k + 1 of
-// column k - 1 (B(k - 1)), then tile (k + 1, k) (the one block k + 1 needs
-// from column k).  So the chain D(k) -> (k + 1, k) -> D(k + 1) is ticketed
-// ahead of the bulk of each column, whose workgroups start once their
-// diagonal block is (nearly) done instead of holding a slot while they
-// wait; every dependency is on a lower ticket.
+// Tickets: the row blocks s0, s0 + 1, ... of the super-step, each for every
+// member that has it, then the rows below, member after member; a workgroup
+// waits only for row blocks of its member above its own, on lower tickets.
 struct StepSched {
   int32_t count;             // members (sorted by size, descending)
   int32_t s0, s1;            // columns [s0, s1)
-  int32_t rlim;              // row blocks [j, min(nb, rlim)) of each column j
-  int32_t gbase[MAXG + 2];   // first ticket of group s0 + g
-  int32_t nd[MAXG + 1];      // D(k): members with more than k block columns
-  int32_t nB[MAXG + 1];      // members with min(nb, rlim) > k + 1 (B(k - 1) and tile (k + 1, k))
-  int32_t nbk[MAXG + 1];     // workgroups of B(k - 1)
-  int32_t pre[MAXB + 1];     // pre[m]: sum of min(nb, rlim) over the members before m
+  int32_t rlim;              // row blocks [s0, min(nb, rlim))
+  int32_t gbase[MAXG + 1];   // first ticket of row block s0 + g; [s1 - s0]: of the rows below
+  int32_t pre[MAXB + 1];     // rows below (i >= s1) of the members before m
 };
 
-__device__ __forceinline__ uint32_t* tile_flag(const Prob& P, int nb, int s0, int i, int c) {
-  return P.csync + (size_t)(c - s0) * nb + i;
+__device__ __forceinline__ uint32_t* tile_flag(uint32_t* csync, int s0, int i, int c) {
+  return csync + (c - s0) * MAXG + (i - s0);
 }
 
-// Wave 0 waits (bounded, one flag per lane) until the flags of tiles (i, c)
-// and (j, c), c in [ca, cb), equal `epoch`; then the workgroup proceeds.
-// All threads call it.
-__device__ __forceinline__ void wait_tiles(const Prob& P, int nb, int s0, int i, int j, int ca,
+// Wave 0 waits (bounded, one flag per lane) until the flags of tiles (j, c),
+// c in [ca, cb), equal `epoch`; then the workgroup proceeds.  All threads
+// call it.
+__device__ __forceinline__ void wait_tiles(uint32_t* csync, int32_t* info, int s0, int j, int ca,
                                            int cb, uint32_t epoch) {
   if (threadIdx.x < 64) {
     const int l = threadIdx.x;
-    const int n = 2 * (cb - ca);
-    const uint32_t* f = l < n ? tile_flag(P, nb, s0, (l & 1) ? j : i, ca + (l >> 1)) : nullptr;
+    const uint32_t* f = l < cb - ca ? tile_flag(csync, s0, j, ca + l) : nullptr;
     for (int spins = 0;; ++spins) {
       const bool ok =
           !f || __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == epoch;
       if (__builtin_amdgcn_ballot_w64(!ok) == 0) break;
       if (spins >= SPIN_LIMIT) {
-        if (l == 0) atomicOr(P.info, PGP_INFO_STALLED);
+        if (l == 0) atomicOr(info, PGP_INFO_STALLED);
         break;
       }
       __builtin_amdgcn_s_sleep(1);
@@ -907,118 +931,260 @@ __device__ __forceinline__ void wait_tiles(const Prob& P, int nb, int s0, int i,
   __syncthreads();
 }
 
+// The thread's 16 operand values v (row m, the k indices operand_k<CK>(kb, q))
+// into an operand buffer of the trailing updates' form.
+template <typename T, int BF16, typename LT>
+__device__ __forceinline__ void stash_operand(LT* d, const T (&v)[16], int m, int kb) {
+  constexpr bool MM = MmajorF32<T, BF16>::value;
+  if constexpr (BF16) {
+    stash_bf16_mmajor(d, 72, v, m, kb);
+  } else if constexpr (MM) {
+    stash_f32_mmajor(d, 68, v, m, kb);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) d[(kb + 4 * q) * KP<T>::value + m] = v[q];
+  }
+}
+template <typename T, int BF16, typename LT>
+__device__ __forceinline__ void mma_operands(const LT* a, const LT* b,
+                                             typename Acc<T>::type (&acc)[2][2]) {
+  if constexpr (BF16)
+    mma64_bf16(a, 72, b, 72, acc);
+  else if constexpr (MmajorF32<T, BF16>::value)
+    mma64_f32_mmajor(a, 68, b, 68, acc);
+  else
+    mma64_kmajor<T>(a, KP<T>::value, b, KP<T>::value, acc);
+}
+
+// LDS of the super-step kernel: the panel product's two operands and the
+// updates' two, or the diagonal factor's block.
 template <typename T, int BF16>
-__global__ __launch_bounds__(NTHREADS) void k_superstep(Prob* const* probs, StepSched ss,
+struct StepArena {
+  static constexpr int OPER = TILE * (BF16 ? 72 : MmajorF32<T, BF16>::value ? 68 : KP<T>::value);
+  static constexpr int all = 2 * TILE * KP<T>::value * (int)sizeof(T) +
+                             2 * OPER * (BF16 ? 2 : (int)sizeof(T));
+  static constexpr int bytes = all > FACTOR_LDS ? all : FACTOR_LDS;
+};
+
+template <typename T, int BF16>
+__global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(Prob* const* probs, StepSched ss,
                                                         uint32_t* ticket, uint32_t epoch) {
-  __shared__ __attribute__((aligned(16))) char arena_b[col_arena_bytes<T, BF16>()];
-  double (*arena)[TILE + 1] = (double (*)[TILE + 1])arena_b;
-  double* xd = (double*)arena_b + TILE * (TILE + 1);
+  __shared__ __attribute__((aligned(16))) char arena[StepArena<T, BF16>::bytes];
   __shared__ int s_val;
   const int t = take_ticket(ticket, &s_val);
   if ((unsigned)t >= gridDim.x) {  // counter not zero at launch: nothing to take
     flag_members_stalled(probs, ss.count);
     return;
   }
-  // ticket -> (member mi, row block i, column j)
-  int g = 0;
-  while (t >= ss.gbase[g + 1]) ++g;
-  const int s0 = ss.s0, k = s0 + g;
-  int q = t - ss.gbase[g];
-  int mi, i, j;
-  if (q < ss.nd[g]) {  // D(k)
-    mi = q;
-    i = j = k;
-  } else if ((q -= ss.nd[g]) < ss.nbk[g]) {
-    // B(k - 1): member m has min(nb_m, rlim) - k - 1 rows, so the members
-    // before m hold pre[m] - (k + 1) m of them
-    int lo = 0, hi = ss.nB[g];
+  // ticket -> (member mi, row block i)
+  const int s0 = ss.s0, s1 = ss.s1;
+  int mi, i;
+  if (t < ss.gbase[s1 - s0]) {
+    int g = 0;
+    while (t >= ss.gbase[g + 1]) ++g;
+    mi = t - ss.gbase[g];
+    i = s0 + g;
+  } else {
+    const int u = t - ss.gbase[s1 - s0];
+    int lo = 0, hi = ss.count;
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
-      if (ss.pre[mid] - (k + 1) * mid <= q)
+      if (ss.pre[mid] <= u)
         lo = mid;
       else
         hi = mid;
     }
     mi = lo;
-    i = k + 1 + (q - (ss.pre[lo] - (k + 1) * lo));
-    j = k - 1;
-  } else {  // tile (k + 1, k)
-    mi = q - ss.nbk[g];
-    i = k + 1;
-    j = k;
+    i = s1 + u - ss.pre[lo];
   }
-  const Prob& P = *probs[mi];
-  const int nb = P.Np / TILE;
-  const int64_t c0 = (int64_t)j * TILE, ri = (int64_t)i * TILE;
-  // the columns before the last are normally final long before: one wait
-  // for all of them, then column j - 1's tiles right before they are fetched
-  if (j - 1 > s0) wait_tiles(P, nb, s0, i, j, s0, j - 1, epoch);
-  auto last_col = [&](int c) {
-    if (c == j - 1) wait_tiles(P, nb, s0, i, j, c, c + 1, epoch);
+  const Prob& P = *uniform(probs[mi]);
+  const int nb = uniform(P.Np) / TILE;
+  int64_t ld = (int64_t)nb * TILE;
+  const int64_t ri = (int64_t)i * TILE;
+  T* const Lp = (T*)uniform((char*)P.L);
+  double* const dinv = uniform(P.dinv);
+  double* const logdiag = uniform(P.logdiag);
+  double* const diagval = uniform(P.diagval);
+  uint32_t* const csync = uniform(P.csync);
+  int32_t* const info = uniform(P.info);
+  const bool diag = i < s1;  // this row block factors its diagonal block
+  constexpr bool CK = MmajorF32<T, BF16>::value || BF16;
+  typedef typename std::conditional<BF16 != 0, unsigned short, T>::type LT;
+  typedef typename Acc<T>::type acc_t;
+  constexpr int PP = KP<T>::value;
+  T* ck = (T*)arena;  // panel product operands: C_ij and DINV_j
+  T* bk = ck + TILE * PP;
+  LT* sa = (LT*)(bk + TILE * PP);  // update operands
+  LT* sb = sa + StepArena<T, BF16>::OPER;
+  // the wave index as a scalar: column addresses stay in scalar registers
+  const unsigned m = threadIdx.x & 63;
+  const int kb = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const auto A = gbl(Lp);
+  // the wave's 16 columns of the tile at (r0, c0): every fourth one, or
+  // (operands) its columns operand_k<CK>
+  auto col4 = [&](int64_t r0, int64_t c0) { return A + (r0 + (c0 + kb) * ld); };
+  auto colk = [&](int64_t r0, int64_t c0) { return A + (r0 + (c0 + operand_k<CK>(kb, 0)) * ld); };
+  constexpr int KS = CK ? 1 : 4;
+  // acc: update of the current (then the next) tile; accd: of the diagonal tile
+  acc_t acc[2][2], accd[2][2], prod[2][2];
+  zero_acc<T>(acc);
+  zero_acc<T>(accd);
+  T av[16], ra[2][16], rb[2][16];
+  auto load_a = [&](int64_t c0) {
+    auto p = col4(ri, c0);
+#pragma unroll
+    for (int q = 0; q < 16; ++q, p += 4 * ld) av[q] = p[m];
   };
-  if (i == j) {
-    update_tile_to_lds<T, BF16, double, true, true>((const T*)P.L, P.Np, s0, j, c0, c0,
-                                                    (char*)arena, &arena[0][0], TILE + 1,
-                                                    false, last_col);
-    FactorOut o{P.L, P.Np, P.dinv + (size_t)j * TILE * TILE,
-                P.logdiag ? P.logdiag + c0 : nullptr, P.diagval ? P.diagval + c0 : nullptr,
-                P.info};
-    // block j's rows wait only for DINV_j: publish before L_jj is stored
-    factor_block_blocked<T>(arena, xd, c0, o, [&]() {
-      publish_wait();
+  // row block j's tile (j, c), published in this launch
+  auto load_rb = [&](T (&v)[16], int j, int c) {
+    auto p = colk((int64_t)j * TILE, (int64_t)c * TILE);
+#pragma unroll
+    for (int q = 0; q < 16; ++q, p += KS * ld) v[q] = ld_coh(p + m);
+  };
+  // k-major LDS image of a D-layout tile
+  auto to_lds = [&](T* d, const acc_t (&v)[2][2]) {
+#pragma unroll
+    for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[acc_col(bn) * PP + acc_row<T>(bm, r)] = (T)v[bm][bn][r];
+  };
+  const int jend = min(i, s1);
+  load_a((int64_t)(jend > s0 ? s0 : i) * TILE);
+  for (int j = s0; j < jend; ++j) {
+    asm volatile("" : "+s"(ld));  // column addresses are formed where they are used
+    const int64_t c0 = (int64_t)j * TILE;
+    const bool next = j + 1 < jend;
+    // C_ij = A_ij - acc
+    if (j > s0) {
+      to_lds(ck, acc);
       __syncthreads();
-      if (threadIdx.x == 0)
-        __hip_atomic_store(tile_flag(P, nb, s0, j, j), epoch, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    });
-  } else {
-    constexpr int PP = KP<T>::value;
-    T* ck = (T*)&arena[0][0];
-    T* bk = ck + TILE * PP;
-    update_tile_to_lds<T, BF16, T, false, true>((const T*)P.L, P.Np, s0, j, ri, c0, (char*)arena,
-                                                ck, PP, true, last_col);
-    wait_tiles(P, nb, s0, j, j, j, j + 1, epoch);  // block j factored, DINV_j published
-    const double* Dj = P.dinv + (size_t)j * TILE * TILE;
-    {
-      const int n = threadIdx.x & 63, pb = threadIdx.x >> 6;
-      for (int qq = 0; qq < 16; ++qq) {
-        const int pp = pb + 4 * qq;
-        bk[pp * PP + n] = (T)ld_coherent(&Dj[n + pp * TILE]);
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      T* p = &ck[(kb + 4 * q) * PP + m];
+      *p = j > s0 ? av[q] - *p : av[q];
+    }
+    // while block j is factored: the next tile's update by the columns
+    // before j (own tiles: complete, see below), two columns ahead in flight
+    zero_acc<T>(acc);
+    if (next && j > s0) {
+      wait_tiles(csync, info, s0, j + 1, s0, j, epoch);
+      auto fetch = [&](int c, T (&a)[16], T (&b)[16]) {
+        auto p = colk(ri, (int64_t)c * TILE);
+#pragma unroll
+        for (int q = 0; q < 16; ++q, p += KS * ld) a[q] = p[m];
+        load_rb(b, j + 1, c);
+      };
+      auto chunk = [&](int c, T (&a)[16], T (&b)[16]) {
+        __syncthreads();  // the previous products are done with LDS
+        stash_operand<T, BF16>(sa, a, m, kb);
+        stash_operand<T, BF16>(sb, b, m, kb);
+        __syncthreads();
+        if (c + 2 < j) fetch(c + 2, a, b);
+        mma_operands<T, BF16>(sa, sb, acc);
+      };
+      fetch(s0, ra[0], rb[0]);
+      if (s0 + 1 < j) fetch(s0 + 1, ra[1], rb[1]);
+      for (int c = s0; c < j; c += 2) {
+        chunk(c, ra[0], rb[0]);
+        if (c + 1 < j) chunk(c + 1, ra[1], rb[1]);
       }
     }
+    wait_tiles(csync, info, s0, j, j, j + 1, epoch);  // block j factored, DINV_j published
+    {
+      const auto Dj = gbl((const double*)dinv + (size_t)j * TILE * TILE);
+      double dv[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) dv[q] = ld_coh(Dj + (kb + 4 * q) * TILE + m);
+      __builtin_amdgcn_sched_barrier(0);  // every load issued before the first is used
+#pragma unroll
+      for (int q = 0; q < 16; ++q) bk[(kb + 4 * q) * PP + m] = (T)dv[q];
+    }
     __syncthreads();
-    typename Acc<T>::type acc[2][2];
-    zero_acc<T>(acc);
-    mma64_kmajor<T>(ck, PP, bk, PP, acc);
-    T* L = (T*)P.L;
+    zero_acc<T>(prod);
+    mma64_kmajor<T>(ck, PP, bk, PP, prod);
+    __syncthreads();
+    // L_ij through LDS: whole columns per store, and the operand of the
+    // following updates
+    to_lds(ck, prod);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) ra[0][q] = ck[operand_k<CK>(kb, q) * PP + m];
+    {
+      auto p = colk(ri, c0);
+      if (diag) {
+#pragma unroll
+        for (int q = 0; q < 16; ++q, p += KS * ld)
+          __hip_atomic_store(p + m, ra[0][q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 16; ++q, p += KS * ld) p[m] = ra[0][q];
+      }
+    }
+    if (next || diag) {
+      load_a(c0 + TILE);  // the next tile (the diagonal one after the last)
+      stash_operand<T, BF16>(sa, ra[0], m, kb);
+      __syncthreads();
+      if (diag) mma_operands<T, BF16>(sa, sa, accd);
+    }
+    // every wave's stores complete: publish the tile (and read it back as an
+    // operand of the next columns)
+    publish_wait();
+    __syncthreads();
+    if (diag && threadIdx.x == 0)
+      __hip_atomic_store(tile_flag(csync, s0, i, j), epoch, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    if (next) {
+      // column j's part of the next tile's update
+      wait_tiles(csync, info, s0, j + 1, j, j + 1, epoch);
+      load_rb(rb[0], j + 1, j);
+      stash_operand<T, BF16>(sb, rb[0], m, kb);
+      __syncthreads();
+      mma_operands<T, BF16>(sa, sb, acc);
+    }
+  }
+  if (diag) {
+    __syncthreads();
+    double (*blk)[TILE + 1] = (double (*)[TILE + 1])arena;
 #pragma unroll
     for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
       for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          st_coh(&L[(size_t)(ri + acc_row<T>(bm, r)) + (size_t)(c0 + acc_col(bn)) * P.Np],
-                 (T)acc[bm][bn][r]);
+          blk[acc_row<T>(bm, r)][acc_col(bn)] = (double)(T)accd[bm][bn][r];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      double* p = &blk[m][kb + 4 * q];
+      *p = (double)(av[q] - (T)*p);
+    }
+    __syncthreads();
+    FactorOut o{Lp, ld, dinv + (size_t)i * TILE * TILE, logdiag ? logdiag + ri : nullptr,
+                diagval ? diagval + ri : nullptr, info};
+    // the rows below wait only for DINV_i: publish before L_ii is stored
+    factor_block_blocked<T>(blk, (double*)(blk + TILE), ri, o, [&]() {
+      publish_wait();
+      __syncthreads();
+      if (threadIdx.x == 0)
+        __hip_atomic_store(tile_flag(csync, s0, i, i), epoch, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    });
   }
-  // every wave's stores complete, then publish the tile
-  publish_wait();
-  __syncthreads();
+  // the member's last workgroup in this launch clears its sync words
   if (threadIdx.x == 0) {
-    __hip_atomic_store(tile_flag(P, nb, s0, i, j), epoch, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    // the member's last workgroup in this launch clears its sync words
-    const int e = min(ss.s1, nb), nbr = min(nb, ss.rlim);
-    const uint32_t total = (uint32_t)((e - s0) * nbr - (s0 + e - 1) * (e - s0) / 2);
-    uint32_t* done = P.csync + (size_t)MAXG * nb;
-    s_val = (atomicAdd(done, 1u) + 1u == total) ? 1 : 0;
+    const uint32_t total = (uint32_t)(min(nb, ss.rlim) - s0);
+    s_val = (atomicAdd(csync + (size_t)16 * nb, 1u) + 1u == total) ? 1 : 0;
   }
   __syncthreads();
   if (s_val) {
-    const int e = min(ss.s1, nb);
-    for (int w = threadIdx.x; w < (e - s0) * nb; w += NTHREADS)
-      __hip_atomic_store(P.csync + w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int e = min(s1, nb) - s0;
+    for (int w = threadIdx.x; w < e * MAXG; w += NTHREADS)
+      if (w % MAXG < e) __hip_atomic_store(csync + w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (threadIdx.x == 0)
-      __hip_atomic_store(P.csync + (size_t)MAXG * nb, 0u, __ATOMIC_RELAXED,
+      __hip_atomic_store(csync + (size_t)16 * nb, 0u, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
   }
 }
@@ -1032,7 +1198,7 @@ __global__ __launch_bounds__(NTHREADS) void k_factor_diag(Prob* const* probs, Sc
   const int64_t c0 = (int64_t)k * TILE;
   if (c0 >= P.Np) return;
   __shared__ double blk[TILE][TILE + 1];
-  __shared__ double xd[4 * XD_BLK];
+  __shared__ double xd[FX_DOUBLES];
   const T* A = (const T*)P.L;
   const int m = threadIdx.x & 63, kb = threadIdx.x >> 6;
   for (int q = 0; q < 16; ++q) {
@@ -1283,33 +1449,23 @@ static void superstep_launch(const Batch& b, int s0, int s1, int rlim, bool tpa,
     ss.s0 = s0;
     ss.s1 = s1;
     ss.rlim = rlim;
-    ss.pre[0] = 0;
-    for (int m = 0; m < n; ++m) ss.pre[m + 1] = ss.pre[m] + std::min(b.np(off + m) / TILE, rlim);
     double fl = 0.0;
+    ss.pre[0] = 0;
     for (int m = 0; m < n; ++m) {
       const int nbm = b.np(off + m) / TILE, nbr = std::min(nbm, rlim);
+      ss.pre[m + 1] = ss.pre[m] + std::max(0, nbr - s1);
       for (int j = s0; j < std::min(s1, nbm); ++j)
         fl += F3 + (double)(nbr - j) * G64 * (j - s0) + (double)(nbr - j - 1) * G64;
     }
     const int ncols = s1 - s0;
     ss.gbase[0] = 0;
-    for (int g = 0; g <= ncols; ++g) {
-      const int k = s0 + g;
-      int nd = 0, nB = 0, nbk = 0;
-      for (int m = 0; m < n; ++m) {
-        const int nbm = b.np(off + m) / TILE, nbr = std::min(nbm, rlim);
-        if (g < ncols && nbm > k) ++nd;
-        if (nbr > k + 1) {
-          ++nB;
-          if (g >= 1) nbk += nbr - k - 1;
-        }
-      }
-      ss.nd[g] = nd;
-      ss.nB[g] = nB;
-      ss.nbk[g] = nbk;
-      ss.gbase[g + 1] = ss.gbase[g] + nd + nbk + (g < ncols ? nB : 0);
+    for (int g = 0; g < ncols; ++g) {
+      int nd = 0;
+      for (int m = 0; m < n; ++m)
+        if (b.np(off + m) / TILE > s0 + g) ++nd;
+      ss.gbase[g + 1] = ss.gbase[g] + nd;
     }
-    const int tot = ss.gbase[ncols + 1];
+    const int tot = ss.gbase[ncols] + ss.pre[n];
     if (tot == 0) continue;
     const uint32_t ep = next_epoch();
     const bool tsu = timer_on(TC_SUPER);

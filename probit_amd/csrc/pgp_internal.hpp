@@ -190,6 +190,19 @@ __device__ __forceinline__ const __attribute__((address_space(1))) T* gbl(const 
   return (const __attribute__((address_space(1))) T*)(uintptr_t)p;
 }
 
+// A value that is the same in every lane, as a scalar.  What a kernel reads
+// from a descriptor after its first store or atomic comes through vector
+// loads; an address formed from it would take two vector registers for each
+// access in flight.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <typename T>
+__device__ __forceinline__ T* uniform(T* p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  return (T*)(((uint64_t)hi << 32) | lo);
+}
+
 // Values handed between workgroups of one launch travel only through
 // relaxed agent-scope accesses: the stores write through the XCD's L2 and
 // the loads read past it, so a publication needs no L2 write-back or
