@@ -79,7 +79,7 @@ constexpr int64_t OFF_PROGRESS_CT = 2560;  // uint64[4] progress words of the wa
 constexpr int64_t HEADER = 4096;
 
 struct WsLayout {
-  int64_t Np, K, L, logdiag, diagval, dinv, vec, symv, csync, panel16, total;
+  int64_t Np, K, L, logdiag, diagval, dinv, vec, symv, csync, xpub, panel16, total;
 };
 // Columns of the BF16 panel copy: a super-step is at most 16 block columns.
 static inline int64_t panel16_pitch(int64_t Np) { return std::min<int64_t>(Np, 16 * TILE); }
@@ -104,6 +104,8 @@ static WsLayout ws_layout(int64_t N, int prec) {
   off += align256(w.Np * (w.Np / TILE) * 8);
   w.csync = off;
   off += align256(csync_words(w.Np) * 4);
+  w.xpub = off;
+  off += align256(w.Np * 16);
   w.panel16 = 0;
   if (prec == PGP_PREC_BF16) {
     w.panel16 = off;
@@ -325,6 +327,7 @@ static Prob make_prob(const pgp_problem_t* pr, const pgp_kernel_t* k, const pgp_
   p.vec = (double*)(ws + L.vec);
   p.symv = (double*)(ws + L.symv);
   p.csync = (uint32_t*)(ws + L.csync);
+  p.xpub = (uint64_t*)(ws + L.xpub);
   p.panel16 = L.panel16 ? (unsigned short*)(ws + L.panel16) : nullptr;
   p.panel16_pitch = (int32_t)panel16_pitch(L.Np);
   p.red = (double*)(ws + OFF_RED);
@@ -1089,7 +1092,8 @@ constexpr int64_t NOALLOC_BYTES = HEADER + 2 * (int64_t)PGP_NOALLOC_MAX_NP * PGP
                                   (int64_t)PGP_NOALLOC_MAX_NP * TILE * 8 +
                                   (int64_t)NVEC * PGP_NOALLOC_MAX_NP * 8 +
                                   (int64_t)PGP_NOALLOC_MAX_NP * (PGP_NOALLOC_MAX_NP / TILE) * 8 +
-                                  csync_words(PGP_NOALLOC_MAX_NP) * 4 + 9 * 256;
+                                  csync_words(PGP_NOALLOC_MAX_NP) * 4 +
+                                  (int64_t)PGP_NOALLOC_MAX_NP * 16 + 10 * 256;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;

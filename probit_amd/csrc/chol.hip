@@ -55,13 +55,6 @@ __device__ __forceinline__ double rsqrt_f64(double p) {
   return fma(r * e, fma(e, 0.375, 0.5), r);
 }
 
-// Broadcast lane `lane`'s double to the whole wave (through scalar registers).
-__device__ __forceinline__ double bcast(double v, int lane) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
-  return __hiloint2double(hi, lo);
-}
-
 // LDS of the diagonal-block factor: the block A ([64][65] doubles) and the
 // exchange area of its waves: the finished 16x16 blocks of three row blocks
 // and the next diagonal sub-block, as register images.

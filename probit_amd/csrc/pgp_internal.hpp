@@ -92,8 +92,10 @@ struct Prob {
   double* pvar;
   // gradient / VB objective
   double* C;  // Np x Np FP64 (C = W^1/2 B^-1 W^1/2, or (sigma^2 I + K)^-1)
-  // single-launch triangular solves: (epoch << 32) | blocks published
+  // column kernel of the Cholesky: (epoch << 32) | columns published
   uint64_t* progress;
+  // single-launch triangular solves: 2 Np words, two per published value
+  uint64_t* xpub;
   // symmetric products: per-tile partial sums, (Np/64) x (Np/64) x 64
   double* symv;
   // wavefront TRSM: one progress word per right-hand-side column tile (4)
@@ -229,6 +231,13 @@ __device__ __forceinline__ void st_coh(T* p, T v) {
 // This wave's outstanding global stores (and loads) complete; also a
 // compiler barrier for memory.
 __device__ __forceinline__ void publish_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Broadcast lane `lane`'s double to the whole wave (through scalar registers).
+__device__ __forceinline__ double bcast(double v, int lane) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+  return __hiloint2double(hi, lo);
+}
 
 // Ticket of this workgroup in start order (thread 0 takes it; the last
 // ticket resets the counter for the next launch on the stream).

@@ -104,168 +104,241 @@ __global__ __launch_bounds__(NTHREADS) void k_trsv(Prob* const* probs, Sched sc,
   }
 }
 
-// ---- single-launch wavefront TRSV --------------------------------------------
-// One workgroup per 64-row block of every member, all in one launch.  In
-// sweep order (forward: blocks 0, 1, ...; transposed: from the last block
-// down), block i accumulates L_ij x_j for every block j before it as soon as
-// x_j is published, then applies DINV_i and publishes x_i.  Publication is a
-// per-member progress word ((epoch << 32) | blocks published) written with
-// release semantics after x_i, read with acquire semantics; x travels through
-// agent-scope (L2-coherent) loads and stores.  Workgroups take their block
-// from a ticket counter in start order, so a workgroup only ever waits for
-// workgroups that are already running: the wait always ends.  Tickets run
-// step-major (`rows`: step s holds the members with more than s blocks, a
-// prefix of the size-sorted batch), so the wave front moves through every
-// member at once instead of member after member.  A wait is
-// also bounded (SPIN_LIMIT polls); if the bound is ever reached the member
-// is flagged PGP_INFO_STALLED and the sweep runs on, so every workgroup exits.
+// ---- single-launch TRSV in segments ------------------------------------------
+// x = L^-1 b (or L^-T b) for every member in one launch: one workgroup of 16
+// waves per segment of SEG block rows, in sweep order (forward: from the
+// first block row; transposed: from the last one up).  Wave (rb, cg) takes 16
+// columns (cg) of block row rb of the segment: it streams the tiles of that
+// block row left (transposed: below) of the segment as their x becomes
+// known, two tiles ahead in registers.  Then the segment's own blocks follow in turn, x_r =
+// DINV_r v_r by the four waves of block row r, handed to the later block
+// rows through LDS.
+//
+// x travels between workgroups as tagged words: value halves in two 64-bit
+// words, each with the launch's epoch in its upper half, so a reader polls
+// the data itself and no separate flag has to follow the data's completion.
+// Both sweeps of a solve write the same buffer (Prob::xpub) in full under
+// different epochs, so a replayed graph of a solve, whose epochs are the
+// captured ones, never finds its own epoch left from the last replay.  One
+// wave of a workgroup polls (one block ahead) and shares x through LDS.
+//
+// Bound: the chain of blocks.  One workgroup per block row with a progress
+// word cost a hand-off through memory per block, 4.7-4.8 us; here the
+// hand-off falls on every SEG-th block, and a sweep over N = 1537 takes 48-52
+// us (FP64) / 33-34 us (FP32) where it took 119.  SEG = 4: the tiles a
+// workgroup streams per block (SEG x 32 KB in FP64) then take about the time
+// its chain needs for one.
+//
+// Workgroups take their segment from a ticket counter in start order, segment
+// major, so a workgroup only waits for running ones, and every wait is
+// bounded (SPIN_LIMIT polls): the member is then flagged PGP_INFO_STALLED and
+// the sweep runs on, so every workgroup exits.
+constexpr int SEG = 4;
+constexpr int SEG_THREADS = 256 * SEG;
 
-template <typename T>
-__global__ __launch_bounds__(NTHREADS) void k_trsv_wave(Prob* const* probs, Sched rows,
-                                                        uint32_t* ticket, uint32_t epoch,
-                                                        int trans, int in, int out) {
-  __shared__ double dk[TILE * (TILE + 1)];  // DINV_i, column-major, column pitch 65
-  __shared__ double part[4][TILE];
-  __shared__ double v[TILE];
+template <typename T, bool TR>
+__global__ __launch_bounds__(SEG_THREADS) void k_trsv_seg(Prob* const* probs, Sched segs,
+                                                          uint32_t* ticket, uint32_t epoch,
+                                                          int in, int out) {
+  __shared__ double xs[2][TILE];      // x of the block being streamed
+  __shared__ double part[sizeof(T) == 8 ? 8 : 16][TILE];  // sums of block row r
+  __shared__ double vs[4][TILE];      // v_r, one copy per wave
+  __shared__ double xq[2][TILE];      // x of the segment's blocks
+  constexpr bool DL = sizeof(T) == 8;
+  __shared__ double dl[DL ? SEG : 1][DL ? TILE : 1][TILE + 1];  // FP64: DINV of the blocks
   __shared__ int s_val;
-  if (threadIdx.x == 0) {
-    const uint32_t t = atomicAdd(ticket, 1u);
-    if (t == gridDim.x - 1) atomicExch(ticket, 0u);  // every ticket taken: reset for the next launch
-    s_val = (int)t;
-  }
-  __syncthreads();
-  const int tk = __builtin_amdgcn_readfirstlane(s_val);
-  if ((unsigned)tk >= gridDim.x) {  // counter not zero at launch: no block to take
-    flag_members_stalled(probs, rows.pre[1] - rows.pre[0]);  // step 0 lists every member
+  const int tk = take_ticket(ticket, &s_val);
+  if ((unsigned)tk >= gridDim.x) {  // counter not zero at launch: no segment to take
+    flag_members_stalled(probs, segs.pre[1] - segs.pre[0]);  // segment 0 lists every member
     return;
   }
-  int m;
-  const int local = sched_member(rows, tk, m);  // step of this member's sweep
-  const Prob& P = *probs[m];
-  const int nb = P.Np / TILE;
-  if (local >= nb) return;
-  const int i = trans ? nb - 1 - local : local;
-  const int64_t ld = P.Np;
-  const T* L = (const T*)P.L;
-  const double* b = vslot(P, in);
-  double* x = vslot(P, out);
-  const double* D = P.dinv + (size_t)i * TILE * TILE;
-  for (int e = threadIdx.x; e < TILE * TILE; e += NTHREADS) dk[(e >> 6) * (TILE + 1) + (e & 63)] = D[e];
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t ri = (int64_t)i * TILE;
-  double pf = 0.0;      // forward: row l, columns 16w.. of each tile
-  double pb[16];        // transposed: rows 16w + rr of block i, lane = row of block j
+  int mi;
+  const int seg = sched_member(segs, tk, mi);
+  const Prob& P = *uniform(probs[mi]);
+  const int nb = uniform(P.Np) / TILE;
+  int64_t ld = (int64_t)nb * TILE;
+  const auto L = gbl((const T*)uniform((char*)P.L));
+  const auto dinv = gbl((const double*)uniform(P.dinv));
+  double* const vec = uniform(P.vec);
+  const auto bv = gbl((const double*)vec + (size_t)in * ld);
+  const auto xv = gbl(vec + (size_t)out * ld);
+  uint64_t* const pub = uniform(P.xpub);
+  int32_t* const info = uniform(P.info);
+  const unsigned l = threadIdx.x & 63;
+  const int w = uniform((int)(threadIdx.x >> 6));
+  const int rb = w >> 2, cg = w & 3;
+  const int b0 = SEG * seg, nblk = min(SEG, nb - b0);
+  auto block = [&](int s) { return TR ? nb - 1 - s : s; };  // sweep position -> block
+  const bool act = rb < nblk;
+  const int i = block(act ? b0 + rb : b0);
+  const int ntile = act ? b0 + rb : 0;  // tiles of this wave's block row
+  // a lane's part of the wave's 64 x 16 strip of a tile: VEC rows from
+  // VEC lr (one 16-byte load) in each of NC columns from NC lg
+  constexpr int VEC = 16 / (int)sizeof(T), RL = TILE / VEC, CG = 64 / RL, NC = 16 / CG;
+  typedef T vec_t __attribute__((ext_vector_type(VEC)));
+  const unsigned lr = l % RL, lg = l / RL;
+  constexpr int DEPTH = 2;
+  vec_t st[DEPTH][NC];
+  auto load = [&](vec_t (&v)[NC], int s) {
+    const int64_t j = block(s);
+    auto p = TR ? L + (j * TILE + ((int64_t)i * TILE + 16 * cg) * ld)
+                : L + ((int64_t)i * TILE + (j * TILE + 16 * cg) * ld);
+    p += lg * NC * ld;
 #pragma unroll
-  for (int rr = 0; rr < 16; ++rr) pb[rr] = 0.0;
-  int done = 0, ready = 0;
-  while (done < local) {
-    if (done >= ready) {
-      __syncthreads();  // everyone has read the previous s_val
-      if (threadIdx.x == 0) {
-        // poll with relaxed loads; the published x is read with coherent
-        // loads issued after the poll, so no cache maintenance is needed
-        int r = 0;
-        for (int spins = 0;; ++spins) {
-          const uint64_t pv = __hip_atomic_load(P.progress, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-          r = ((uint32_t)(pv >> 32) == epoch) ? (int)(uint32_t)pv : 0;
-          if (r > done) break;
-          if (spins >= SPIN_LIMIT) {
-            atomicOr(P.info, PGP_INFO_STALLED);
-            r = local;
-            break;
+    for (int c = 0; c < NC; ++c, p += ld)
+      v[c] = *(const __attribute__((address_space(1))) vec_t*)(p + VEC * lr);
+  };
+#pragma unroll
+  for (int u = 0; u < DEPTH; ++u)
+    if (u < ntile) load(st[u], u);
+  // forward: sums of the lane's VEC rows; transposed: of its NC columns
+  constexpr int NA = TR ? NC : VEC;
+  double acc[NA];
+#pragma unroll
+  for (int c = 0; c < NA; ++c) acc[c] = 0.0;
+  auto consume = [&](const vec_t (&v)[NC], const double* x) {
+    if constexpr (TR) {
+      double xe[VEC];
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) xe[e] = x[VEC * lr + e];
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[c] = fma((double)v[c][e], xe[e], acc[c]);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const double xc = x[16 * cg + NC * lg + c];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[e] = fma((double)v[c][e], xc, acc[e]);
+      }
+    }
+  };
+  // x_r = DINV_r v_r (transposed: DINV_r^T): wave cg of block row r forms rows
+  // 16 cg + (l & 15), a lane 16 of the 64 terms (from 16 (l >> 4)).  DINV_r is
+  // fetched ahead of the stream: into registers, or (FP64, whose tiles take
+  // them) into LDS
+  const unsigned xr = 16 * cg + (l & 15), kq = 16 * (l >> 4);
+  double dv[DL ? 1 : 16];
+  if (act) {
+    const auto D = dinv + (size_t)i * TILE * TILE;
+    if constexpr (DL) {
+      double t[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) t[k] = D[(16 * cg + k) * TILE + l];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) dl[rb][16 * cg + k][l] = t[k];
+    } else {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) dv[k] = TR ? D[TILE * xr + kq + k] : D[(kq + k) * TILE + xr];
+    }
+  }
+  // DINV_r(xr, kq + k), transposed DINV_r(kq + k, xr)
+  auto dval = [&](int k) {
+    if constexpr (DL)
+      return TR ? dl[rb][xr][kq + k] : dl[rb][kq + k][xr];
+    else
+      return dv[k];
+  };
+  const double b = bv[(size_t)i * TILE + l];
+  uint64_t wa = 0, wb = 0;  // the polling wave's next words
+  auto peek = [&](int s) {
+    const uint64_t* p = pub + 2 * ((size_t)block(s) * TILE + l);
+    wa = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    wb = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (w == 0 && b0 > 0) peek(0);
+  auto stream = [&](int s, vec_t (&v)[NC]) {
+    asm volatile("" : "+s"(ld));  // column addresses are formed where they are used
+    if (w == 0) {
+      for (int spins = 0;; ++spins) {
+        const bool ok = (uint32_t)(wa >> 32) == epoch && (uint32_t)(wb >> 32) == epoch;
+        if (__builtin_amdgcn_ballot_w64(!ok) == 0) break;
+        if (spins >= SPIN_LIMIT) {
+          if (l == 0) atomicOr(info, PGP_INFO_STALLED);
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        peek(s);
+      }
+      xs[s & 1][l] = __longlong_as_double((long long)((wb << 32) | (wa & 0xffffffffu)));
+      if (s + 1 < b0) peek(s + 1);
+    }
+    __syncthreads();
+    if (act) {
+      consume(v, xs[s & 1]);
+      if (s + DEPTH < ntile) load(v, s + DEPTH);
+    }
+  };
+  for (int s = 0; s < b0; s += DEPTH) {  // b0 is a multiple of DEPTH
+    stream(s, st[0]);
+    stream(s + 1, st[1]);
+  }
+#pragma unroll
+  for (int r = 0; r < SEG; ++r) {
+    if (r >= nblk) break;
+    if (rb == r) {
+      if constexpr (TR) {
+        // column sums over the lane's row lanes by a transposing butterfly:
+        // row lane lr ends with column (lr / (RL / NC)) of the NC
+        double v[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c] = acc[c];
+#pragma unroll
+        for (int h = NC / 2, bit = RL / 2; h >= 1; h >>= 1, bit >>= 1) {
+          const bool up = (l & bit) != 0;
+#pragma unroll
+          for (int q = 0; q < h; ++q) {
+            const double give = up ? v[q] : v[q + h];
+            const double keep = up ? v[q + h] : v[q];
+            v[q] = keep + __shfl_xor(give, bit);
           }
-          __builtin_amdgcn_s_sleep(1);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        s_val = r;
-      }
-      __syncthreads();
-      ready = __builtin_amdgcn_readfirstlane(s_val);
-    }
-    const int lim = ready < local ? ready : local;
-    // four published tiles at a time: their loads are in flight together
-    for (; done + 4 <= lim; done += 4) {
-      if (!trans) {
-        double xv[4];
-        T lv[4][16];
+        double cs = v[0];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int64_t rj = (int64_t)(done + u) * TILE;
-          xv[u] = ld_coherent(&x[rj + 16 * w + (l & 15)]);
-#pragma unroll
-          for (int c = 0; c < 16; ++c) lv[u][c] = L[(size_t)(ri + l) + (size_t)(rj + 16 * w + c) * ld];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int c = 0; c < 16; ++c) pf += (double)lv[u][c] * __shfl(xv[u], c);
+        for (int bit = RL / NC / 2; bit >= 1; bit >>= 1) cs += __shfl_xor(cs, bit);
+        if (lr % (RL / NC) == 0) part[0][16 * cg + NC * lg + lr / (RL / NC)] = cs;
       } else {
-        double xl[4];
-        T lv[4][16];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int64_t rj = (int64_t)(nb - 1 - (done + u)) * TILE;
-          xl[u] = ld_coherent(&x[rj + l]);
-#pragma unroll
-          for (int rr = 0; rr < 16; ++rr)
-            lv[u][rr] = L[(size_t)(rj + l) + (size_t)(ri + 16 * w + rr) * ld];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int rr = 0; rr < 16; ++rr) pb[rr] += (double)lv[u][rr] * xl[u];
+        for (int e = 0; e < VEC; ++e) part[CG * cg + lg][VEC * lr + e] = acc[e];
       }
     }
-    for (; done < lim; ++done) {
-      const int j = trans ? nb - 1 - done : done;
-      const int64_t rj = (int64_t)j * TILE;
-      if (!trans) {
-        const double xv = ld_coherent(&x[rj + 16 * w + (l & 15)]);
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-          const double xc = __shfl(xv, c);
-          pf += (double)L[(size_t)(ri + l) + (size_t)(rj + 16 * w + c) * ld] * xc;
-        }
+    __syncthreads();
+    if (rb == r) {
+      double sum = 0.0;
+      if constexpr (TR) {
+        sum = part[0][l];
       } else {
-        const double xl = ld_coherent(&x[rj + l]);
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr)
-          pb[rr] += (double)L[(size_t)(rj + l) + (size_t)(ri + 16 * w + rr) * ld] * xl;
+        for (int g = 0; g < 4 * CG; ++g) sum += part[g][l];
+      }
+      vs[cg][l] = b - sum;  // read back by this wave only
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      double a0 = 0.0, a1 = 0.0;
+#pragma unroll
+      for (int k = 0; k < 16; k += 2) {
+        a0 = fma(dval(k), vs[cg][kq + k], a0);
+        a1 = fma(dval(k + 1), vs[cg][kq + k + 1], a1);
+      }
+      double x = a0 + a1;
+      x += __shfl_xor(x, 16);
+      x += __shfl_xor(x, 32);
+      if (l < 16) {
+        xq[r & 1][xr] = x;
+        const uint64_t u = (uint64_t)__double_as_longlong(x), tag = (uint64_t)epoch << 32;
+        uint64_t* p = pub + 2 * ((size_t)i * TILE + xr);
+        __hip_atomic_store(p, tag | (u & 0xffffffffu), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p + 1, tag | (u >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        xv[(size_t)i * TILE + xr] = x;
       }
     }
-  }
-  // v = b_i - sum_j (...)
-  if (!trans) {
-    part[w][l] = pf;
-  } else {
-#pragma unroll
-    for (int rr = 0; rr < 16; ++rr) {
-      double t = pb[rr];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off);
-      if (l == 0) part[0][16 * w + rr] = t;
+    if (r + 1 >= nblk) break;
+    __syncthreads();
+    if (act && rb > r) {
+      consume(st[r % DEPTH], xq[r & 1]);
+      if (r + DEPTH < rb) load(st[r % DEPTH], b0 + r + DEPTH);
     }
-  }
-  __syncthreads();
-  if (threadIdx.x < TILE) {
-    const double acc = trans ? part[0][l] : (part[0][l] + part[1][l]) + (part[2][l] + part[3][l]);
-    v[l] = b[ri + l] - acc;
-  }
-  __syncthreads();
-  // x_i = DINV_i v (forward) or DINV_i^T v (transposed)
-  double a = 0.0;
-#pragma unroll
-  for (int q = 16 * w; q < 16 * w + 16; ++q)
-    a += (trans ? dk[q + l * (TILE + 1)] : dk[l + q * (TILE + 1)]) * v[q];
-  part[w][l] = a;
-  __syncthreads();
-  if (threadIdx.x < TILE) {  // wave 0: store x_i, wait for the stores, then publish
-    st_coherent(&x[ri + l], (part[0][l] + part[1][l]) + (part[2][l] + part[3][l]));
-    publish_wait();
-    if (threadIdx.x == 0)
-      __hip_atomic_store(P.progress, ((uint64_t)epoch << 32) | (uint64_t)(local + 1),
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -285,19 +358,19 @@ uint32_t next_epoch() {
 }
 
 void launch_trsv(const Batch& bt, int prec, int trans, int in, int out, hipStream_t s) {
-  if (bt.ticket && wavefront_trsv() && bt.maxNp / TILE <= MAXB) {
-    // step-major schedule: step s holds the members with more than s blocks
-    // (a prefix: members are sorted by size), one workgroup each
-    const int nb = bt.maxNp / TILE;
+  const int nseg = (bt.maxNp / TILE + SEG - 1) / SEG;
+  if (bt.ticket && wavefront_trsv() && nseg <= MAXB) {
+    // segment-major schedule: segment t holds the members with more than t
+    // segments (a prefix: members are sorted by size), one workgroup each
     Sched rows;
-    rows.count = nb;
+    rows.count = nseg;
     int tot = 0;
-    for (int st = 0; st < nb; ++st) {
+    for (int st = 0; st < nseg; ++st) {
       rows.pre[st] = tot;
       for (int m = 0; m < bt.count; ++m)
-        if (bt.np(m) / TILE > st) ++tot;
+        if (bt.np(m) / TILE > SEG * st) ++tot;
     }
-    rows.pre[nb] = tot;
+    rows.pre[nseg] = tot;
     if (tot == 0) return;
     const bool on = timer_on(TC_TRSV);
     const double esz = prec == PGP_PREC_FP64 ? 8.0 : 4.0;
@@ -313,12 +386,14 @@ void launch_trsv(const Batch& bt, int prec, int trans, int in, int out, hipStrea
       timer_begin(TC_TRSV, s);
     }
     const uint32_t ep = next_epoch();
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(tot), dim3(SEG_THREADS), 0, s, bt.dprobs, rows, bt.ticket,
+                         ep, in, out);
+    };
     if (prec == PGP_PREC_FP64)
-      hipLaunchKernelGGL(k_trsv_wave<double>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                         bt.ticket, ep, trans, in, out);
+      trans ? go(k_trsv_seg<double, true>) : go(k_trsv_seg<double, false>);
     else
-      hipLaunchKernelGGL(k_trsv_wave<float>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                         bt.ticket, ep, trans, in, out);
+      trans ? go(k_trsv_seg<float, true>) : go(k_trsv_seg<float, false>);
     if (on) timer_end(TC_TRSV, s, fl, by);
     return;
   }
@@ -476,7 +551,7 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged_raw(const T* L, int64_
 // for every block j < i as soon as (j, ct) publishes, then forms
 // X_i = DINV_i (S_i - acc) and publishes it: X_i through agent-scope stores,
 // a wait for their completion, then the member's progress word of column
-// tile ct.  Start-order tickets and bounded waits as in k_trsv_wave.
+// tile ct.  Start-order tickets and bounded waits as in k_trsv_seg.
 constexpr int WAVE_NCT = 4;
 
 template <typename T>
