@@ -29,7 +29,7 @@ namespace pgp {
 
 // grad.hip
 void launch_sym_from_inv(const Batch& b, int prec, int use_scale, hipStream_t s);
-void launch_fill_rhs(const Batch& b, int prec, int mode, hipStream_t s);
+void launch_tri_inverse(const Batch& b, int prec, hipStream_t s);
 void launch_sigma_diag(const Batch& b, int prec, hipStream_t s);
 void launch_grad_trace(const Batch& b, double* partials, double* out, hipStream_t s);
 void launch_vb_trace(const Batch& b, double* out, hipStream_t s);
@@ -149,7 +149,7 @@ static bool predict_refine(int prec) {
 static void predict_launches(const Batch& b, int prec, int maxM, hipStream_t s) {
   const int maxMp = (int)round_up(maxM, TILE);
   launch_cross_prep(b, prec, maxM, s);
-  launch_trsm(b, prec, maxMp, 0, s);
+  launch_trsm(b, prec, maxMp, s);
   if (predict_refine(prec)) {
     launch_trsm_t(b, prec, maxMp, s);
     launch_pred_refine(b, prec, maxM, s);
@@ -778,7 +778,7 @@ int pgp_trsm(int precision, const void* L, int64_t N, int64_t ld, double* dinv, 
   if (ld < N || ld_s < N) return fail(-4, "ld < N");
   hipStream_t s = (hipStream_t)stream;
   launch_dinv_raw(precision, L, N, ld, dinv, s);
-  launch_trsm_raw_dinv(precision, L, N, ld, dinv, S, M, ld_s, 0, s);
+  launch_trsm_raw_dinv(precision, L, N, ld, dinv, S, M, ld_s, s);
   return check_launch();
 }
 
@@ -1286,7 +1286,7 @@ int pgp_predict_covariance(const pgp_kernel_t* kernel, const double* Xtest, int6
   write_prob(ws, p, 0, s);
   const Batch b = single_batch(ws, p.Np);
   launch_cross_prep(b, p.prec, (int)M, s);
-  launch_trsm(b, p.prec, (int)PL.Mp, 0, s);
+  launch_trsm(b, p.prec, (int)PL.Mp, s);
   launch_pred_cov(b, p.prec, (int)PL.Mp, cov, ld, s);
   rc = check_launch();
   if (rc) return rc;
@@ -1327,13 +1327,9 @@ int pgp_laplace_grad(const pgp_kernel_t* kernel, const pgp_likelihood_t* lik, do
   const int prec = p.prec;
   launch_lik_final(b, 1, s);  // G, W, S, LL, D3 at the resident f
   // C = S Linv^T Linv S
-  launch_fill_rhs(b, prec, 1, s);
-  launch_trsm(b, prec, p.Np, 1, s);
+  launch_tri_inverse(b, prec, s);
   launch_sym_from_inv(b, prec, 1, s);
-  // Sigma_ii from V = L^-1 (S K)
-  launch_fill_rhs(b, prec, 0, s);
-  launch_trsm(b, prec, p.Np, 0, s);
-  launch_sigma_diag(b, prec, s);
+  launch_sigma_diag(b, prec, s);  // X1 = Sigma_ii
   // shat = s2 - C K s2, s2 = -1/2 Sigma d3;  X2 <- K shat
   launch_vec_op(b, OP_GRAD_S2, s);       // X2 = -0.5 X1 .* D3
   launch_gemv_sym(b, V_X2, V_X4, 0, s);  // X4 = K s2
@@ -1412,8 +1408,7 @@ int pgp_vb_grad(const pgp_kernel_t* kernel, const pgp_likelihood_t* lik, double*
   double* gather = (double*)(ws + OFF_GATHER);
   // C = A^-1 = S B^-1 S from the resident factor (W = 1/sigma^2, S = 1/sigma)
   launch_vec_op(b, OP_VB_PREC, s);
-  launch_fill_rhs(b, prec, 1, s);
-  launch_trsm(b, prec, p.Np, 1, s);
+  launch_tri_inverse(b, prec, s);
   launch_sym_from_inv(b, prec, 1, s);
   // f = K a; d1, W = -d2, S = sqrt(max(W, 0)) of the likelihood
   launch_gemv_sym(b, V_Z, V_F, 0, s);
@@ -1531,8 +1526,7 @@ int pgp_vb_fit(const pgp_problem_t* problem, const pgp_kernel_t* kernel,
   launch_gemv_sym(b, V_Z, V_F, 0, s);
   launch_lik_final(b, 0, s);
   launch_reduce(b, RED_FINAL, gather, s);
-  launch_fill_rhs(b, prec, 1, s);
-  launch_trsm(b, prec, p.Np, 1, s);
+  launch_tri_inverse(b, prec, s);
   launch_sym_from_inv(b, prec, 0, s);
   double* tr_out = (double*)(gw + G.out);
   launch_vb_trace(b, tr_out, s);

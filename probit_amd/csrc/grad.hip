@@ -10,13 +10,16 @@
 //   d/dtheta_K = sum_ij dK_ij/dtheta G_ij,  G = C/2 - a a^T/2 + (shat a^T + a shat^T)/2,
 //   d/dtheta_l = sum_i [-L_p - Sigma_ii L_ffp / 2 + (K shat)_i L_fp].
 // This file holds the O(N^3) pieces reused from the resident factor:
-//   * k_sym_from_inv: C = S (Linv^T Linv) S (or Linv^T Linv for VB), full;
+//   * k_inv_merge: Linv = L^-1 by doubling;
+//   * k_sym_from_inv: C = S (Linv^T Linv) S (or Linv^T Linv for VB), lower;
 //   * k_grad_trace: tiles of sum_ij dK_ij/dtheta G_ij with dK recomputed from
 //     X in registers, lower tiles only (off-diagonal tiles count twice),
 //     per-tile partials reduced in a fixed order by k_sum_partials;
 //   * k_vb_trace: tr(C) and sum_ij K_ij C_ij of objective_VB
 //     (probit/implicit/VB.py:28-30).
 #include <math.h>
+
+#include <algorithm>
 
 #include "mfma.hpp"
 #include "pgp_internal.hpp"
@@ -34,35 +37,115 @@ __device__ __forceinline__ void lower_tile_g(int t, int& ti, int& tj) {
   tj = t - i * (i + 1) / 2;
 }
 
-// C(i0.., j0..) = scale_i * sum_k X(k, i) X(k, j) * scale_j, X column-major
-// lower triangular (Linv), so the k range starts at max(i0, j0).
+// ---- X = L^-1 ------------------------------------------------------------------
+// The explicit inverse of the resident factor (lower triangular, in P.S) by
+// doubling: its diagonal tiles are DINV; two neighbouring inverted diagonal
+// blocks of h tiles give the inverse of their 2h-tile block,
+//   X_21 = -X_22 (L_21 X_11),
+// two launches per doubling, every tile of every pair its own workgroup.  The
+// product L_21 X_11 waits in the unused upper tiles (tile (i, j) of it at
+// (j, i)).  Bound: FP64 MFMA once the blocks are large (N^3 / 3 flops in
+// all), the launches before.  A forward substitution of the identity has
+// the factor's block rows as a serial chain instead: 3.1 ms at N = 4096
+// (FP64), 16 x 22 us at N = 512, where this takes 0.87 ms and 6 x 10 us.
+template <typename T>
+__global__ __launch_bounds__(NTHREADS) void k_inv_diag(Prob* const* probs) {
+  const Prob& P = *probs[blockIdx.y];
+  const int i = blockIdx.x;
+  if (i >= P.Np / TILE) return;
+  const auto D = gbl(P.dinv + (size_t)i * TILE * TILE);
+  const auto X = gbl((T*)P.S) + (size_t)i * TILE * (P.Np + 1);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int e = threadIdx.x + NTHREADS * q;
+    X[(size_t)(e >> 6) * P.Np + (e & 63)] = (T)D[e];
+  }
+}
+
+template <typename T, bool SECOND>
+__global__ __launch_bounds__(NTHREADS) void k_inv_merge(Prob* const* probs, int h) {
+  const Prob& P = *probs[blockIdx.z];
+  const int nb = P.Np / TILE;
+  const int a = 2 * h * blockIdx.y, mid = a + h;
+  // the longest sums first: first product k from j, second k up to i
+  const int j = a + (int)blockIdx.x % h;
+  const int i = SECOND ? min(nb, mid + h) - 1 - (int)blockIdx.x / h : mid + (int)blockIdx.x / h;
+  if (i >= nb || i < mid) return;
+  const int64_t ld = P.Np;
+  const unsigned m = threadIdx.x & 63;
+  const int kb = uniform((int)(threadIdx.x >> 6));
+  const auto L = gbl((const T*)P.L);
+  const auto X = gbl((T*)P.S);
+  __shared__ GemmLds<T> lds;
+  typename Acc<T>::type acc[2][2];
+  zero_acc<T>(acc);
+  auto tile = [&](auto base, int r, int c, T (&v)[16]) {
+    auto p = base + ((int64_t)r * TILE + ((int64_t)c * TILE + kb) * ld);
+#pragma unroll
+    for (int q = 0; q < 16; ++q, p += 4 * ld) v[q] = p[m];
+  };
+  if constexpr (!SECOND)
+    gemm_tiles<T, false>(
+        j, mid, [&](int k, T (&v)[16]) { tile(L, i, k, v); },
+        [&](int k, T (&v)[16]) { tile(X, k, j, v); }, lds, acc);
+  else
+    gemm_tiles<T, false>(
+        mid, i + 1, [&](int k, T (&v)[16]) { tile(X, i, k, v); },
+        [&](int k, T (&v)[16]) { tile(X, j, k, v); }, lds, acc);
+  const int r0 = SECOND ? i : j, c0 = SECOND ? j : i;
+#pragma unroll
+  for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+    for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        X[(size_t)(r0 * TILE + acc_row<T>(bm, r)) + (size_t)(c0 * TILE + acc_col(bn)) * ld] =
+            (T)(SECOND ? -acc[bm][bn][r] : acc[bm][bn][r]);
+}
+
+template <typename T>
+static void tri_inverse(const Batch& b, hipStream_t s) {
+  const int nb = b.maxNp / TILE;
+  hipLaunchKernelGGL(k_inv_diag<T>, dim3(nb, b.count), dim3(NTHREADS), 0, s, b.dprobs);
+  for (int h = 1; h < nb; h *= 2) {
+    const dim3 g(h * std::min(h, nb - h), (nb - h + 2 * h - 1) / (2 * h), b.count);
+    hipLaunchKernelGGL((k_inv_merge<T, false>), g, dim3(NTHREADS), 0, s, b.dprobs, h);
+    hipLaunchKernelGGL((k_inv_merge<T, true>), g, dim3(NTHREADS), 0, s, b.dprobs, h);
+  }
+}
+
+void launch_tri_inverse(const Batch& b, int prec, hipStream_t s) {
+  if (prec == PGP_PREC_FP64)
+    tri_inverse<double>(b, s);
+  else
+    tri_inverse<float>(b, s);
+}
+
+// C(i0.., j0..) = scale_i * sum_k X(k, i) X(k, j) * scale_j, X = L^-1, so the
+// k range starts at i0 >= j0: the lower tiles of C (its readers take the
+// lower triangle only), those with the longest sums first.
 template <typename T>
 __global__ __launch_bounds__(NTHREADS) void k_sym_from_inv(Prob* const* probs, int use_scale) {
   const Prob& P = *probs[blockIdx.y];
   const int nb = P.Np / TILE;
-  if ((int)blockIdx.x >= nb * nb) return;
-  const int ti = blockIdx.x % nb, tj = blockIdx.x / nb;
-  const T* X = (const T*)P.S;  // Linv (Np x Np) lives in the gradient buffer
+  if ((int)blockIdx.x >= nb * (nb + 1) / 2) return;
+  int ti, tj;
+  lower_tile_g(blockIdx.x, ti, tj);
   const int64_t ld = P.Np;
-  __shared__ T As[TILE * (TILE + 1)];
-  __shared__ T Bs[TILE * (TILE + 1)];
-  typedef typename Acc<T>::type acc_t;
-  acc_t acc[2][2];
+  const auto X = gbl((const T*)P.S);
+  __shared__ GemmLds<T> lds;
+  typename Acc<T>::type acc[2][2];
   zero_acc<T>(acc);
-  const int kstart = ti > tj ? ti : tj;
-  const int r = threadIdx.x & 63, cb = threadIdx.x >> 6;
-  for (int kb = kstart; kb < nb; ++kb) {
-    // As[kk][m] = X(kb*64 + kk, ti*64 + m); Bs[kk][n] = X(kb*64 + kk, tj*64 + n)
-#pragma unroll 4
-    for (int q = 0; q < 16; ++q) {
-      const int c = cb + 4 * q;
-      As[r * (TILE + 1) + c] = X[(size_t)(kb * TILE + r) + (size_t)(ti * TILE + c) * ld];
-      Bs[r * (TILE + 1) + c] = X[(size_t)(kb * TILE + r) + (size_t)(tj * TILE + c) * ld];
-    }
-    __syncthreads();
-    mma64_kmajor<T>(As, TILE + 1, Bs, TILE + 1, acc);
-    __syncthreads();
-  }
+  const unsigned m = threadIdx.x & 63;
+  const int kb = uniform((int)(threadIdx.x >> 6));
+  auto rows = [&](int k, int t, T (&v)[16]) {
+    auto p = X + ((int64_t)k * TILE + ((int64_t)t * TILE + kb) * ld);
+#pragma unroll
+    for (int q = 0; q < 16; ++q, p += 4 * ld) v[q] = p[m];
+  };
+  gemm_tiles<T, true>(
+      ti, nb, [&](int k, T (&v)[16]) { rows(k, ti, v); },
+      [&](int k, T (&v)[16]) { rows(k, tj, v); }, lds, acc);
   const double* S = vslot(P, V_S);
 #pragma unroll
   for (int bm = 0; bm < 2; ++bm)
@@ -81,48 +164,53 @@ __global__ __launch_bounds__(NTHREADS) void k_sym_from_inv(Prob* const* probs, i
 
 void launch_sym_from_inv(const Batch& b, int prec, int use_scale, hipStream_t s) {
   const int nb = b.maxNp / TILE;
-  dim3 g(nb * nb, b.count);
+  dim3 g(nb * (nb + 1) / 2, b.count);
   if (prec == PGP_PREC_FP64)
     hipLaunchKernelGGL(k_sym_from_inv<double>, g, dim3(NTHREADS), 0, s, b.dprobs, use_scale);
   else
     hipLaunchKernelGGL(k_sym_from_inv<float>, g, dim3(NTHREADS), 0, s, b.dprobs, use_scale);
 }
 
-// RHS for V = L^-1 (S .* K): G2(i, j) = S_i K_ij  (storage T); also the
-// identity right-hand side for Linv (mode 1).
-template <typename T>
-__global__ __launch_bounds__(NTHREADS) void k_fill_rhs(Prob* const* probs, int mode) {
+// Sigma_ii = K_ii - (K C K)_ii where W_i < 0 (S_i = 0, so K C K says nothing
+// about W_i): one workgroup per such row, from the lower triangle of C.  The
+// other rows come from (K C)_ii = W_i Sigma_ii (gemv_epilogue's mode 4).
+__global__ __launch_bounds__(NTHREADS) void k_sigma_negative(Prob* const* probs) {
   const Prob& P = *probs[blockIdx.y];
-  const int64_t n2 = (int64_t)P.Np * P.Np;
-  const int64_t e = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
-  if (e >= n2) return;
-  const int i = (int)(e % P.Np), j = (int)(e / P.Np);
-  T* out = (T*)P.S;
-  double v;
-  if (mode == 1)
-    v = (i == j) ? 1.0 : 0.0;
-  else
-    v = vslot(P, V_S)[i] * P.K[e];
-  out[e] = (T)v;
+  const int i = blockIdx.x;
+  if (i >= P.N || !(vslot(P, V_W)[i] < 0.0)) return;
+  const double* k = P.K + (size_t)i * P.Np;
+  double q = 0.0;
+  for (int c = threadIdx.x >> 6; c < P.N; c += 4) {
+    const double* col = P.C + (size_t)c * P.Np;
+    double a = 0.0;
+    for (int r = c + (threadIdx.x & 63); r < P.N; r += 64) a += (r == c ? 1.0 : 2.0) * col[r] * k[r];
+    q += a * k[c];
+  }
+  __shared__ double red[NTHREADS];
+  red[threadIdx.x] = q;
+  __syncthreads();
+  for (int st = NTHREADS / 2; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) vslot(P, V_X1)[i] = k[i] - red[0];
 }
 
-void launch_fill_rhs(const Batch& b, int prec, int mode, hipStream_t s) {
-  const int64_t n2 = (int64_t)b.maxNp * b.maxNp;
-  dim3 g((unsigned)((n2 + NTHREADS - 1) / NTHREADS), b.count);
-  if (prec == PGP_PREC_FP64)
-    hipLaunchKernelGGL(k_fill_rhs<double>, g, dim3(NTHREADS), 0, s, b.dprobs, mode);
-  else
-    hipLaunchKernelGGL(k_fill_rhs<float>, g, dim3(NTHREADS), 0, s, b.dprobs, mode);
+// Right-hand side S_i K_ij of V = L^-1 S K (factors stored in FP32).
+__global__ __launch_bounds__(NTHREADS) void k_fill_rhs(Prob* const* probs) {
+  const Prob& P = *probs[blockIdx.y];
+  const int64_t e = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
+  if (e >= (int64_t)P.Np * P.Np) return;
+  ((float*)P.S)[e] = (float)(vslot(P, V_S)[e % P.Np] * P.K[e]);
 }
 
 // Sigma_jj = K_jj - ||V_:,j||^2 into X1 (one wave per column).
-template <typename T>
-__global__ __launch_bounds__(NTHREADS) void k_sigma_diag(Prob* const* probs) {
+__global__ __launch_bounds__(NTHREADS) void k_sigma_norms(Prob* const* probs) {
   const Prob& P = *probs[blockIdx.y];
   const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (j >= P.Np) return;
   const int lane = threadIdx.x & 63;
-  const T* V = (const T*)P.S + (size_t)j * P.Np;
+  const float* V = (const float*)P.S + (size_t)j * P.Np;
   double q = 0.0;
   for (int i = lane; i < P.Np; i += 64) {
     const double v = (double)V[i];
@@ -133,12 +221,34 @@ __global__ __launch_bounds__(NTHREADS) void k_sigma_diag(Prob* const* probs) {
   if (lane == 0) vslot(P, V_X1)[j] = (j < P.N) ? P.K[(size_t)j * P.Np + j] - q : 0.0;
 }
 
+// diag Sigma into X1, Sigma = (K^-1 + W)^-1 = K - K C K.  FP64 factors: from C
+// and K alone.  Sigma W = K C, so Sigma_ii = (sum_j K_ij C_ij) / W_i, two N^2
+// passes where the column norms of L^-1 S K take a solve with N right-hand
+// sides (N^3 flops: 3.2 ms at N = 4096, now 0.05).  The terms of the sum
+// carry S_i, so its relative error grows only as max(S) / S_i where W_i is
+// small, and there the third derivative it is multiplied with goes with W_i.
+// Factors stored in FP32 keep the column norms: C then carries the factor's
+// FP32 error, which the norms damp (noise gradient of a Gaussian fit at N =
+// 2000: 7e-5 relative error from the norms, 1e-3 from C).
 void launch_sigma_diag(const Batch& b, int prec, hipStream_t s) {
-  dim3 g((b.maxNp + 3) / 4, b.count);
-  if (prec == PGP_PREC_FP64)
-    hipLaunchKernelGGL(k_sigma_diag<double>, g, dim3(NTHREADS), 0, s, b.dprobs);
-  else
-    hipLaunchKernelGGL(k_sigma_diag<float>, g, dim3(NTHREADS), 0, s, b.dprobs);
+  if (prec == PGP_PREC_FP64) {
+    launch_hadamard_tiles(b, s);
+    launch_symv_reduce(b, V_X1, V_X1, 4, s);
+    hipLaunchKernelGGL(k_sigma_negative, dim3(b.maxNp, b.count), dim3(NTHREADS), 0, s, b.dprobs);
+    return;
+  }
+  const int64_t n2 = (int64_t)b.maxNp * b.maxNp;
+  hipLaunchKernelGGL(k_fill_rhs, dim3((unsigned)((n2 + NTHREADS - 1) / NTHREADS), b.count),
+                     dim3(NTHREADS), 0, s, b.dprobs);
+  launch_trsm(b, prec, b.maxNp, s);
+  hipLaunchKernelGGL(k_sigma_norms, dim3((b.maxNp + 3) / 4, b.count), dim3(NTHREADS), 0, s,
+                     b.dprobs);
+}
+
+// Parameter p of (variance, lengthscale[GMAXD], period[GMAXD]) is one of the
+// kernel's.
+__device__ __forceinline__ bool grad_par_used(int p, int D, int periodic) {
+  return p <= D || (periodic && p > GMAXD && p <= GMAXD + D);
 }
 
 // Fused trace: partials[tile][p] = w_tile * sum_{(i,j) in tile} dK_ij/dtheta_p G_ij
@@ -218,41 +328,42 @@ __global__ __launch_bounds__(NTHREADS) void k_grad_trace(Prob* const* probs, dou
       }
     }
   }
-  // fixed-order block reduction of each accumulator
-  __shared__ double red[4];
+  // fixed-order block reduction of the accumulators in use
+  __shared__ double red[NPAR][4];
+#pragma unroll
   for (int p = 0; p < NPAR; ++p) {
+    if (!grad_par_used(p, D, P.periodic)) continue;
     double v = acc[p];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0)
-      partials[((size_t)blockIdx.y * ntiles + blockIdx.x) * NPAR + p] =
-          (red[0] + red[1]) + (red[2] + red[3]);
+    if ((threadIdx.x & 63) == 0) red[p][threadIdx.x >> 6] = v;
   }
+  __syncthreads();
+  const int p = threadIdx.x;
+  if (p < NPAR && grad_par_used(p, D, P.periodic))
+    partials[((size_t)blockIdx.y * ntiles + blockIdx.x) * NPAR + p] =
+        (red[p][0] + red[p][1]) + (red[p][2] + red[p][3]);
 }
 
-// out[b * NPAR + p] = sum over tiles (fixed order)
+// out[b * NPAR + p] = sum over tiles (fixed order), one workgroup per p
 __global__ __launch_bounds__(NTHREADS) void k_sum_partials(Prob* const* probs,
                                                            const double* partials, double* out) {
-  const Prob& P = *probs[blockIdx.x];
+  const Prob& P = *probs[blockIdx.y];
   const int T = P.Np / TILE;
   const int ntiles = T * (T + 1) / 2;
+  const int p = blockIdx.x;
   __shared__ double red[NTHREADS];
-  for (int p = 0; p < NPAR; ++p) {
-    double v = 0.0;
+  double v = 0.0;
+  if (grad_par_used(p, P.D, P.periodic))
     for (int t = threadIdx.x; t < ntiles; t += NTHREADS)
-      v += partials[((size_t)blockIdx.x * ntiles + t) * NPAR + p];
-    red[threadIdx.x] = v;
-    __syncthreads();
-    for (int st = NTHREADS / 2; st > 0; st >>= 1) {
-      if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[(size_t)blockIdx.x * NPAR + p] = red[0];
+      v += partials[((size_t)blockIdx.y * ntiles + t) * NPAR + p];
+  red[threadIdx.x] = v;
+  __syncthreads();
+  for (int st = NTHREADS / 2; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
     __syncthreads();
   }
+  if (threadIdx.x == 0) out[(size_t)blockIdx.y * NPAR + p] = red[0];
 }
 
 int grad_npar() { return NPAR; }
@@ -262,20 +373,18 @@ void launch_grad_trace(const Batch& b, double* partials, double* out, hipStream_
   const int T = b.maxNp / TILE;
   dim3 g(T * (T + 1) / 2, b.count);
   hipLaunchKernelGGL(k_grad_trace, g, dim3(NTHREADS), 0, s, b.dprobs, partials);
-  hipLaunchKernelGGL(k_sum_partials, dim3(b.count), dim3(NTHREADS), 0, s, b.dprobs, partials, out);
+  hipLaunchKernelGGL(k_sum_partials, dim3(NPAR, b.count), dim3(NTHREADS), 0, s, b.dprobs, partials, out);
 }
 
-// VB traces: out[0] = tr(C), out[1] = sum_ij K_ij C_ij over the N x N block.
+// VB traces: out[0] = tr(C), out[1] = sum_ij K_ij C_ij over the N x N block
+// (the row sums of K o C, in X1).
 __global__ __launch_bounds__(NTHREADS) void k_vb_trace(Prob* const* probs, double* out) {
   const Prob& P = *probs[blockIdx.x];
+  const double* rows = vslot(P, V_X1);
   double tr = 0.0, kc = 0.0;
-  const int64_t n2 = (int64_t)P.Np * P.Np;
-  for (int64_t e = threadIdx.x; e < n2; e += NTHREADS) {
-    const int i = (int)(e % P.Np), j = (int)(e / P.Np);
-    if (i >= P.N || j >= P.N) continue;
-    const double c = P.C[e];
-    kc += P.K[e] * c;
-    if (i == j) tr += c;
+  for (int i = threadIdx.x; i < P.N; i += NTHREADS) {
+    kc += rows[i];
+    tr += P.C[(size_t)i + (size_t)i * P.Np];
   }
   __shared__ double r1[NTHREADS], r2[NTHREADS];
   r1[threadIdx.x] = tr;
@@ -295,6 +404,8 @@ __global__ __launch_bounds__(NTHREADS) void k_vb_trace(Prob* const* probs, doubl
 }
 
 void launch_vb_trace(const Batch& b, double* out, hipStream_t s) {
+  launch_hadamard_tiles(b, s);
+  launch_symv_reduce(b, V_X1, V_X1, 0, s);
   hipLaunchKernelGGL(k_vb_trace, dim3(b.count), dim3(NTHREADS), 0, s, b.dprobs, out);
 }
 

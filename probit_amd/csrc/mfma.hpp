@@ -188,6 +188,44 @@ __device__ __forceinline__ int acc_col(int bn) {
   return 32 * (w & 1) + 16 * bn + (l & 15);
 }
 
+// acc += sum over k in [k0, k1) of A_k B_k for 64 x 64 tiles: the next pair of
+// tiles is fetched into registers while the current one is multiplied from
+// LDS.  Thread (lane, wave): fb(k, v) fetches v[q] = B_k(lane, wave + 4 q);
+// fa(k, v) v[q] = A_k(lane, wave + 4 q), or (AROW) A_k(wave + 4 q, lane), the
+// tile being given by its rows of k.  LDS is free again on return.
+template <typename T>
+struct GemmLds {
+  static constexpr int PB = 65;
+  T a[64 * (KP<T>::value > PB ? KP<T>::value : PB)];
+  T b[64 * PB];
+};
+template <typename T, bool AROW, class FA, class FB>
+__device__ __forceinline__ void gemm_tiles(int k0, int k1, FA fa, FB fb, GemmLds<T>& lds,
+                                           typename Acc<T>::type (&acc)[2][2]) {
+  constexpr int PB = GemmLds<T>::PB, PA = AROW ? PB : KP<T>::value;
+  if (k0 >= k1) return;
+  const int m = threadIdx.x & 63, kb = threadIdx.x >> 6;
+  T ra[16], rb[16];
+  fa(k0, ra);
+  fb(k0, rb);
+  for (int k = k0; k < k1; ++k) {
+    if (k > k0) __syncthreads();  // the previous products are done with LDS
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int c = kb + 4 * q;
+      lds.a[AROW ? m * PA + c : c * PA + m] = ra[q];
+      lds.b[m * PB + c] = rb[q];
+    }
+    __syncthreads();
+    if (k + 1 < k1) {
+      fa(k + 1, ra);
+      fb(k + 1, rb);
+    }
+    mma64_kmajor<T>(lds.a, PA, lds.b, PB, acc);
+  }
+  __syncthreads();
+}
+
 // Load a 64x64 column-major global block (rows r0.., cols c0.., ld) into
 // k-major LDS dst[k * pitch + m] = G(r0 + m, c0 + k), converting to TL.
 template <typename TG, typename TL>

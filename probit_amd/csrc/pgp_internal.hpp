@@ -340,12 +340,12 @@ int launch_dinv_raw(int prec, const void* A, int64_t N, int64_t ld, double* dinv
 
 // solve.hip
 void launch_trsv(const Batch& b, int prec, int trans, int in, int out, hipStream_t s);
-void launch_trsm(const Batch& b, int prec, int maxMp, int lower_rhs, hipStream_t s);
+void launch_trsm(const Batch& b, int prec, int maxMp, hipStream_t s);
 void launch_trsm_t(const Batch& b, int prec, int maxMp, hipStream_t s);
 int launch_trsv_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const double* dinv,
                          double* b, double* x, int trans, hipStream_t s);
 int launch_trsm_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const double* dinv,
-                         void* S, int64_t M, int64_t lds, int lower_rhs, hipStream_t s);
+                         void* S, int64_t M, int64_t lds, hipStream_t s);
 
 // vec.hip
 enum VecOp {
@@ -372,6 +372,8 @@ enum RedWhat { RED_STEP = 0, RED_FINAL = 1 };
 void launch_gemv_sym(const Batch& b, int x_slot, int out_slot, int mode, hipStream_t s);
 // the two halves of launch_gemv_sym's symmetric product (modes < 10)
 void launch_symv_tiles(const Batch& b, int x_slot, hipStream_t s);
+// per-tile partial sums of the row sums of K o C, for launch_symv_reduce
+void launch_hadamard_tiles(const Batch& b, hipStream_t s);
 void launch_symv_reduce(const Batch& b, int x_slot, int out_slot, int mode, hipStream_t s);
 void launch_vec_op(const Batch& b, int op, hipStream_t s);
 void launch_copy_slot(const Batch& b, int src, int dst, hipStream_t s);

@@ -457,17 +457,14 @@ int launch_trsv_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const d
 // Every workgroup writes only its own rows and reads only rows finished in
 // earlier launches, so workgroups of one launch never race, whatever order
 // they run in.  Launch 0 holds only the w == 0 workgroups.
-// lower_rhs: S is lower triangular (identity-like right-hand side): tiles
-// with ct > k, and the updates of tile ct == k, are zero and are skipped.
 template <typename T>
 __device__ __forceinline__ void trsm_step(const T* L, int64_t ld, const double* dinv, int k, T* S, int64_t lds,
-                          int w, int ct, int lower_rhs) {
+                          int w, int ct) {
   constexpr int PP = KP<T>::value;  // A operand: conflict-free MFMA reads
   constexpr int PB = TILE + 1;       // B operand: written transposed, conflict-free stores
   __shared__ T As[TILE * PP];
   __shared__ T Bs[TILE * PB];
   typedef typename Acc<T>::type acc_t;
-  if (lower_rhs && (ct > k || (ct == k && w > 0))) return;
   const int64_t r0 = (int64_t)(k + w) * TILE;
   const int64_t n0 = (int64_t)ct * TILE;
   acc_t acc[2][2];
@@ -525,8 +522,7 @@ __device__ __forceinline__ void trsm_step(const T* L, int64_t ld, const double* 
 }
 
 template <typename T>
-__global__ __launch_bounds__(NTHREADS) void k_trsm_lagged(Prob* const* probs, Sched sc, int k,
-                                                          int lower_rhs) {
+__global__ __launch_bounds__(NTHREADS) void k_trsm_lagged(Prob* const* probs, Sched sc, int k) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
   const int nb = P.Np / TILE;
@@ -534,14 +530,14 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged(Prob* const* probs, Sc
   const int rows = k == 0 ? 1 : nb - k;  // row blocks of this launch
   const int w = bx % rows, ct = bx / rows;
   if (ct >= P.Mp / TILE) return;
-  trsm_step<T>((const T*)P.L, P.Np, P.dinv, k, (T*)P.S, P.Np, w, ct, lower_rhs);
+  trsm_step<T>((const T*)P.L, P.Np, P.dinv, k, (T*)P.S, P.Np, w, ct);
 }
 
 template <typename T>
 __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged_raw(const T* L, int64_t ld,
                                                               const double* dinv, int k, T* S,
-                                                              int64_t lds, int lower_rhs) {
-  trsm_step<T>(L, ld, dinv, k, S, lds, blockIdx.x, blockIdx.y, lower_rhs);
+                                                              int64_t lds) {
+  trsm_step<T>(L, ld, dinv, k, S, lds, blockIdx.x, blockIdx.y);
 }
 
 // Wavefront TRSM for narrow right-hand sides (at most WAVE_NCT column
@@ -832,8 +828,7 @@ static bool wavefront_trsm() {
 // rank-64G product: S is read and written once per super-step, not once per
 // block row.  A workgroup writes only its own rows and reads rows finished
 // in earlier launches (or by itself), so workgroups of one launch never
-// race.  lower_rhs: S is lower triangular (identity-like right-hand side):
-// the blocks X_c[:, ct] with c < ct are zero and are skipped.
+// race.
 constexpr int TRSM_G = 4;
 
 // acc += sum_{c in [c0, c1)} L(r0.., 64c..) S(64c.., n0..): MFMA tile
@@ -881,7 +876,7 @@ __device__ __forceinline__ void trsm_acc(const T* L, int64_t ld, const T* S, int
 // u < nct solves SS_q for column tile u; the others update one row block.
 template <typename T>
 __device__ __forceinline__ void trsm_ss(const T* L, int64_t ld, const double* dinv, int nb, int q, T* S,
-                        int64_t lds, int nct, int u, int lower_rhs) {
+                        int64_t lds, int nct, int u) {
   constexpr int PP = KP<T>::value;
   constexpr int PB = TILE + 1;
   __shared__ T As[TILE * PP];
@@ -895,10 +890,9 @@ __device__ __forceinline__ void trsm_ss(const T* L, int64_t ld, const double* di
     const int64_t n0 = (int64_t)ct * TILE;
     const int kend = min(G * q + G, nb);
     for (int k = G * q; k < kend; ++k) {
-      if (lower_rhs && ct > k) continue;  // X_k[:, ct] stays zero
       const int64_t r0 = (int64_t)k * TILE;
       zero_acc<T>(acc);
-      trsm_acc<T>(L, ld, S, lds, r0, n0, lower_rhs ? max(p0, ct) : p0, k, G * q, As, Bs, acc);
+      trsm_acc<T>(L, ld, S, lds, r0, n0, p0, k, G * q, As, Bs, acc);
       // B = S_k - acc (rounded to T), A = DINV_k
 #pragma unroll
       for (int bm = 0; bm < 2; ++bm)
@@ -932,11 +926,9 @@ __device__ __forceinline__ void trsm_ss(const T* L, int64_t ld, const double* di
   const int ct = v % nct;
   const int i = G * (q + 1) + v / nct;
   if (q == 0 || i >= nb) return;
-  const int c0 = lower_rhs ? max(p0, ct) : p0;
-  if (c0 >= G * q) return;
   const int64_t r0 = (int64_t)i * TILE, n0 = (int64_t)ct * TILE;
   zero_acc<T>(acc);
-  trsm_acc<T>(L, ld, S, lds, r0, n0, c0, G * q, G * q, As, Bs, acc);
+  trsm_acc<T>(L, ld, S, lds, r0, n0, p0, G * q, G * q, As, Bs, acc);
 #pragma unroll
   for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
@@ -955,23 +947,19 @@ static inline int trsm_units(int nb, int q, int nct) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(NTHREADS) void k_trsm(Prob* const* probs, Sched sc, int q,
-                                                   int lower_rhs) {
+__global__ __launch_bounds__(NTHREADS) void k_trsm(Prob* const* probs, Sched sc, int q) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
-  trsm_ss<T>((const T*)P.L, P.Np, P.dinv, P.Np / TILE, q, (T*)P.S, P.Np, P.Mp / TILE, bx,
-             lower_rhs);
+  trsm_ss<T>((const T*)P.L, P.Np, P.dinv, P.Np / TILE, q, (T*)P.S, P.Np, P.Mp / TILE, bx);
 }
 
-static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, int lower_rhs, hipStream_t s) {
+static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, hipStream_t s) {
   const int nb = bt.maxNp / TILE;
   const bool on = timer_on(TC_TRSM);
   for (int k = 0; k < nb; ++k) {
-    // lower_rhs: column tiles ct > k of an identity-like right-hand side
-    // stay zero, so only ct <= k are scheduled
     auto nct_of = [&](int m) {
       const int mp = bt.hm ? (bt.hm[m] + TILE - 1) / TILE * TILE : maxMp;
-      return lower_rhs ? std::min(k + 1, mp / TILE) : mp / TILE;
+      return mp / TILE;
     };
     sched_launch(
         bt,
@@ -982,9 +970,9 @@ static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, int lower_r
         [&](Prob* const* dp, const Sched& sc, int n) {
           if (on) timer_begin(TC_TRSM, s);
           if (prec == PGP_PREC_FP64)
-            hipLaunchKernelGGL(k_trsm_lagged<double>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, k, lower_rhs);
+            hipLaunchKernelGGL(k_trsm_lagged<double>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, k);
           else
-            hipLaunchKernelGGL(k_trsm_lagged<float>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, k, lower_rhs);
+            hipLaunchKernelGGL(k_trsm_lagged<float>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, k);
           if (on) {
             // step k of an N^2 M-flop solve: the update of rows k.. by block
             // k - 1 (2 * 64 per entry) and the 64-row triangle (64^2 per column)
@@ -1006,9 +994,9 @@ static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, int lower_r
 // schedule.
 constexpr int TRSM_WIDE = 16;
 
-void launch_trsm(const Batch& bt, int prec, int maxMp, int lower_rhs, hipStream_t s) {
+void launch_trsm(const Batch& bt, int prec, int maxMp, hipStream_t s) {
   const int nct = maxMp / TILE;
-  if (!lower_rhs && bt.ticket && nct <= WAVE_NCT && bt.maxNp / TILE <= MAXB && wavefront_trsm()) {
+  if (bt.ticket && nct <= WAVE_NCT && bt.maxNp / TILE <= MAXB && wavefront_trsm()) {
     // row-major schedule: row i holds the members with more than i block
     // rows (a prefix: members are sorted by size), nct workgroups each
     const int nb = bt.maxNp / TILE;
@@ -1043,7 +1031,7 @@ void launch_trsm(const Batch& bt, int prec, int maxMp, int lower_rhs, hipStream_
     return;
   }
   if (maxMp / TILE < TRSM_WIDE) {
-    launch_trsm_lagged(bt, prec, maxMp, lower_rhs, s);
+    launch_trsm_lagged(bt, prec, maxMp, s);
     return;
   }
   const int nb = bt.maxNp / TILE;
@@ -1059,9 +1047,9 @@ void launch_trsm(const Batch& bt, int prec, int maxMp, int lower_rhs, hipStream_
         [&](Prob* const* dp, const Sched& sc, int n) {
           if (on) timer_begin(TC_TRSM, s);
           if (prec == PGP_PREC_FP64)
-            hipLaunchKernelGGL(k_trsm<double>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, q, lower_rhs);
+            hipLaunchKernelGGL(k_trsm<double>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, q);
           else
-            hipLaunchKernelGGL(k_trsm<float>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, q, lower_rhs);
+            hipLaunchKernelGGL(k_trsm<float>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, q);
           if (on) {
             // super-step q of an N^2 M-flop solve: its rows' left-looking
             // products and triangles, and the rank-64G update of the rows
@@ -1086,23 +1074,22 @@ void launch_trsm(const Batch& bt, int prec, int maxMp, int lower_rhs, hipStream_
 
 template <typename T>
 __global__ __launch_bounds__(NTHREADS) void k_trsm_raw(const T* L, int64_t ld, const double* dinv,
-                                                       int nb, int q, T* S, int64_t lds, int nct,
-                                                       int lower_rhs) {
-  trsm_ss<T>(L, ld, dinv, nb, q, S, lds, nct, blockIdx.x, lower_rhs);
+                                                       int nb, int q, T* S, int64_t lds, int nct) {
+  trsm_ss<T>(L, ld, dinv, nb, q, S, lds, nct, blockIdx.x);
 }
 
 int launch_trsm_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const double* dinv,
-                         void* S, int64_t M, int64_t lds, int lower_rhs, hipStream_t s) {
+                         void* S, int64_t M, int64_t lds, hipStream_t s) {
   const int nb = (int)(N / TILE), nct = (int)(M / TILE);
   if (nct < TRSM_WIDE) {
     for (int k = 0; k < nb; ++k) {
       dim3 g(k == 0 ? 1 : nb - k, (unsigned)nct);
       if (prec == PGP_PREC_FP64)
         hipLaunchKernelGGL(k_trsm_lagged_raw<double>, g, dim3(NTHREADS), 0, s, (const double*)L,
-                           ld, dinv, k, (double*)S, lds, lower_rhs);
+                           ld, dinv, k, (double*)S, lds);
       else
         hipLaunchKernelGGL(k_trsm_lagged_raw<float>, g, dim3(NTHREADS), 0, s, (const float*)L, ld,
-                           dinv, k, (float*)S, lds, lower_rhs);
+                           dinv, k, (float*)S, lds);
     }
     return 0;
   }
@@ -1111,10 +1098,10 @@ int launch_trsm_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const d
     const dim3 g((unsigned)trsm_units(nb, q, nct));
     if (prec == PGP_PREC_FP64)
       hipLaunchKernelGGL(k_trsm_raw<double>, g, dim3(NTHREADS), 0, s, (const double*)L, ld, dinv,
-                         nb, q, (double*)S, lds, nct, lower_rhs);
+                         nb, q, (double*)S, lds, nct);
     else
       hipLaunchKernelGGL(k_trsm_raw<float>, g, dim3(NTHREADS), 0, s, (const float*)L, ld, dinv,
-                         nb, q, (float*)S, lds, nct, lower_rhs);
+                         nb, q, (float*)S, lds, nct);
   }
   return 0;
 }

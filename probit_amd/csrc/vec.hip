@@ -25,6 +25,8 @@ __device__ __forceinline__ double wave_sum(double v) {
 // mode 1: out = SF .* Kx              (SF: the W^1/2 of the factored B)
 // mode 2: out = R - DL - S^2 .* Kx     (Laplace residual of (I + W K) d = r, x = DL)
 // mode 3: out = X1 - sigma^2 x - Kx    (VB residual of (sigma^2 I + K) w = rhs, rhs in X1)
+// mode 4: out = Kx / W within [0, K_ii] (K_ii where W = 0): diag of (K^-1 + W)^-1
+//         from the row sums of K o C
 // (modes >= 10: the same with the matrix C in place of K)
 __device__ __forceinline__ void gemv_epilogue(const Prob& P, int i, const double* x, int os,
                                               int mode, double sum) {
@@ -41,6 +43,11 @@ __device__ __forceinline__ void gemv_epilogue(const Prob& P, int i, const double
       v = vslot(P, V_R)[i] - x[i] - si * si * sum;
       break;
     }
+    case 4: {
+      const double W = vslot(P, V_W)[i];
+      v = i >= P.N ? 0.0 : W > 0.0 ? fmin(fmax(sum / W, 0.0), P.variance) : P.variance;
+      break;
+    }
     default: {
       const double s2 = (i < P.N) ? P.noise_std * P.noise_std : 1.0;
       v = vslot(P, V_X1)[i] - s2 * x[i] - sum;
@@ -48,30 +55,6 @@ __device__ __forceinline__ void gemv_epilogue(const Prob& P, int i, const double
     }
   }
   vslot(P, os)[i] = v;
-}
-
-// Full-matrix product, one wave per output (used for the matrix C).
-__global__ __launch_bounds__(NTHREADS) void k_gemv_sym(Prob* const* probs, Sched sc, int xs,
-                                                       int os, int mode) {
-  int bx;
-  const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
-  const int i = bx * 4 + (threadIdx.x >> 6);
-  if (i >= P.Np) return;
-  const int lane = threadIdx.x & 63;
-  const double* col = (mode >= 10 ? P.C : P.K) + (size_t)i * P.Np;
-  mode %= 10;
-  const double* x = vslot(P, xs);
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  int j = lane;
-  for (; j + 192 < P.Np; j += 256) {
-    a0 += col[j] * x[j];
-    a1 += col[j + 64] * x[j + 64];
-    a2 += col[j + 128] * x[j + 128];
-    a3 += col[j + 192] * x[j + 192];
-  }
-  for (; j < P.Np; j += 64) a0 += col[j] * x[j];
-  const double sum = wave_sum((a0 + a1) + (a2 + a3));
-  if (lane == 0) gemv_epilogue(P, i, x, os, mode, sum);
 }
 
 // Symmetric product y = K x reading each lower 64x64 tile of K once: the
@@ -88,6 +71,9 @@ __device__ __forceinline__ void lower_tile_v(int t, int& ti, int& tj) {
   tj = t - i * (i + 1) / 2;
 }
 
+// MAT: the matrix is K, C, or (with x = 1: row sums) K o C.
+enum SymvMat { SYMV_K = 0, SYMV_C = 1, SYMV_HADAMARD = 2 };
+template <int MAT>
 __global__ __launch_bounds__(NTHREADS) void k_symv_tiles(Prob* const* probs, Sched sc, int xs) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
@@ -99,16 +85,26 @@ __global__ __launch_bounds__(NTHREADS) void k_symv_tiles(Prob* const* probs, Sch
   const size_t ld = (size_t)P.Np;
   const int r = threadIdx.x & 63, w = threadIdx.x >> 6;
   const double* x = vslot(P, xs);
-  const double* Kt = P.K + (size_t)ti * TILE + (size_t)tj * TILE * ld;
+  const size_t tile = (size_t)ti * TILE + (size_t)tj * TILE * ld;
+  const double* Kt = (MAT == SYMV_C ? P.C : P.K) + tile;
   // lane r holds row r of the wave's 16 columns c = w + 4q (coalesced down
   // each column); the tile never goes through LDS
   double k[16];
 #pragma unroll
   for (int q = 0; q < 16; ++q) k[q] = Kt[(size_t)r + (size_t)(w + 4 * q) * ld];
-  const double xi = x[ti * TILE + r];
+  if constexpr (MAT == SYMV_HADAMARD) {
+    const double* Ct = P.C + tile;
+    double c[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) c[q] = Ct[(size_t)r + (size_t)(w + 4 * q) * ld];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) k[q] *= c[q];
+  }
+  const double xi = MAT == SYMV_HADAMARD ? 1.0 : x[ti * TILE + r];
   double rs = 0.0;
 #pragma unroll
-  for (int q = 0; q < 16; ++q) rs += k[q] * x[tj * TILE + w + 4 * q];
+  for (int q = 0; q < 16; ++q)
+    rs += MAT == SYMV_HADAMARD ? k[q] : k[q] * x[tj * TILE + w + 4 * q];
   rpart[w][r] = rs;
   double* part = P.symv;
   if (ti != tj) {
@@ -157,21 +153,8 @@ __global__ __launch_bounds__(NTHREADS) void k_symv_reduce(Prob* const* probs, Sc
   gemv_epilogue(P, i, vslot(P, xs), os, mode, a0 + a1);
 }
 
-void launch_gemv_sym(const Batch& b, int x_slot, int out_slot, int mode, hipStream_t s) {
-  if (mode >= 10) {
-    sched_launch(
-        b, [&](int m) { return (b.np(m) + 3) / 4; },
-        [&](Prob* const* dp, const Sched& sc, int n) {
-          hipLaunchKernelGGL(k_gemv_sym, dim3(n), dim3(NTHREADS), 0, s, dp, sc, x_slot, out_slot,
-                             mode);
-        });
-    return;
-  }
-  launch_symv_tiles(b, x_slot, s);
-  launch_symv_reduce(b, x_slot, out_slot, mode, s);
-}
-
-void launch_symv_tiles(const Batch& b, int x_slot, hipStream_t s) {
+template <int MAT>
+static void symv_tiles(const Batch& b, int x_slot, hipStream_t s) {
   sched_launch(
       b,
       [&](int m) {
@@ -179,8 +162,24 @@ void launch_symv_tiles(const Batch& b, int x_slot, hipStream_t s) {
         return t * (t + 1) / 2;
       },
       [&](Prob* const* dp, const Sched& sc, int n) {
-        hipLaunchKernelGGL(k_symv_tiles, dim3(n), dim3(NTHREADS), 0, s, dp, sc, x_slot);
+        hipLaunchKernelGGL(k_symv_tiles<MAT>, dim3(n), dim3(NTHREADS), 0, s, dp, sc, x_slot);
       });
+}
+
+void launch_gemv_sym(const Batch& b, int x_slot, int out_slot, int mode, hipStream_t s) {
+  if (mode >= 10)
+    symv_tiles<SYMV_C>(b, x_slot, s);
+  else
+    symv_tiles<SYMV_K>(b, x_slot, s);
+  launch_symv_reduce(b, x_slot, out_slot, mode % 10, s);
+}
+
+void launch_symv_tiles(const Batch& b, int x_slot, hipStream_t s) {
+  symv_tiles<SYMV_K>(b, x_slot, s);
+}
+
+void launch_hadamard_tiles(const Batch& b, hipStream_t s) {
+  symv_tiles<SYMV_HADAMARD>(b, V_X1, s);
 }
 
 void launch_symv_reduce(const Batch& b, int x_slot, int out_slot, int mode, hipStream_t s) {

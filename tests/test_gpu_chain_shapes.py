@@ -37,3 +37,27 @@ def test_fit_at_schedule_edges(N, mode, tol, vtol):
     m_ref, v_ref = O.predict(spec, X, Xt, w_ref, p_ref)
     assert rel_err(mean.cpu().numpy(), m_ref) < tol
     assert rel_err(var.cpu().numpy(), v_ref) < vtol
+
+
+# the gradient's tolerance against the closed form of the oracle
+# (tests/test_gpu_laplace.py: 1e-7)
+@pytest.mark.parametrize("N", [64, 130, 200, 321, 577])
+@pytest.mark.parametrize("lik", ["gaussian", "probit"])
+def test_gradient_at_doubling_edges(N, lik):
+    import probit_amd as P
+    D = 2
+    X, y, theta, lp, spec = small_problem(N, N, D, lik)
+    ll = P.log_gaussian_likelihood if lik == "gaussian" else P.log_probit_likelihood
+    gp = P.LaplaceGP(data=(X, y), prior=make_prior("EQ"), log_likelihood=ll, tolerance=1e-11)
+    val, ((g_ls, g_var), g_lik) = gp.value_and_grad()((theta, lp))
+    K = O.gram(spec, X)
+    w = O.laplace_weight_converged(K, y, lik_kind(lik), lp)
+    ref = O.laplace_objective_gradient(spec, X, y, lik_kind(lik), lp, w)
+    ref_ls = sum(ref[f"lengthscale{d}"] for d in range(D))
+    assert abs(val - O.objective_LA(spec, X, y, lik_kind(lik), lp, w)) < 1e-9 * abs(val)
+    for got, want in [(g_ls, ref_ls), (g_var, ref["variance"]), (g_lik[0], ref["noise_std"])]:
+        assert abs(got - want) <= 1e-7 * max(1.0, abs(want))
+    if lik == "probit":
+        cut = np.asarray(g_lik[1])[1:-1]
+        want = np.asarray(ref["cutpoints"])[1:-1]
+        assert np.max(np.abs(cut - want)) <= 1e-7 * max(1.0, np.max(np.abs(want)))
