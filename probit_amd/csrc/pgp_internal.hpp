@@ -327,12 +327,17 @@ int launch_potrf_raw(int prec, void* A, int64_t N, int64_t ld, double* dinv, dou
                      int32_t* info, hipStream_t s);
 
 // Prior sampling workspace (padded size Np): K / its factor (Np x Np FP64),
-// the diagonal-block inverses (Np x 64 FP64), the factor status word.
+// the diagonal-block inverses (Np x 64 FP64), then a page with the factor's
+// descriptor, pointer array, status word and ticket counter, and its sync
+// words.
 inline int64_t prior_ws_offset_dinv(int64_t Np) { return (Np * Np * 8 + 255) / 256 * 256; }
-inline int64_t prior_ws_offset_info(int64_t Np) {
+inline int64_t prior_ws_offset_page(int64_t Np) {
   return prior_ws_offset_dinv(Np) + (Np * TILE * 8 + 255) / 256 * 256;
 }
-inline int64_t prior_ws_bytes(int64_t Np) { return prior_ws_offset_info(Np) + 256; }
+inline int64_t prior_ws_offset_csync(int64_t Np) { return prior_ws_offset_page(Np) + 4096; }
+inline int64_t prior_ws_bytes(int64_t Np) {
+  return prior_ws_offset_csync(Np) + (csync_words(Np) * 4 + 255) / 256 * 256;
+}
 int launch_prior_sample(const pgp_kernel_t* kernel, const double* X, int64_t N, double jitter,
                         const double* z, int64_t S, int64_t ldz, double* f, int64_t ldf,
                         char* ws, hipStream_t s);
