@@ -75,8 +75,9 @@ constexpr int64_t OFF_RED = 2176;   // double[NRED]
 constexpr int64_t OFF_GATHER = 2432;  // double[8] scratch for reductions
 constexpr int64_t OFF_PROGRESS = 2496;  // uint64 progress word of the wavefront solves
 constexpr int64_t OFF_TICKET = 2504;    // uint32 workgroup-order counter (single-problem launches)
-constexpr int64_t OFF_PROGRESS_CT = 2560;  // uint64[4] progress words of the wavefront TRSM
+constexpr int64_t OFF_PROGRESS_CT = 2560;  // uint64[PROGRESS_CT] words of the wavefront TRSM
 constexpr int64_t HEADER = 4096;
+static_assert(OFF_PROGRESS_CT + 8 * PROGRESS_CT <= HEADER, "progress words fit the header");
 
 struct WsLayout {
   int64_t Np, K, L, logdiag, diagval, dinv, vec, symv, csync, xpub, panel16, total;
@@ -190,7 +191,8 @@ __global__ void k_write_prob(Prob* dst, Prob val, int reset) {
     if (threadIdx.x < NRED) val.red[threadIdx.x] = 0.0;
     // progress word and ticket counter of the header
     if (threadIdx.x < 2) reinterpret_cast<uint64_t*>((char*)dst + OFF_PROGRESS)[threadIdx.x] = 0;
-    if (threadIdx.x < 4) reinterpret_cast<uint64_t*>((char*)dst + OFF_PROGRESS_CT)[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < PROGRESS_CT; i += blockDim.x)
+      reinterpret_cast<uint64_t*>((char*)dst + OFF_PROGRESS_CT)[i] = 0;
     if (val.csync)
       for (int64_t w = threadIdx.x; w < csync_words(val.Np); w += blockDim.x) val.csync[w] = 0;
   }
@@ -222,7 +224,7 @@ __global__ void k_scatter_probs(Prob* const* dst, const Prob* src, int n, int re
     if (threadIdx.x < 4) v.info[threadIdx.x] = 0;
     if (threadIdx.x < NRED) v.red[threadIdx.x] = 0.0;
     if (threadIdx.x == 0) v.progress[0] = 0;
-    if (threadIdx.x < 4) v.progress_ct[threadIdx.x] = 0;
+    for (int w = threadIdx.x; w < PROGRESS_CT; w += blockDim.x) v.progress_ct[w] = 0;
     if (v.csync)
       for (int64_t w = threadIdx.x; w < csync_words(v.Np); w += blockDim.x) v.csync[w] = 0;
   }

@@ -98,7 +98,8 @@ struct Prob {
   uint64_t* xpub;
   // symmetric products: per-tile partial sums, (Np/64) x (Np/64) x 64
   double* symv;
-  // wavefront TRSM: one progress word per right-hand-side column tile (4)
+  // wavefront TRSM: one progress word per right-hand-side column tile of a
+  // launch (PROGRESS_CT)
   uint64_t* progress_ct;
   // predict with the FP64 variance correction: (Np/64) x Mp partial sums
   // (NULL: the variance from the column norms of L^-1 S)
@@ -135,6 +136,7 @@ struct Batch {
 // launch holds exactly the workgroups that have work, whatever the spread of
 // member sizes.  Passed by value as a kernel argument.
 constexpr int MAXB = 512;  // members per launch; larger batches are split
+constexpr int PROGRESS_CT = 128;  // column tiles of one wavefront TRSM launch
 struct Sched {
   int32_t count;
   int32_t pre[MAXB + 1];

@@ -444,10 +444,13 @@ int launch_trsv_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const d
 }
 
 // ---- TRSM: S <- L^-1 S, S is Np x Mp (ld lds) ----
-// Two schedules.  For narrow right-hand sides (a few column tiles, as in
-// serving) one launch per block row keeps every launch to two short tile
-// products per workgroup; for wide ones the super-step schedule below reads
-// and writes S G times less often.
+// FP64 solves, the transposed solves, and FP32 solves of at most WAVE_NCT
+// column tiles (serving) run as one wavefront launch (k_trsm_rows, below).
+// The others, wider FP32 solves, take a launch per block row (up to TRSM_WIDE
+// column tiles) or per super-step of G block rows: they subtract each block
+// row's (super-step's) product from S in FP32, and a wavefront's one sum over
+// all of them would round differently.  So do solves without a ticket
+// counter, or on a bare matrix.
 //
 // Per block row (lagged).
 // Lagged schedule.  Launch k, workgroup (w, ct), row block i = k + w:
@@ -540,19 +543,29 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged_raw(const T* L, int64_
   trsm_step<T>(L, ld, dinv, k, S, lds, blockIdx.x, blockIdx.y);
 }
 
-// Wavefront TRSM for narrow right-hand sides (at most WAVE_NCT column
-// tiles), all members in one launch: one workgroup per (block row i,
-// member, column tile ct), numbered row-major so that the wave front moves
-// through every member at once.  Workgroup (i, ct) accumulates L_ij X_j[:, ct]
-// for every block j < i as soon as (j, ct) publishes, then forms
-// X_i = DINV_i (S_i - acc) and publishes it: X_i through agent-scope stores,
-// a wait for their completion, then the member's progress word of column
-// tile ct.  Start-order tickets and bounded waits as in k_trsv_seg.
+// Wavefront TRSM for the column tiles [ct0, ct0 + nct) (nct <= PROGRESS_CT),
+// all members in one launch: one workgroup per (block row i, member, column
+// tile ct), numbered row-major so that the wave front moves through every
+// member and column tile at once.  Workgroup (i, ct) accumulates L_ij X_j[:,
+// ct] for every block j < i as soon as (j, ct) publishes, then forms X_i =
+// DINV_i (S_i - acc) and publishes it: X_i through agent-scope stores, a wait
+// for their completion, then the member's progress word of column tile ct.
+// S is read and written once.  Start-order tickets and bounded waits as in
+// k_trsv_seg.
+//
+// Bound by the tile products once a row's work (nct products per earlier
+// block, over 256 CUs) exceeds the chain's step (the last product, DINV's and
+// the hand-off, ~9 us); FP64 at N = 3000, M = 5000: 2400 us as 12 super-step
+// launches, whose solving workgroups run 30 tile products in a row; 1712 in
+// one wavefront launch; 1235 (37 TFLOP/s) with the operands fetched a product
+// ahead.  N = 1537, M = 501: 590 -> 269 us.  Transposed, FP32 at N = 8192, M =
+// 4096: 20.3 ms in 16 launches of 4 column tiles, 3.5 ms (79 TFLOP/s) in one.
 constexpr int WAVE_NCT = 4;
 
 template <typename T>
 __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sched rows, int nct,
-                                                        uint32_t* ticket, uint32_t epoch) {
+                                                        int ct0, uint32_t* ticket,
+                                                        uint32_t epoch) {
   constexpr int PP = KP<T>::value;  // A operand: conflict-free MFMA reads
   constexpr int PB = TILE + 1;       // B operand: written transposed, conflict-free stores
   __shared__ T As[TILE * PP];
@@ -566,38 +579,52 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
   }
   int local;
   const int i = sched_member(rows, tk, local);
-  const int m = local / nct, ct = local - m * nct;
+  const int m = local / nct, lct = local - m * nct, ct = ct0 + lct;
   const Prob& P = *probs[m];
   if (ct >= P.Mp / TILE || i >= P.Np / TILE) return;
-  uint64_t* prog = P.progress_ct + ct;
+  uint64_t* prog = P.progress_ct + lct;
   const auto L = gbl((const T*)P.L);
-  T* S = (T*)P.S;
+  const auto S = gbl((T*)P.S);
   const int64_t ld = P.Np;
   const int64_t ri = (int64_t)i * TILE, n0 = (int64_t)ct * TILE;
-  const int r = threadIdx.x & 63, cb = threadIdx.x >> 6;
-  // Operands that exist before the launch are fetched into registers ahead
-  // of the waits: DINV_i and S_i at once, the next L_ij while X_j is awaited.
-  T dv[16], la[16], sv[2][2][4];
-  {
-    const auto D = gbl(P.dinv + (size_t)i * TILE * TILE);
-    const auto Sg = gbl((const T*)P.S);
+  const unsigned r = threadIdx.x & 63;
+  const int cb = uniform((int)(threadIdx.x >> 6));
+  // la: the next A operand (L_ij, at last DINV_i), fetched during the
+  // product before its own; xb: the next X_j, fetched as early when it is
+  // known to be published, and during the last product S_i.
+  T la[16], xb[16];
+  auto fetch_l = [&](int k) {
+    auto p = L + (ri + ((int64_t)k * TILE + cb) * ld);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) dv[q] = (T)D[r + (size_t)(cb + 4 * q) * TILE];
+    for (int q = 0; q < 16; ++q, p += 4 * ld) la[q] = p[r];
+  };
+  auto fetch_d = [&]() {
+    const auto D = gbl(P.dinv + (size_t)i * TILE * TILE + (size_t)cb * TILE);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) la[q] = (T)D[r + (size_t)(4 * q) * TILE];
+  };
+  auto fetch_s = [&]() {  // accumulator layout
 #pragma unroll
     for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
       for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          sv[bm][bn][q] =
-              Sg[(size_t)(ri + acc_row<T>(bm, q)) + (size_t)(n0 + acc_col(bn)) * ld];
-  }
-  auto fetch_l = [&](int j) {
-#pragma unroll
-    for (int q = 0; q < 16; ++q)
-      la[q] = L[(size_t)(ri + r) + (size_t)((int64_t)j * TILE + cb + 4 * q) * ld];
+          xb[8 * bm + 4 * bn + q] =
+              S[(size_t)(ri + acc_row<T>(bm, q)) + (size_t)(n0 + acc_col(bn)) * ld];
   };
-  if (i > 0) fetch_l(0);
+  auto fetch_x = [&](int k) {  // published in this launch: coherent loads
+    auto p = S + ((int64_t)k * TILE + (n0 + cb) * ld);
+#pragma unroll
+    for (int q = 0; q < 16; ++q, p += 4 * ld)
+      xb[q] = __hip_atomic_load(p + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (i > 0) {
+    fetch_l(0);
+  } else {
+    fetch_d();
+    fetch_s();
+  }
   acc_t acc[2][2];
   zero_acc<T>(acc);
   int done = 0, ready = 0;
@@ -607,23 +634,24 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
       if (threadIdx.x == 0) s_val = wait_progress(prog, epoch, done + 1, P.info);
       __syncthreads();
       ready = min(__builtin_amdgcn_readfirstlane(s_val), i);
+      fetch_x(done);
     }
-    for (; done < ready; ++done) {
-      const int64_t rj = (int64_t)done * TILE;
-      __syncthreads();  // the previous product is done with LDS
+    __syncthreads();  // the previous product is done with LDS
 #pragma unroll
-      for (int q = 0; q < 16; ++q) As[(cb + 4 * q) * PP + r] = la[q];
-      // B[kk][n] = X_j(kk, n), published in this launch: coherent loads
-#pragma unroll 4
-      for (int q = 0; q < 16; ++q) {
-        const int c = cb + 4 * q;
-        Bs[r * PB + c] = __hip_atomic_load(&S[(size_t)(rj + r) + (size_t)(n0 + c) * ld],
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      if (done + 1 < i) fetch_l(done + 1);
-      __syncthreads();
-      mma64_kmajor<T>(As, PP, Bs, PB, acc);
+    for (int q = 0; q < 16; ++q) {
+      As[(cb + 4 * q) * PP + r] = la[q];
+      Bs[r * PB + cb + 4 * q] = xb[q];  // B(k, n) = X_j(k, n)
     }
+    ++done;
+    if (done < i) {
+      fetch_l(done);
+      if (done < ready) fetch_x(done);
+    } else {
+      fetch_d();
+      fetch_s();
+    }
+    __syncthreads();
+    mma64_kmajor<T>(As, PP, Bs, PB, acc);
   }
   // X_i = DINV_i (S_i - acc)
   __syncthreads();
@@ -634,10 +662,10 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int row = acc_row<T>(bm, q), col = acc_col(bn);
-        Bs[row * PB + col] = sv[bm][bn][q] - acc[bm][bn][q];
+        Bs[row * PB + col] = xb[8 * bm + 4 * bn + q] - acc[bm][bn][q];
       }
 #pragma unroll
-  for (int q = 0; q < 16; ++q) As[(cb + 4 * q) * PP + r] = dv[q];
+  for (int q = 0; q < 16; ++q) As[(cb + 4 * q) * PP + r] = la[q];
   __syncthreads();
   zero_acc<T>(acc);
   mma64_kmajor<T>(As, PP, Bs, PB, acc);
@@ -657,7 +685,7 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
 }
 
 // Transposed wavefront TRSM: X <- L^-T X in place on the predict buffer S,
-// for the column tiles [ct0, ct0 + nct) (nct <= WAVE_NCT), all members in
+// for the column tiles [ct0, ct0 + nct) (nct <= PROGRESS_CT), all members in
 // one launch.  Step t of a member is its block row i = nb - 1 - t (the sweep
 // runs from the last block row up): workgroup (t, member, ct) accumulates
 // L_ji^T X_j[:, ct] for every j > i as soon as step nb - 1 - j publishes,
@@ -688,32 +716,48 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
   const int i = nb - 1 - t;
   uint64_t* prog = P.progress_ct + lct;
   const auto L = gbl((const T*)P.L);
-  T* S = (T*)P.S;
+  const auto S = gbl((T*)P.S);
   const int64_t ld = P.Np;
   const int64_t ri = (int64_t)i * TILE, n0 = (int64_t)ct * TILE;
-  const int r = threadIdx.x & 63, cb = threadIdx.x >> 6;
-  T dv[16], la[16], sv[2][2][4];
-  {
-    const auto D = gbl(P.dinv + (size_t)i * TILE * TILE);
-    const auto Sg = gbl((const T*)P.S);
+  const unsigned r = threadIdx.x & 63;
+  const int cb = uniform((int)(threadIdx.x >> 6));
+  // la: the next A operand (L_ji, at last DINV_i), fetched during the
+  // product before its own; xb: the next X_j, fetched as early when it is
+  // known to be published, and during the last product S_i.
+  T la[16], xb[16];
+  // fetch_l(k): la[q] = L_ji(r, cb + 4q), j = nb - 1 - k: A(m, k) = L_ji(k, m)
+  auto fetch_l = [&](int k) {
+    auto p = L + ((int64_t)(nb - 1 - k) * TILE + (ri + cb) * ld);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) dv[q] = (T)D[r + (size_t)(cb + 4 * q) * TILE];
+    for (int q = 0; q < 16; ++q, p += 4 * ld) la[q] = p[r];
+  };
+  auto fetch_d = [&]() {
+    const auto D = gbl(P.dinv + (size_t)i * TILE * TILE + (size_t)cb * TILE);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) la[q] = (T)D[r + (size_t)(4 * q) * TILE];
+  };
+  auto fetch_s = [&]() {  // accumulator layout
 #pragma unroll
     for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
       for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          sv[bm][bn][q] =
-              Sg[(size_t)(ri + acc_row<T>(bm, q)) + (size_t)(n0 + acc_col(bn)) * ld];
-  }
-  // la[q] = L_ji(r, cb + 4q) = L(64 j + r, 64 i + cb + 4q): A(m, k) = L_ji(k, m)
-  auto fetch_l = [&](int j) {
-#pragma unroll
-    for (int q = 0; q < 16; ++q)
-      la[q] = L[(size_t)((int64_t)j * TILE + r) + (size_t)(ri + cb + 4 * q) * ld];
+          xb[8 * bm + 4 * bn + q] =
+              S[(size_t)(ri + acc_row<T>(bm, q)) + (size_t)(n0 + acc_col(bn)) * ld];
   };
-  if (t > 0) fetch_l(nb - 1);
+  auto fetch_x = [&](int k) {  // published in this launch: coherent loads
+    auto p = S + ((int64_t)(nb - 1 - k) * TILE + (n0 + cb) * ld);
+#pragma unroll
+    for (int q = 0; q < 16; ++q, p += 4 * ld)
+      xb[q] = __hip_atomic_load(p + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (t > 0) {
+    fetch_l(0);
+  } else {
+    fetch_d();
+    fetch_s();
+  }
   acc_t acc[2][2];
   zero_acc<T>(acc);
   int done = 0, ready = 0;
@@ -723,23 +767,24 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
       if (threadIdx.x == 0) s_val = wait_progress(prog, epoch, done + 1, P.info);
       __syncthreads();
       ready = min(__builtin_amdgcn_readfirstlane(s_val), t);
+      fetch_x(done);
     }
-    for (; done < ready; ++done) {
-      const int64_t rj = (int64_t)(nb - 1 - done) * TILE;
-      __syncthreads();  // the previous product is done with LDS
+    __syncthreads();  // the previous product is done with LDS
 #pragma unroll
-      for (int q = 0; q < 16; ++q) As[r * PA + cb + 4 * q] = la[q];
-      // B[kk][n] = X_j(kk, n), published in this launch: coherent loads
-#pragma unroll 4
-      for (int q = 0; q < 16; ++q) {
-        const int c = cb + 4 * q;
-        Bs[r * PB + c] = __hip_atomic_load(&S[(size_t)(rj + r) + (size_t)(n0 + c) * ld],
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      if (done + 1 < t) fetch_l(nb - 2 - done);
-      __syncthreads();
-      mma64_kmajor<T>(As, PA, Bs, PB, acc);
+    for (int q = 0; q < 16; ++q) {
+      As[r * PA + cb + 4 * q] = la[q];
+      Bs[r * PB + cb + 4 * q] = xb[q];  // B(k, n) = X_j(k, n)
     }
+    ++done;
+    if (done < t) {
+      fetch_l(done);
+      if (done < ready) fetch_x(done);
+    } else {
+      fetch_d();
+      fetch_s();
+    }
+    __syncthreads();
+    mma64_kmajor<T>(As, PA, Bs, PB, acc);
   }
   // X_i = DINV_i^T (X_i - acc)
   __syncthreads();
@@ -750,10 +795,10 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int row = acc_row<T>(bm, q), col = acc_col(bn);
-        Bs[row * PB + col] = sv[bm][bn][q] - acc[bm][bn][q];
+        Bs[row * PB + col] = xb[8 * bm + 4 * bn + q] - acc[bm][bn][q];
       }
 #pragma unroll
-  for (int q = 0; q < 16; ++q) As[r * PA + cb + 4 * q] = dv[q];  // A(m, k) = DINV_i(k, m)
+  for (int q = 0; q < 16; ++q) As[r * PA + cb + 4 * q] = la[q];  // A(m, k) = DINV_i(k, m)
   __syncthreads();
   zero_acc<T>(acc);
   mma64_kmajor<T>(As, PA, Bs, PB, acc);
@@ -773,12 +818,12 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
 }
 
 // S <- L^-T S for every member's Mp right-hand sides (Mp <= maxMp): one
-// wavefront launch per group of WAVE_NCT column tiles.
+// wavefront launch per group of PROGRESS_CT column tiles.
 void launch_trsm_t(const Batch& bt, int prec, int maxMp, hipStream_t s) {
   const int nb = bt.maxNp / TILE;
   const int mt = maxMp / TILE;
-  for (int ct0 = 0; ct0 < mt; ct0 += WAVE_NCT) {
-    const int nct = std::min(WAVE_NCT, mt - ct0);
+  for (int ct0 = 0; ct0 < mt; ct0 += PROGRESS_CT) {
+    const int nct = std::min(PROGRESS_CT, mt - ct0);
     Sched rows;
     rows.count = nb;
     int tot = 0;
@@ -995,39 +1040,43 @@ static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, hipStream_t
 constexpr int TRSM_WIDE = 16;
 
 void launch_trsm(const Batch& bt, int prec, int maxMp, hipStream_t s) {
-  const int nct = maxMp / TILE;
-  if (bt.ticket && nct <= WAVE_NCT && bt.maxNp / TILE <= MAXB && wavefront_trsm()) {
-    // row-major schedule: row i holds the members with more than i block
-    // rows (a prefix: members are sorted by size), nct workgroups each
-    const int nb = bt.maxNp / TILE;
-    Sched rows;
-    rows.count = nb;
-    int tot = 0;
-    double fl = 0.0;
-    for (int i = 0; i < nb; ++i) {
-      rows.pre[i] = tot;
-      for (int m = 0; m < bt.count; ++m)
-        if (bt.np(m) / TILE > i) tot += nct;
-    }
-    rows.pre[nb] = tot;
-    if (tot == 0) return;
-    const bool on = timer_on(TC_TRSM);
-    if (on) {
-      for (int m = 0; m < bt.count; ++m) {
-        const double np = bt.np(m);
-        const double mp = bt.hm ? (bt.hm[m] + TILE - 1) / TILE * TILE : maxMp;
-        fl += np * np * mp;
+  const int mt = maxMp / TILE;
+  if (bt.ticket && (prec == PGP_PREC_FP64 || mt <= WAVE_NCT) && bt.maxNp / TILE <= MAXB &&
+      wavefront_trsm()) {
+    for (int ct0 = 0; ct0 < mt; ct0 += PROGRESS_CT) {
+      // row-major schedule: row i holds the members with more than i block
+      // rows (a prefix: members are sorted by size), nct workgroups each
+      const int nct = std::min(PROGRESS_CT, mt - ct0);
+      const int nb = bt.maxNp / TILE;
+      Sched rows;
+      rows.count = nb;
+      int tot = 0;
+      double fl = 0.0;
+      for (int i = 0; i < nb; ++i) {
+        rows.pre[i] = tot;
+        for (int m = 0; m < bt.count; ++m)
+          if (bt.np(m) / TILE > i) tot += nct;
       }
-      timer_begin(TC_TRSM, s);
+      rows.pre[nb] = tot;
+      if (tot == 0) return;
+      const bool on = timer_on(TC_TRSM);
+      if (on) {
+        for (int m = 0; m < bt.count; ++m) {
+          const double np = bt.np(m);
+          const int mm = bt.hm ? (bt.hm[m] + TILE - 1) / TILE : mt;
+          fl += np * np * TILE * std::max(0, std::min(nct, mm - ct0));
+        }
+        timer_begin(TC_TRSM, s);
+      }
+      const uint32_t ep = next_epoch();
+      if (prec == PGP_PREC_FP64)
+        hipLaunchKernelGGL(k_trsm_rows<double>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
+                           nct, ct0, bt.ticket, ep);
+      else
+        hipLaunchKernelGGL(k_trsm_rows<float>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
+                           nct, ct0, bt.ticket, ep);
+      if (on) timer_end(TC_TRSM, s, fl, 0.0);
     }
-    const uint32_t ep = next_epoch();
-    if (prec == PGP_PREC_FP64)
-      hipLaunchKernelGGL(k_trsm_rows<double>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                         nct, bt.ticket, ep);
-    else
-      hipLaunchKernelGGL(k_trsm_rows<float>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                         nct, bt.ticket, ep);
-    if (on) timer_end(TC_TRSM, s, fl, 0.0);
     return;
   }
   if (maxMp / TILE < TRSM_WIDE) {

@@ -61,3 +61,24 @@ def test_gradient_at_doubling_edges(N, lik):
         cut = np.asarray(g_lik[1])[1:-1]
         want = np.asarray(ref["cutpoints"])[1:-1]
         assert np.max(np.abs(cut - want)) <= 1e-7 * max(1.0, np.max(np.abs(want)))
+
+
+# the wide solves of predict: one block row, whole and ragged column tiles,
+# and the edge of a launch's 128 column tiles (the fit's tolerances above)
+@pytest.mark.parametrize("N,M", [(64, 300), (65, 1025), (300, 8192), (300, 8193), (130, 16449)])
+@pytest.mark.parametrize("mode,tol,vtol", [("fp64", 1e-9, 1e-9), ("fp32", 1e-5, 1e-5)])
+def test_predict_at_column_tile_edges(N, M, mode, tol, vtol):
+    import probit_amd as P
+    D = 2
+    X, y, theta, lp, spec = small_problem(N, N, D, "probit")
+    gp = P.LaplaceGP(data=(X, y), prior=make_prior("EQ"), precision_mode=mode,
+                     log_likelihood=P.log_probit_likelihood, tolerance=1e-8)
+    w, p = gp.approximate_posterior((theta, lp))
+    K = O.gram(spec, X)
+    w_ref, _, _ = O.laplace_weight(K, y, lik_kind("probit"), lp, tol=1e-8)
+    p_ref, _ = O.laplace_precision(K, y, lik_kind("probit"), lp, w_ref)
+    Xt = np.random.default_rng(M).normal(size=(M, D))
+    mean, var = gp.predict(Xt, (theta, lp), w, p)
+    m_ref, v_ref = O.predict(spec, X, Xt, w_ref, p_ref)
+    assert rel_err(mean.cpu().numpy(), m_ref) < tol
+    assert rel_err(var.cpu().numpy(), v_ref) < vtol
