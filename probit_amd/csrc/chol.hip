@@ -479,12 +479,14 @@ __device__ __forceinline__ void syrk_tile_multi(T* A_, int64_t ld, int kc0, int 
   LT* sa = (LT*)arena;
   LT* sb = sa + TILE * PITCH;
   typedef typename Acc<T>::type acc_t;
-  const int m = threadIdx.x & 63, kb = threadIdx.x >> 6;
+  const unsigned m = threadIdx.x & 63;
+  const int kb = uniform((int)(threadIdx.x >> 6));
   T ra[16], rb[16];
   acc_t acc[2][2];
   zero_acc<T>(acc);
   // the m-major FP32 and BF16 stagings take 16 consecutive k per thread
   constexpr bool CK = MM || BF16;
+  constexpr int KS = CK ? 1 : 4;
   u16x8 ua[2], ub[2];  // SH: a thread's 16 BF16 operand values of each row
   auto fetch = [&](int c) {
     if constexpr (SH) {
@@ -496,12 +498,12 @@ __device__ __forceinline__ void syrk_tile_multi(T* A_, int64_t ld, int kc0, int 
       ub[0] = *(const u16x8*)pb;
       ub[1] = *(const u16x8*)(pb + 8);
     } else {
-      const int64_t c0 = (int64_t)c * TILE;
+      auto pa = A + (ri + ((int64_t)c * TILE + operand_k<CK>(kb, 0)) * ld);
+      auto pb = A + (rj + ((int64_t)c * TILE + operand_k<CK>(kb, 0)) * ld);
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int k = operand_k<CK>(kb, q);
-        ra[q] = A[(size_t)(ri + m) + (size_t)(c0 + k) * ld];
-        rb[q] = A[(size_t)(rj + m) + (size_t)(c0 + k) * ld];
+      for (int q = 0; q < 16; ++q, pa += KS * ld, pb += KS * ld) {
+        ra[q] = pa[m];
+        rb[q] = pb[m];
       }
     }
   };

@@ -459,7 +459,7 @@ __global__ __launch_bounds__(NTHREADS) void k_pred_refine(Prob* const* probs, Sc
     }
     __syncthreads();
     if (k0 + KC < kend + TILE) fetch(k0 + KC);
-    mma64_kmajor_k32<double>(sa, PA, sb, PA, acc);
+    mma64_kmajor<double, KC / 4>(sa, PA, sb, PA, acc);
   }
   __syncthreads();  // operands are dead: the input rows take their place
   double* xs = sa;

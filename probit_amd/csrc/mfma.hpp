@@ -67,46 +67,35 @@ __device__ __forceinline__ void zero_acc(typename Acc<T>::type (&acc)[2][2]) {
       for (int r = 0; r < 4; ++r) acc[i][j][r] = (T)0;
 }
 
-// acc += A B over K = 64, k-major LDS operands (double / float).
-template <typename T>
+// acc += A B over K = 4 STEPS, k-major LDS operands (double / float).  The
+// operands of a step are read while the previous step's four MFMAs run: left
+// to itself the compiler reads them right before their use, and every step
+// then waits for LDS.
+template <typename T, int STEPS = 16>
 __device__ __forceinline__ void mma64_kmajor(const T* As, int pa, const T* Bs, int pb,
                                              typename Acc<T>::type (&acc)[2][2]) {
   const int l = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int wr = 32 * (w >> 1), wc = 32 * (w & 1);
   const int lr = l & 15, lk = l >> 4;
-#pragma unroll 4
-  for (int kk = 0; kk < 64; kk += 4) {
-    const T a0 = As[(kk + lk) * pa + wr + lr];
-    const T a1 = As[(kk + lk) * pa + wr + 16 + lr];
-    const T b0 = Bs[(kk + lk) * pb + wc + lr];
-    const T b1 = Bs[(kk + lk) * pb + wc + 16 + lr];
-    acc[0][0] = mfma16(a0, b0, acc[0][0]);
-    acc[0][1] = mfma16(a0, b1, acc[0][1]);
-    acc[1][0] = mfma16(a1, b0, acc[1][0]);
-    acc[1][1] = mfma16(a1, b1, acc[1][1]);
-  }
-}
-
-// mma64_kmajor over K = 32 (k-major operands of 32 rows): the first or the
-// second half of mma64_kmajor's k steps, in the same order.
-template <typename T>
-__device__ __forceinline__ void mma64_kmajor_k32(const T* As, int pa, const T* Bs, int pb,
-                                                 typename Acc<T>::type (&acc)[2][2]) {
-  const int l = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-  const int wr = 32 * (w >> 1), wc = 32 * (w & 1);
-  const int lr = l & 15, lk = l >> 4;
-#pragma unroll 4
-  for (int kk = 0; kk < 32; kk += 4) {
-    const T a0 = As[(kk + lk) * pa + wr + lr];
-    const T a1 = As[(kk + lk) * pa + wr + 16 + lr];
-    const T b0 = Bs[(kk + lk) * pb + wc + lr];
-    const T b1 = Bs[(kk + lk) * pb + wc + 16 + lr];
-    acc[0][0] = mfma16(a0, b0, acc[0][0]);
-    acc[0][1] = mfma16(a0, b1, acc[0][1]);
-    acc[1][0] = mfma16(a1, b0, acc[1][0]);
-    acc[1][1] = mfma16(a1, b1, acc[1][1]);
+  T a[2][2], b[2][2];
+  auto read = [&](int kk, T (&av)[2], T (&bv)[2]) {
+    av[0] = As[(kk + lk) * pa + wr + lr];
+    av[1] = As[(kk + lk) * pa + wr + 16 + lr];
+    bv[0] = Bs[(kk + lk) * pb + wc + lr];
+    bv[1] = Bs[(kk + lk) * pb + wc + 16 + lr];
+  };
+  read(0, a[0], b[0]);
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) {
+    const int u = s & 1;
+    if (s + 1 < STEPS) read(4 * (s + 1), a[u ^ 1], b[u ^ 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    acc[0][0] = mfma16(a[u][0], b[u][0], acc[0][0]);
+    acc[0][1] = mfma16(a[u][0], b[u][1], acc[0][1]);
+    acc[1][0] = mfma16(a[u][1], b[u][0], acc[1][0]);
+    acc[1][1] = mfma16(a[u][1], b[u][1], acc[1][1]);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
