@@ -647,6 +647,8 @@ __global__ __launch_bounds__(NTHREADS) void k_syrk_outer(Prob* const* probs, Sch
   if (Tk <= 0 || bx >= Tk * (Tk + 1) / 2) return;
   int ti, tj;
   blocked_tile(bx, Tk, ti, tj);
+  ti = uniform(ti);  // (the square root's)
+  tj = uniform(tj);
   const int c1 = s_end * TILE;
   const FactorOut o{P.L, P.Np, P.dinv + (size_t)s_end * TILE * TILE,
                     P.logdiag ? P.logdiag + c1 : nullptr, P.diagval ? P.diagval + c1 : nullptr,
@@ -655,6 +657,252 @@ __global__ __launch_bounds__(NTHREADS) void k_syrk_outer(Prob* const* probs, Sch
   syrk_tile_multi<T, BF16, FUSE, BF16 != 0>(
       (T*)P.L, P.Np, s0, s_end, (int64_t)(s_end + ti) * TILE, (int64_t)(s_end + tj) * TILE,
       FUSE && ti == 0 && tj == 0, o, P.panel16, (int64_t)s_end * TILE, P.panel16_pitch);
+}
+
+// The outer update in tiles of 128 x 128, a wave 64 x 64 of it: half the
+// operand bytes per flop of the 64-tiles.  The operands come in chunks of KC
+// columns through two LDS buffers (one barrier per chunk), a chunk fetched
+// into registers during the product before its own.  The k order inside and
+// across the MFMA steps is the 64-tile's, so both give the same bits.  Bound
+// by the MFMAs (60 TFLOP/s FP64, 121 FP32 at the sizes below), BF16 by C's
+// bytes; per launch, 64- against 128-tiles: FP64, 184 block rows, K = 512:
+// 1570 -> 1188 us; FP32, 244, K = 768: 1946 -> 1569; BF16, 248, K = 512: 622
+// -> 323.  A third of FP32's gain is the addresses: tile indices from a square
+// root and descriptor fields arrive in vector registers, and 80 64-bit vector
+// additions per chunk then hold up the MFMAs (hence uniform()).
+template <typename T, int BF16>
+struct Outer128;
+template <>
+struct Outer128<double, 0> {
+  static constexpr int KC = 16, P = 144;  // k-major, rows of 128
+  typedef double LT;
+  static constexpr int OP = KC * P;  // elements of one operand chunk
+};
+template <>
+struct Outer128<float, 0> {
+  static constexpr int KC = 32, P = 36;  // m-major; 16-byte reads, 4 = P mod 32
+  typedef float LT;
+  static constexpr int OP = 128 * P;
+};
+template <>
+struct Outer128<float, 1> {
+  static constexpr int KC = 64, P = 72;  // m-major
+  typedef unsigned short LT;
+  static constexpr int OP = 128 * P;
+};
+
+template <typename T, int BF16>
+__global__ __launch_bounds__(NTHREADS, 2) void k_syrk_outer128(Prob* const* probs, Sched sc,
+                                                               int s0, int s_end) {
+  typedef Outer128<T, BF16> O;
+  typedef typename O::LT LT;
+  constexpr bool F64 = std::is_same<T, double>::value;
+  int bx;
+  const int g = xcd_contiguous(blockIdx.x, gridDim.x);
+  const Prob& P = *probs[sched_member(sc, g, bx)];
+  const int Tb = uniform(P.Np) / TILE - s_end, Tk = (Tb + 1) / 2;
+  if (Tk <= 0 || bx >= Tk * (Tk + 1) / 2) return;
+  int ti, tj;
+  blocked_tile(bx, Tk, ti, tj);
+  ti = uniform(ti);  // (the square root's)
+  tj = uniform(tj);
+  __shared__ __attribute__((aligned(16))) LT lds[4 * O::OP];
+  const int64_t ld = uniform(P.Np);
+  const int64_t ri = (int64_t)s_end * TILE + 128 * ti, rj = (int64_t)s_end * TILE + 128 * tj;
+  // an odd last block row: the upper 64 rows of its tile stand in for the
+  // missing ones, and the waves they belong to have nothing to do
+  const bool fulli = 2 * ti + 1 < Tb, fullj = 2 * tj + 1 < Tb;
+  const int t = threadIdx.x, l = t & 63, w = uniform(t >> 6);
+  const int wr = 64 * (w >> 1), wc = 64 * (w & 1);
+  const bool active = (wr == 0 || fulli) && (wc == 0 || fullj) && (ti != tj || wr >= wc);
+  const int lr = l & 15, lk = l >> 4;
+  typedef typename Acc<T>::type acc_t;
+  acc_t acc[4][4];  // [row block][column block]
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = (T)0;
+  const auto A = gbl(uniform((T*)P.L));
+  const int nc = (s_end - s0) * (TILE / O::KC);
+
+  // ---- a chunk of both operands: registers, LDS, MFMA steps ----
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  typedef typename std::conditional<
+      F64, d2, typename std::conditional<BF16 != 0, u16x8, floatx4>::type>::type chunk_t;
+  typedef typename std::conditional<F64, double, chunk_t>::type frag_t;
+  chunk_t ra[4], rb[4];
+  const int mt = F64 ? 2 * l : BF16 ? t >> 1 : t & 127;  // the thread's row of the tile
+  const unsigned ma = fulli ? mt : mt & 63, mb = fullj ? mt : mt & 63;
+  const auto p16 = gbl(uniform((const unsigned short*)P.panel16));
+  const unsigned pitch = uniform(P.panel16_pitch);
+  // Parts 0..3 of chunk c into registers, and from there into LDS buffer u.
+  auto fetch = [&](int c, int q) {
+    if constexpr (F64) {
+      typedef const __attribute__((address_space(1))) d2* gd2;
+      const auto p = A + ((int64_t)s0 * TILE + c * O::KC + w + 4 * q) * ld;
+      ra[q] = *(gd2)(p + ri + ma);
+      rb[q] = *(gd2)(p + rj + mb);
+    } else if constexpr (BF16 != 0) {
+      typedef const __attribute__((address_space(1))) u16x8* gu8;
+      const unsigned h = 32 * (t & 1) + 8 * q;
+      ra[q] = *(gu8)(p16 + (128 * ti * (int64_t)pitch + c * O::KC) + (ma * pitch + h));
+      rb[q] = *(gu8)(p16 + (128 * tj * (int64_t)pitch + c * O::KC) + (mb * pitch + h));
+    } else {
+      // LDS column e holds k = 16 (e / 8) + 8 (chunk & 1) + e % 8 of a block of
+      // 64: the k of eight of its sixteen MFMA steps (mma64_f32_mmajor's order)
+      auto p = A + ((int64_t)s0 * TILE + (c >> 1) * TILE + 32 * (w >> 1) + 8 * (c & 1) +
+                    16 * (q >> 1) + 4 * (q & 1)) * ld;
+#pragma unroll
+      for (int e = 0; e < 4; ++e, p += ld) {
+        ra[q][e] = (p + ri)[ma];
+        rb[q][e] = (p + rj)[mb];
+      }
+    }
+  };
+  auto stash = [&](int u, int q) {
+    LT* da = lds + 2 * u * O::OP;
+    LT* db = da + O::OP;
+    const int o = F64 ? (w + 4 * q) * O::P + 2 * l
+                      : mt * O::P + (BF16 ? 32 * (t & 1) + 8 * q : 16 * (w >> 1) + 4 * q);
+    *(chunk_t*)&da[o] = ra[q];
+    *(chunk_t*)&db[o] = rb[q];
+  };
+  // Operands of MFMA group s (F64: one step of four k; FP32: four steps; BF16:
+  // one of 32 k).
+  auto read = [&](const LT* da, int s, frag_t (&a)[4], frag_t (&b)[4]) {
+    const LT* db = da + O::OP;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int oa = F64 ? (4 * s + lk) * O::P + wr + 16 * i + lr
+                         : (wr + 16 * i + lr) * O::P + 8 * lk + (BF16 ? 32 : 4) * s;
+      const int ob = F64 ? (4 * s + lk) * O::P + wc + 16 * i + lr
+                         : (wc + 16 * i + lr) * O::P + 8 * lk + (BF16 ? 32 : 4) * s;
+      a[i] = *(const frag_t*)&da[oa];
+      b[i] = *(const frag_t*)&db[ob];
+    }
+  };
+  constexpr int NG = F64 ? 4 : 2;  // MFMA groups of a chunk
+  auto mfmas = [&](frag_t (&a)[4], frag_t (&b)[4], auto part) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < (F64 || BF16 ? 1 : 4); ++e) {
+      if constexpr (!F64 && !BF16) {
+        part(e);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          // (FP64 transposed: rows of D are the tile's columns, so that 16
+          // lanes hold consecutive rows of C, whole 128-byte lines)
+          if constexpr (F64)
+            acc[i][j] = mfma16(b[j], a[i], acc[i][j]);
+          else if constexpr (BF16 != 0)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, a[i]), __builtin_bit_cast(bf16x8, b[j]), acc[i][j], 0,
+                0, 0);
+          else
+            acc[i][j] = mfma16(a[i][e], b[j][e], acc[i][j]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // Chunk c is multiplied from one buffer while chunk c + 1 goes from the
+  // registers into the other and chunk c + 2 is fetched, a part at a time
+  // between the MFMA groups.
+  auto chunk = [&](int c, auto st, auto ft) {
+    __syncthreads();  // chunk c is in its buffer; the other one is read
+    const LT* da = lds + 2 * (c & 1) * O::OP;
+    auto part = [&](int q) {
+      if constexpr (st.value) stash((c & 1) ^ 1, q);
+      if constexpr (ft.value) fetch(c + 2, q);
+    };
+    if (active) {
+      frag_t a[2][4], b[2][4];
+      read(da, 0, a[0], b[0]);
+#pragma unroll
+      for (int s = 0; s < NG; ++s) {
+        if (s + 1 < NG) read(da, s + 1, a[(s & 1) ^ 1], b[(s & 1) ^ 1]);
+        if constexpr (F64) part(s);
+        if constexpr (BF16 != 0) {
+          part(2 * s);
+          part(2 * s + 1);
+        }
+        mfmas(a[s & 1], b[s & 1], [&](int e) {
+          if ((e & 1) == 0) part(2 * s + e / 2);
+        });
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) part(q);
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < 4; ++q) fetch(0, q);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) stash(0, q);
+  if (nc > 1)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) fetch(1, q);
+  int c = 0;
+  for (; c + 2 < nc; ++c) chunk(c, std::true_type{}, std::true_type{});
+  if (c + 1 < nc) chunk(c++, std::true_type{}, std::false_type{});
+  chunk(c, std::false_type{}, std::false_type{});
+  if (!active) return;
+  // ---- C -= acc ----
+  if constexpr (F64) {
+    const auto C = A + (ri + wr + (rj + wc) * ld);
+    const unsigned o = lr + lk * (unsigned)ld;
+    double v[2][16];
+    auto load = [&](int j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[j & 1][4 * i + r] = (C + (16 * i + (16 * j + 4 * r) * ld))[o];
+    };
+    load(0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j < 3) load(j + 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          (C + (16 * i + (16 * j + 4 * r) * ld))[o] = v[j & 1][4 * i + r] - acc[i][j][r];
+    }
+  } else {
+    typedef __attribute__((address_space(1))) floatx4* gf4;
+    const auto C = A + (ri + wr + (rj + wc) * ld);
+    const unsigned o = 4 * lk + lr * (unsigned)ld;
+    floatx4 v[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i][j] = *(gf4)(C + (16 * i + 16 * j * ld) + o);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *(gf4)(C + (16 * i + 16 * j * ld) + o) = v[i][j] - acc[i][j];
+  }
+}
+
+// Whether an outer update of t128 128-tiles takes them, or the 64-tiles.  Two
+// workgroups of 128-tiles fit a CU, and a CU given one more than its
+// neighbours keeps the launch waiting for a whole tile (K = 512 FP64: 73 us
+// for one, 133 for two), four times a 64-tile's.  Measured, 128- against
+// 64-tiles: FP64 (K = 512) 210 tiles 79 / 93 us, 300 132 / 121, 406 133 / 164,
+// 528 200 / 207, 1176 335 / 424; FP32 (K = 768) 210 64 / 69, 351 109 / 101,
+// 528 160 / 148, 741 163 / 196; 78 tiles (of 24 block rows) 74 / 50 FP64.
+// BF16 is bound by C's bytes and the operands', not by the tile's MFMAs: 210
+// 15 / 23, 300 24 / 29, 528 34 / 47.
+static bool outer_wide(long long t128, bool bf16) {
+  constexpr int CUS = 256;
+  if (bf16) return t128 >= 3 * CUS / 4;
+  return t128 >= 5 * CUS / 2 || (t128 >= 3 * CUS / 4 && t128 <= CUS);
 }
 
 // BF16 copy of the panel columns [s0, s_end) of the rows below the
@@ -1531,10 +1779,21 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
             hipLaunchKernelGGL(k_panel_bf16, dim3(n), dim3(NTHREADS), 0, s, dp, sc, s0, s_end);
           });
     }
-    sched_launch(b, outer_tiles, [&](Prob* const* dp, const Sched& sc, int n) {
+    auto outer_tiles128 = [&](int m) {
+      const int t = (std::max(0, b.np(m) / TILE - s_end) + 1) / 2;
+      return t * (t + 1) / 2;
+    };
+    long long t128 = 0;
+    for (int m = 0; m < b.count; ++m) t128 += outer_tiles128(m);
+    const bool wide = !fuse && outer_wide(t128, BF16 != 0);
+    auto tiles = [&](int m) { return wide ? outer_tiles128(m) : outer_tiles(m); };
+    sched_launch(b, tiles, [&](Prob* const* dp, const Sched& sc, int n) {
       if (tsy) timer_begin(TC_SYRK, s);
       if (fuse)
         hipLaunchKernelGGL((k_syrk_outer<T, BF16, 1>), dim3(n), dim3(NTHREADS), 0, s, dp, sc, s0,
+                           s_end);
+      else if (wide)
+        hipLaunchKernelGGL((k_syrk_outer128<T, BF16>), dim3(n), dim3(NTHREADS), 0, s, dp, sc, s0,
                            s_end);
       else
         hipLaunchKernelGGL((k_syrk_outer<T, BF16, 0>), dim3(n), dim3(NTHREADS), 0, s, dp, sc, s0,

@@ -82,3 +82,29 @@ def test_predict_at_column_tile_edges(N, M, mode, tol, vtol):
     m_ref, v_ref = O.predict(spec, X, Xt, w_ref, p_ref)
     assert rel_err(mean.cpu().numpy(), m_ref) < tol
     assert rel_err(var.cpu().numpy(), v_ref) < vtol
+
+
+# a batch whose outer updates together fill the chip takes the 128-tiles (odd
+# and even block counts below the first super-step), each member alone the
+# 64-tiles: the same bits
+@pytest.mark.parametrize("mode,count", [("fp64", 5), ("fp32", 8), ("bf16", 6)])
+def test_outer_update_tilings_agree(mode, count):
+    import torch
+
+    import probit_amd as P
+    from probit_amd.serving import ServingEngine
+    sizes = [1600 + 50 * (k % 2) - k for k in range(count)]
+    probs = [small_problem(200 + k, N, 2, "probit", "EQ", noise=0.5) for k, N in enumerate(sizes)]
+    eng = ServingEngine(precision=mode, capacity=8)
+    for tag, (X, y, theta, lp, _) in enumerate(probs):
+        assert eng.submit(tag, X, y, "EQ", theta[0], theta[1], "probit", lp[0], lp[1])
+    out = {}
+    while eng.in_flight:
+        for c in eng.step():
+            out[c.tag] = c
+    eng.close()
+    for tag, (X, y, theta, lp, _) in enumerate(probs):
+        gp = P.LaplaceGP(data=(X, y), prior=make_prior("EQ"), precision_mode=mode,
+                         log_likelihood=P.log_probit_likelihood)
+        w, p = gp.approximate_posterior((theta, lp))
+        assert torch.equal(w, out[tag].weight) and torch.equal(p, out[tag].precision), tag
