@@ -153,7 +153,7 @@ static void predict_launches(const Batch& b, int prec, int maxM, hipStream_t s) 
   launch_trsm(b, prec, maxMp, s);
   if (predict_refine(prec)) {
     launch_trsm_t(b, prec, maxMp, s);
-    launch_pred_refine(b, prec, maxM, s);
+    launch_pred_refine(b, maxM, s);
   }
   launch_predict_final(b, prec, maxM, s);
 }

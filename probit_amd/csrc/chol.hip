@@ -464,12 +464,13 @@ __device__ __forceinline__ int xcd_contiguous(int g, int total) {
 // the same values the stash would convert, so no conversion and half the
 // operand bytes.
 template <typename T, int BF16, int FUSE, bool SH = false>
-__device__ __forceinline__ void syrk_tile_multi(T* A_, int64_t ld, int kc0, int kc1, int64_t ri, int64_t rj,
+__device__ __forceinline__ void syrk_tile_multi(T* A_, int ld_, int kc0, int kc1, int ri_, int rj_,
                                 bool factor, const FactorOut& o,
                                 const unsigned short* p16 = nullptr, int64_t p16_row0 = 0,
                                 int p16_pitch = 0) {
   static_assert(!SH || BF16, "the panel copy holds BF16 operands");
-  auto A = gbl(A_);
+  const auto A = gbl(uniform(A_));
+  const int64_t ld = uniform(ld_), ri = uniform(ri_), rj = uniform(rj_);
   constexpr bool MM = MmajorF32<T, BF16>::value;
   constexpr int PITCH = BF16 ? 72 : MM ? 68 : KP<T>::value;
   typedef typename std::conditional<BF16 != 0, unsigned short, T>::type LT;
@@ -606,7 +607,7 @@ __global__ __launch_bounds__(NTHREADS) void k_col_update(Prob* const* probs, Sch
   const FactorOut o{P.L, P.Np, P.dinv + (size_t)j * TILE * TILE,
                     P.logdiag ? P.logdiag + c1 : nullptr, P.diagval ? P.diagval + c1 : nullptr,
                     P.info};
-  syrk_tile_multi<T, BF16, FUSE>((T*)P.L, P.Np, s0, j, (int64_t)i * TILE, (int64_t)j * TILE,
+  syrk_tile_multi<T, BF16, FUSE>((T*)P.L, P.Np, s0, j, i * TILE, j * TILE,
                                  FUSE && i == j, o);
 }
 
@@ -655,7 +656,7 @@ __global__ __launch_bounds__(NTHREADS) void k_syrk_outer(Prob* const* probs, Sch
                     P.info};
   // BF16 factors read the operands from the panel copy (k_panel_bf16)
   syrk_tile_multi<T, BF16, FUSE, BF16 != 0>(
-      (T*)P.L, P.Np, s0, s_end, (int64_t)(s_end + ti) * TILE, (int64_t)(s_end + tj) * TILE,
+      (T*)P.L, P.Np, s0, s_end, (s_end + ti) * TILE, (s_end + tj) * TILE,
       FUSE && ti == 0 && tj == 0, o, P.panel16, (int64_t)s_end * TILE, P.panel16_pitch);
 }
 

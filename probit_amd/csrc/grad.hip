@@ -65,17 +65,18 @@ __global__ __launch_bounds__(NTHREADS) void k_inv_diag(Prob* const* probs) {
 template <typename T, bool SECOND>
 __global__ __launch_bounds__(NTHREADS) void k_inv_merge(Prob* const* probs, int h) {
   const Prob& P = *probs[blockIdx.z];
-  const int nb = P.Np / TILE;
+  const int nb = uniform(P.Np) / TILE;
   const int a = 2 * h * blockIdx.y, mid = a + h;
   // the longest sums first: first product k from j, second k up to i
-  const int j = a + (int)blockIdx.x % h;
-  const int i = SECOND ? min(nb, mid + h) - 1 - (int)blockIdx.x / h : mid + (int)blockIdx.x / h;
+  const int j = uniform(a + (int)blockIdx.x % h);
+  const int i = uniform(SECOND ? min(nb, mid + h) - 1 - (int)blockIdx.x / h
+                               : mid + (int)blockIdx.x / h);
   if (i >= nb || i < mid) return;
-  const int64_t ld = P.Np;
+  const int64_t ld = uniform(P.Np);
   const unsigned m = threadIdx.x & 63;
   const int kb = uniform((int)(threadIdx.x >> 6));
-  const auto L = gbl((const T*)P.L);
-  const auto X = gbl((T*)P.S);
+  const auto L = gbl(uniform((const T*)P.L));
+  const auto X = gbl(uniform((T*)P.S));
   __shared__ GemmLds<T> lds;
   typename Acc<T>::type acc[2][2];
   zero_acc<T>(acc);
@@ -127,12 +128,14 @@ void launch_tri_inverse(const Batch& b, int prec, hipStream_t s) {
 template <typename T>
 __global__ __launch_bounds__(NTHREADS) void k_sym_from_inv(Prob* const* probs, int use_scale) {
   const Prob& P = *probs[blockIdx.y];
-  const int nb = P.Np / TILE;
+  const int nb = uniform(P.Np) / TILE;
   if ((int)blockIdx.x >= nb * (nb + 1) / 2) return;
   int ti, tj;
   lower_tile_g(blockIdx.x, ti, tj);
-  const int64_t ld = P.Np;
-  const auto X = gbl((const T*)P.S);
+  ti = uniform(ti);
+  tj = uniform(tj);
+  const int64_t ld = uniform(P.Np);
+  const auto X = gbl(uniform((const T*)P.S));
   __shared__ GemmLds<T> lds;
   typename Acc<T>::type acc[2][2];
   zero_acc<T>(acc);
@@ -146,7 +149,8 @@ __global__ __launch_bounds__(NTHREADS) void k_sym_from_inv(Prob* const* probs, i
   gemm_tiles<T, true>(
       ti, nb, [&](int k, T (&v)[16]) { rows(k, ti, v); },
       [&](int k, T (&v)[16]) { rows(k, tj, v); }, lds, acc);
-  const double* S = vslot(P, V_S);
+  const auto S = gbl(vslot(P, V_S));
+  const auto C = gbl(P.C);
 #pragma unroll
   for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
@@ -158,7 +162,7 @@ __global__ __launch_bounds__(NTHREADS) void k_sym_from_inv(Prob* const* probs, i
         double v = (double)acc[bm][bn][rr];
         if (use_scale) v *= S[i] * S[j];
         if (i >= P.N || j >= P.N) v = 0.0;
-        P.C[(size_t)i + (size_t)j * ld] = v;
+        C[(size_t)i + (size_t)j * ld] = v;
       }
 }
 

@@ -160,42 +160,52 @@ void launch_gram_self(const Batch& b, hipStream_t s) {
 // the symmetric product K x, x = vector slot rs, in the slots k_symv_reduce
 // adds (row sums of tile (I, J) in part[I][J], column sums in part[J][I];
 // see k_symv_tiles), so the Newton step's K r costs no second read of K.
+// Bound by memory: N = 16384 into FP32 500 -> 366 us (4.4 TB/s), every load of
+// K before the first store.
 template <typename T>
 __global__ __launch_bounds__(NTHREADS) void k_form_B(Prob* const* probs, Sched sc, int vb,
                                                      int rs) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
-  const int Tn = P.Np / TILE;
+  const int Tn = uniform(P.Np) / TILE;
   if (bx >= Tn * (Tn + 1) / 2) return;
   int ti, tj;
-  lower_tile(bx, ti, tj);
-  const int il = threadIdx.x & 63;
-  const int jg = threadIdx.x >> 6;
-  const int i = ti * TILE + il;
-  const int64_t ld = P.Np;
-  T* L = (T*)P.L;
-  const double* S = vslot(P, V_S);
+  lower_tile(Tn * (Tn + 1) / 2 - 1 - bx, tj, ti);  // down the columns
+  ti = uniform(Tn - 1 - ti);
+  tj = uniform(Tn - 1 - tj);
+  const unsigned il = threadIdx.x & 63;
+  const int jg = uniform((int)(threadIdx.x >> 6));
+  const int i = ti * TILE + il, j0 = tj * TILE + jg * 16;
+  const int64_t ld = uniform(P.Np);
+  const double* vec = uniform(P.vec);
+  const auto S = gbl(vec + V_S * ld);
+  const auto Sj = scalar(vec + V_S * ld) + j0;
+  const int64_t tile = ti * TILE + j0 * ld;
+  const auto Kt = gbl(uniform(P.K)) + tile;
+  const auto Lt = gbl(uniform((T*)P.L)) + tile;
   const double si = S[i];
-  const double s2 = P.noise_std * P.noise_std;
+  const double noise = P.noise_std;
+  const int N = P.N;
   double k[16];
-  for (int c = 0; c < 16; ++c) {
-    const int j = tj * TILE + jg * 16 + c;
-    const double kij = P.K[(size_t)i + (size_t)j * ld];
-    k[c] = kij;
-    double v;
-    if (vb == 1) {  // sigma^2 I + K
-      v = kij + ((i == j) ? ((i < P.N) ? s2 : 1.0) : 0.0);
-    } else {        // s I + S K S: s = 1 (B), or sigma (vb == 2, the VB adjoint's B_sigma)
-      v = si * kij * S[j] + ((i == j) ? ((vb == 2 && i < P.N) ? P.noise_std : 1.0) : 0.0);
-    }
-    L[(size_t)i + (size_t)j * ld] = (T)v;
+#pragma unroll
+  for (int c = 0; c < 16; ++c) k[c] = (Kt + c * ld)[il];
+  if (vb == 1) {  // sigma^2 I + K
+    const double d = i < N ? noise * noise : 1.0;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) (Lt + c * ld)[il] = (T)(k[c] + (i == j0 + c ? d : 0.0));
+  } else {  // s I + S K S: s = 1 (B), or sigma (vb == 2, the VB adjoint's B_sigma)
+    const double d = vb == 2 && i < N ? noise : 1.0;
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+      (Lt + c * ld)[il] = (T)(si * k[c] * Sj[c] + (i == j0 + c ? d : 0.0));
   }
   if (rs < 0) return;
   __shared__ double rpart[4][TILE];
-  const double* x = vslot(P, rs);
+  const auto x = gbl(vec + rs * ld);
+  const auto xj = scalar(vec + rs * ld) + j0;
   double rsum = 0.0;
 #pragma unroll
-  for (int c = 0; c < 16; ++c) rsum += k[c] * x[tj * TILE + jg * 16 + c];
+  for (int c = 0; c < 16; ++c) rsum += k[c] * xj[c];
   rpart[jg][il] = rsum;
   double* part = P.symv;
   if (ti != tj) {
@@ -326,22 +336,21 @@ __global__ __launch_bounds__(NTHREADS) void k_pred_cov(Prob* const* probs, Sched
                                                        int64_t ld) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
-  const int Mt = P.Mp / TILE;
+  const int Mt = uniform(P.Mp) / TILE;
   if (bx >= Mt * (Mt + 1) / 2) return;
   int ti, tj;
   lower_tile(bx, ti, tj);
+  ti = uniform(ti);
+  tj = uniform(tj);
   constexpr int PA = TILE + 1;
   __shared__ double sa[TILE * PA], sb[TILE * PA];
-  __shared__ double xs[TILE * PGP_MAX_DIM];
-  __shared__ double zs[TILE * PGP_MAX_DIM];
   __shared__ KShared ks;
+  static_assert(PGP_MAX_DIM <= PA, "input rows fit the operand buffers");
   const int D = P.D, M = P.M;
-  stage_params(ks, P.inv_ls2, P.pi_over_per);
-  load_rows(xs, P.Xt, ti * TILE, M, D);
-  load_rows(zs, P.Xt, tj * TILE, M, D);
-  const T* V = (const T*)P.S;
-  const size_t np = (size_t)P.Np;
-  const int kl = threadIdx.x & 63, cg = threadIdx.x >> 6;
+  const auto V = gbl(uniform((const T*)P.S));
+  const int64_t np = uniform(P.Np);
+  const unsigned kl = threadIdx.x & 63;
+  const int cg = uniform((int)(threadIdx.x >> 6));
   doublex4 acc[2][2];
   zero_acc<double>(acc);
   // k-major operands sa[k][m] = V(k0 + k, 64 ti + m), read coalesced along
@@ -351,12 +360,12 @@ __global__ __launch_bounds__(NTHREADS) void k_pred_cov(Prob* const* probs, Sched
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       const int c = cg + 4 * q;
-      ra[q] = V[(size_t)(k0 + kl) + (size_t)(ti * TILE + c) * np];
-      rb[q] = V[(size_t)(k0 + kl) + (size_t)(tj * TILE + c) * np];
+      ra[q] = (V + (k0 + (ti * TILE + c) * np))[kl];
+      rb[q] = (V + (k0 + (tj * TILE + c) * np))[kl];
     }
   };
   fetch(0);
-  for (int k0 = 0; k0 < P.Np; k0 += TILE) {
+  for (int k0 = 0; k0 < np; k0 += TILE) {
     __syncthreads();  // the previous chunk's products are done with LDS
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
@@ -365,9 +374,16 @@ __global__ __launch_bounds__(NTHREADS) void k_pred_cov(Prob* const* probs, Sched
       sb[kl * PA + c] = (double)rb[q];
     }
     __syncthreads();
-    if (k0 + TILE < P.Np) fetch(k0 + TILE);
+    if (k0 + TILE < np) fetch(k0 + TILE);
     mma64_kmajor<double>(sa, PA, sb, PA, acc);
   }
+  __syncthreads();  // operands are dead: the input rows take their place
+  double* xs = sa;
+  double* zs = sb;
+  stage_params(ks, P.inv_ls2, P.pi_over_per);
+  load_rows(xs, P.Xt, ti * TILE, M, D);
+  load_rows(zs, P.Xt, tj * TILE, M, D);
+  __syncthreads();
 #pragma unroll
   for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
@@ -412,14 +428,19 @@ void launch_pred_cov(const Batch& b, int prec, int maxMp, double* cov, int64_t l
 // of A, an FP64 MFMA product over those tiles of K (FP64), then per entry
 // z (2 s - z) - u A with s recomputed in FP64 from the inputs, summed over the
 // tile's 64 rows in a fixed order into qpart[I][j].  Z (the predict buffer
-// after both solves) holds z in the factor's storage type.
-template <typename T>
+// after both solves) holds z in FP32.  Tile rows with the longest sums first.
+//
+// Bound by the FP64 MFMAs and the fetches between them: N = 8192, M = 4096
+// 7.8 -> 5.2 ms (53 TFLOP/s) with the addresses from scalar registers, not 64-
+// bit vector additions, and the longest tiles not last.  Tiles of 128 x 128
+// with a wave 64 x 64: 4.7 there, but a batch of narrow predicts has too few
+// of them (256 test points: 176 -> 324 us a launch).
 __global__ __launch_bounds__(NTHREADS) void k_pred_refine(Prob* const* probs, Sched sc) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
-  const int nrt = P.Np / TILE, nct = P.Mp / TILE;
+  const int nrt = uniform(P.Np) / TILE, nct = uniform(P.Mp) / TILE;
   if (bx >= nrt * nct) return;
-  const int ti = bx % nrt, tj = bx / nrt;
+  const int ti = uniform(nrt - 1 - bx / nct), tj = uniform(bx % nct);
   constexpr int PA = TILE + 1;
   constexpr int KC = 32;  // k rows staged per step (half a tile: LDS and
                           // prefetch registers for more resident workgroups)
@@ -428,13 +449,15 @@ __global__ __launch_bounds__(NTHREADS) void k_pred_refine(Prob* const* probs, Sc
   __shared__ KShared ks;
   static_assert(TILE * PGP_MAX_DIM <= KC * PA, "input rows fit the operand buffers");
   const int D = P.D, M = P.M;
-  const size_t np = (size_t)P.Np;
-  const double* K = P.K;
-  const T* Z = (const T*)P.S;
-  const double* Ws = vslot(P, V_S);
+  const int64_t np = uniform(P.Np);
+  const auto K = gbl(uniform(P.K));
+  const auto Z = gbl(uniform((const float*)P.S));
+  const auto Ws = gbl(uniform(vslot(P, V_S)));
   const int t = threadIdx.x;
-  const int am = t & 63, ag = t >> 6;  // A: row m, k = ag + 4q
-  const int bk = t & 31, bg = t >> 5;  // B: row k, n = bg + 8q
+  const unsigned am = t & 63;  // A: row m, k = ag + 4q
+  const int ag = uniform(t >> 6);
+  const unsigned bk = t & 31, bg = t >> 5;  // B: row k, n = bg + 8q
+  const unsigned bo = bk + bg * (unsigned)np;
   doublex4 acc[2][2];
   zero_acc<double>(acc);
   // ra[q] = K(64 ti + am, k0 + ag + 4q); rb[q] = c U(k0 + bk, 64 tj + bg + 8q),
@@ -445,8 +468,8 @@ __global__ __launch_bounds__(NTHREADS) void k_pred_refine(Prob* const* probs, Sc
     const double w = (k0 < kend ? 2.0 : 1.0) * Ws[k0 + bk];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      ra[q] = K[(size_t)(ti * TILE + am) + (size_t)(k0 + ag + 4 * q) * np];
-      rb[q] = w * (double)Z[(size_t)(k0 + bk) + (size_t)(tj * TILE + bg + 8 * q) * np];
+      ra[q] = (K + (ti * TILE + (k0 + ag + 4 * q) * np))[am];
+      rb[q] = w * (double)(Z + (k0 + (tj * TILE + 8 * q) * np))[bo];
     }
   };
   fetch(0);
@@ -505,7 +528,7 @@ __global__ __launch_bounds__(NTHREADS) void k_pred_refine(Prob* const* probs, Sc
     P.qpart[(size_t)ti * P.Mp + tj * TILE + threadIdx.x] = red[0][threadIdx.x] + red[1][threadIdx.x];
 }
 
-void launch_pred_refine(const Batch& b, int prec, int maxM, hipStream_t s) {
+void launch_pred_refine(const Batch& b, int maxM, hipStream_t s) {
   const bool on = timer_on(TC_REFINE);
   sched_launch(
       b,
@@ -524,14 +547,11 @@ void launch_pred_refine(const Batch& b, int prec, int maxM, hipStream_t s) {
             const double np = b.np(m), mp = (b.mcount(m, maxM) + TILE - 1) / TILE * TILE;
             fl += np * (np + TILE) * mp;
             by += 0.5 * np * (np + TILE) * 8.0 * (mp / TILE) +
-                  2.0 * np * mp * (prec == PGP_PREC_FP64 ? 8 : 4);
+                  2.0 * np * mp * 4.0;
           }
           timer_begin(TC_REFINE, s);
         }
-        if (prec == PGP_PREC_FP64)
-          hipLaunchKernelGGL(k_pred_refine<double>, dim3(n), dim3(NTHREADS), 0, s, dp, sc);
-        else
-          hipLaunchKernelGGL(k_pred_refine<float>, dim3(n), dim3(NTHREADS), 0, s, dp, sc);
+        hipLaunchKernelGGL(k_pred_refine, dim3(n), dim3(NTHREADS), 0, s, dp, sc);
         if (on) timer_end(TC_REFINE, s, fl, by);
       });
 }

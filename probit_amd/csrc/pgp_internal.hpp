@@ -207,6 +207,13 @@ __device__ __forceinline__ T* uniform(T* p) {
   return (T*)(((uint64_t)hi << 32) | lo);
 }
 
+// A pointer whose loads may be scalar: for values written before the launch
+// and read at wave-uniform addresses.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T* scalar(const T* p) {
+  return (const __attribute__((address_space(4))) T*)(uintptr_t)p;
+}
+
 // Values handed between workgroups of one launch travel only through
 // relaxed agent-scope accesses: the stores write through the XCD's L2 and
 // the loads read past it, so a publication needs no L2 write-back or
@@ -304,7 +311,7 @@ void launch_gram_self(const Batch& b, hipStream_t s);
 // launch_symv_reduce)
 void launch_form_B(const Batch& b, int prec_vb, hipStream_t s, int rs = -1);
 void launch_cross_prep(const Batch& b, int prec, int maxM, hipStream_t s);
-void launch_pred_refine(const Batch& b, int prec, int maxM, hipStream_t s);
+void launch_pred_refine(const Batch& b, int maxM, hipStream_t s);
 int launch_gram_raw(const pgp_kernel_t* k, int dtype, const double* X, int64_t N,
                     const double* Z, int64_t M, void* out, int64_t ld, hipStream_t s);
 

@@ -533,7 +533,8 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged(Prob* const* probs, Sc
   const int rows = k == 0 ? 1 : nb - k;  // row blocks of this launch
   const int w = bx % rows, ct = bx / rows;
   if (ct >= P.Mp / TILE) return;
-  trsm_step<T>((const T*)P.L, P.Np, P.dinv, k, (T*)P.S, P.Np, w, ct);
+  trsm_step<T>(uniform((const T*)P.L), uniform(P.Np), uniform(P.dinv), k, uniform((T*)P.S),
+               uniform(P.Np), uniform(w), uniform(ct));
 }
 
 template <typename T>
@@ -557,9 +558,9 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged_raw(const T* L, int64_
 // block, over 256 CUs) exceeds the chain's step (the last product, DINV's and
 // the hand-off, ~9 us); FP64 at N = 3000, M = 5000: 2400 us as 12 super-step
 // launches, whose solving workgroups run 30 tile products in a row; 1712 in
-// one wavefront launch; 1235 (37 TFLOP/s) with the operands fetched a product
+// one wavefront launch; 1207 (38 TFLOP/s) with the operands fetched a product
 // ahead.  N = 1537, M = 501: 590 -> 269 us.  Transposed, FP32 at N = 8192, M =
-// 4096: 20.3 ms in 16 launches of 4 column tiles, 3.5 ms (79 TFLOP/s) in one.
+// 4096: 20.3 ms in 16 launches of 4 column tiles, 2.8 ms (98 TFLOP/s) in one.
 constexpr int WAVE_NCT = 4;
 
 template <typename T>
@@ -578,14 +579,14 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
     return;
   }
   int local;
-  const int i = sched_member(rows, tk, local);
-  const int m = local / nct, lct = local - m * nct, ct = ct0 + lct;
+  const int i = sched_member(rows, uniform(tk), local);
+  const int m = uniform(local / nct), lct = local - m * nct, ct = ct0 + lct;
   const Prob& P = *probs[m];
   if (ct >= P.Mp / TILE || i >= P.Np / TILE) return;
   uint64_t* prog = P.progress_ct + lct;
-  const auto L = gbl((const T*)P.L);
-  const auto S = gbl((T*)P.S);
-  const int64_t ld = P.Np;
+  const auto L = gbl(uniform((const T*)P.L));
+  const auto S = gbl(uniform((T*)P.S));
+  const int64_t ld = uniform(P.Np);
   const int64_t ri = (int64_t)i * TILE, n0 = (int64_t)ct * TILE;
   const unsigned r = threadIdx.x & 63;
   const int cb = uniform((int)(threadIdx.x >> 6));
@@ -599,7 +600,7 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
     for (int q = 0; q < 16; ++q, p += 4 * ld) la[q] = p[r];
   };
   auto fetch_d = [&]() {
-    const auto D = gbl(P.dinv + (size_t)i * TILE * TILE + (size_t)cb * TILE);
+    const auto D = gbl(uniform(P.dinv)) + ((size_t)i * TILE * TILE + (size_t)cb * TILE);
 #pragma unroll
     for (int q = 0; q < 16; ++q) la[q] = (T)D[r + (size_t)(4 * q) * TILE];
   };
@@ -708,16 +709,16 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
     return;
   }
   int local;
-  const int t = sched_member(rows, tk, local);
-  const int m = local / nct, lct = local - m * nct;
+  const int t = sched_member(rows, uniform(tk), local);
+  const int m = uniform(local / nct), lct = local - m * nct;
   const Prob& P = *probs[m];
-  const int nb = P.Np / TILE, ct = ct0 + lct;
+  const int nb = uniform(P.Np) / TILE, ct = ct0 + lct;
   if (ct >= P.Mp / TILE || t >= nb) return;
   const int i = nb - 1 - t;
   uint64_t* prog = P.progress_ct + lct;
-  const auto L = gbl((const T*)P.L);
-  const auto S = gbl((T*)P.S);
-  const int64_t ld = P.Np;
+  const auto L = gbl(uniform((const T*)P.L));
+  const auto S = gbl(uniform((T*)P.S));
+  const int64_t ld = uniform(P.Np);
   const int64_t ri = (int64_t)i * TILE, n0 = (int64_t)ct * TILE;
   const unsigned r = threadIdx.x & 63;
   const int cb = uniform((int)(threadIdx.x >> 6));
@@ -732,7 +733,7 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
     for (int q = 0; q < 16; ++q, p += 4 * ld) la[q] = p[r];
   };
   auto fetch_d = [&]() {
-    const auto D = gbl(P.dinv + (size_t)i * TILE * TILE + (size_t)cb * TILE);
+    const auto D = gbl(uniform(P.dinv)) + ((size_t)i * TILE * TILE + (size_t)cb * TILE);
 #pragma unroll
     for (int q = 0; q < 16; ++q) la[q] = (T)D[r + (size_t)(4 * q) * TILE];
   };
@@ -888,17 +889,22 @@ __device__ __forceinline__ void trsm_acc(const T* L, int64_t ld, const T* S, int
   constexpr int PP = KP<T>::value;  // A operand: conflict-free MFMA reads
   constexpr int PB = TILE + 1;       // B operand: written transposed, conflict-free stores
   if (c0 >= c1) return;
-  const int m = threadIdx.x & 63, kb = threadIdx.x >> 6;
+  const unsigned m = threadIdx.x & 63;
+  const int kb = uniform((int)(threadIdx.x >> 6));
   T ra[16], rb[16];
   auto fetch = [&](int c) {
     const int64_t cc = (int64_t)c * TILE;
-    const bool fresh = c >= c_fresh;
+    auto pa = gbl(L) + (r0 + (cc + kb) * ld);  // A(m, k)
+    auto pb = gbl(S) + (cc + (n0 + kb) * lds);  // B(m, k): row m, column k
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int k = kb + 4 * q;
-      ra[q] = L[(size_t)(r0 + m) + (size_t)(cc + k) * ld];  // A(m, k)
-      const T* sp = &S[(size_t)(cc + m) + (size_t)(n0 + k) * lds];  // B(m, k): row m, column k
-      rb[q] = fresh ? __hip_atomic_load(sp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *sp;
+    for (int q = 0; q < 16; ++q, pa += 4 * ld) ra[q] = pa[m];
+    if (c >= c_fresh) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q, pb += 4 * lds)
+        rb[q] = __hip_atomic_load(pb + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 16; ++q, pb += 4 * lds) rb[q] = pb[m];
     }
   };
   fetch(c0);
@@ -928,6 +934,7 @@ __device__ __forceinline__ void trsm_ss(const T* L, int64_t ld, const double* di
   __shared__ T Bs[TILE * PB];
   typedef typename Acc<T>::type acc_t;
   constexpr int G = TRSM_G;
+  u = uniform(u);
   const int p0 = q > 0 ? G * (q - 1) : 0;  // first column of P (or of SS_0)
   acc_t acc[2][2];
   if (u < nct) {
@@ -968,8 +975,8 @@ __device__ __forceinline__ void trsm_ss(const T* L, int64_t ld, const double* di
   }
   // update of row block i >= G(q+1) by P = [G(q-1), Gq)
   const int v = u - nct;
-  const int ct = v % nct;
-  const int i = G * (q + 1) + v / nct;
+  const int ct = uniform(v % nct);
+  const int i = uniform(G * (q + 1) + v / nct);
   if (q == 0 || i >= nb) return;
   const int64_t r0 = (int64_t)i * TILE, n0 = (int64_t)ct * TILE;
   zero_acc<T>(acc);
@@ -995,7 +1002,9 @@ template <typename T>
 __global__ __launch_bounds__(NTHREADS) void k_trsm(Prob* const* probs, Sched sc, int q) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
-  trsm_ss<T>((const T*)P.L, P.Np, P.dinv, P.Np / TILE, q, (T*)P.S, P.Np, P.Mp / TILE, bx);
+  const int np = uniform(P.Np);
+  trsm_ss<T>(uniform((const T*)P.L), np, uniform(P.dinv), np / TILE, q, uniform((T*)P.S), np,
+             uniform(P.Mp) / TILE, bx);
 }
 
 static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, hipStream_t s) {
@@ -1035,6 +1044,8 @@ static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, hipStream_t
   }
 }
 
+// FP32, N = 8192, M = 4096: 196 -> 117 us a launch with the addresses from
+// scalar registers (376 vector registers held one workgroup a CU; 152 hold 3).
 // Right-hand sides of at least this many column tiles take the super-step
 // schedule.
 constexpr int TRSM_WIDE = 16;

@@ -77,26 +77,31 @@ template <int MAT>
 __global__ __launch_bounds__(NTHREADS) void k_symv_tiles(Prob* const* probs, Sched sc, int xs) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
-  const int nb = P.Np / TILE;
+  const int nb = uniform(P.Np) / TILE;
   if (bx >= nb * (nb + 1) / 2) return;
   int ti, tj;
   lower_tile_v(bx, ti, tj);
+  ti = uniform(ti);
+  tj = uniform(tj);
   __shared__ double rpart[4][TILE];
-  const size_t ld = (size_t)P.Np;
-  const int r = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const double* x = vslot(P, xs);
-  const size_t tile = (size_t)ti * TILE + (size_t)tj * TILE * ld;
-  const double* Kt = (MAT == SYMV_C ? P.C : P.K) + tile;
+  const int64_t ld = uniform(P.Np);
+  const unsigned r = threadIdx.x & 63;
+  const int w = uniform((int)(threadIdx.x >> 6));
+  const double* xp = uniform(P.vec) + xs * ld;
+  const auto x = gbl(xp);
+  const auto xj = scalar(xp) + (tj * TILE + w);
+  const int64_t tile = ti * TILE + (tj * TILE + w) * ld;
+  const auto Kt = gbl(uniform(MAT == SYMV_C ? P.C : P.K)) + tile;
   // lane r holds row r of the wave's 16 columns c = w + 4q (coalesced down
   // each column); the tile never goes through LDS
   double k[16];
 #pragma unroll
-  for (int q = 0; q < 16; ++q) k[q] = Kt[(size_t)r + (size_t)(w + 4 * q) * ld];
+  for (int q = 0; q < 16; ++q) k[q] = (Kt + 4 * q * ld)[r];
   if constexpr (MAT == SYMV_HADAMARD) {
-    const double* Ct = P.C + tile;
+    const auto Ct = gbl(uniform(P.C)) + tile;
     double c[16];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) c[q] = Ct[(size_t)r + (size_t)(w + 4 * q) * ld];
+    for (int q = 0; q < 16; ++q) c[q] = (Ct + 4 * q * ld)[r];
 #pragma unroll
     for (int q = 0; q < 16; ++q) k[q] *= c[q];
   }
@@ -104,9 +109,9 @@ __global__ __launch_bounds__(NTHREADS) void k_symv_tiles(Prob* const* probs, Sch
   double rs = 0.0;
 #pragma unroll
   for (int q = 0; q < 16; ++q)
-    rs += MAT == SYMV_HADAMARD ? k[q] : k[q] * x[tj * TILE + w + 4 * q];
+    rs += MAT == SYMV_HADAMARD ? k[q] : k[q] * xj[4 * q];
   rpart[w][r] = rs;
-  double* part = P.symv;
+  const auto part = gbl(uniform(P.symv));
   if (ti != tj) {
     // column sums K_IJ^T x_I of the wave's 16 columns: a transposing
     // butterfly halves the values per lane at each of lane bits 5..2, then
