@@ -635,19 +635,38 @@ __device__ __forceinline__ void blocked_tile(int t, int Tk, int& ti, int& tj) {
   }
 }
 
+// Tile t of the first w tile columns of a lower triangle: its top w x w
+// triangle, then whole rows.
+__device__ __forceinline__ void column_tile(int t, int w, int& ti, int& tj) {
+  const int v = t - w * (w + 1) / 2;
+  if (v < 0) {
+    lower_tile_c(t, ti, tj);
+  } else {
+    ti = w + v / w;
+    tj = v % w;
+  }
+}
+
 // Outer update closing a super-step [s0, s_end): every lower tile (i, j),
-// s_end <= j <= i, gets A_ij -= sum_{c in [s0, s_end)} L_ic L_jc^T.
+// s_end <= j <= i, j < s_end + wd, gets A_ij -= sum_{c in [s0, s_end)} L_ic
+// L_jc^T.
+__host__ __device__ __forceinline__ int outer_tiles64(int Tk, int wd) {
+  const int w = wd < Tk ? wd : Tk;
+  return w * Tk - w * (w - 1) / 2;
+}
 template <typename T, int BF16, int FUSE>
 __global__ __launch_bounds__(NTHREADS) void k_syrk_outer(Prob* const* probs, Sched sc, int s0,
-                                                         int s_end) {
+                                                         int s_end, int wd) {
   int bx;
   const int g = xcd_contiguous(blockIdx.x, gridDim.x);
   const Prob& P = *probs[sched_member(sc, g, bx)];
-  const int nb = P.Np / TILE;
-  const int Tk = nb - s_end;
-  if (Tk <= 0 || bx >= Tk * (Tk + 1) / 2) return;
+  const int Tk = uniform(P.Np) / TILE - s_end;
+  if (Tk <= 0 || bx >= outer_tiles64(Tk, wd)) return;
   int ti, tj;
-  blocked_tile(bx, Tk, ti, tj);
+  if (wd >= Tk)
+    blocked_tile(bx, Tk, ti, tj);
+  else
+    column_tile(bx, wd, ti, tj);
   ti = uniform(ti);  // (the square root's)
   tj = uniform(tj);
   const int c1 = s_end * TILE;
@@ -692,24 +711,32 @@ struct Outer128<float, 1> {
   static constexpr int OP = 128 * P;
 };
 
+// 128-tiles of a lower triangle of tb block rows
+__host__ __device__ __forceinline__ int tiles128(int tb) {
+  const int t = (tb + 1) / 2;
+  return tb > 0 ? t * (t + 1) / 2 : 0;
+}
+
+// Tile bx (blocked_tile's order) of the lower triangle from block row and
+// column `base` on, or (wd > 0) bx of its first wd block columns (even):
+// A -= the product of the panel columns [s0, s1), s1 <= base.  lds: 4 OP
+// elements.  All threads call it.
 template <typename T, int BF16>
-__global__ __launch_bounds__(NTHREADS, 2) void k_syrk_outer128(Prob* const* probs, Sched sc,
-                                                               int s0, int s_end) {
+__device__ __forceinline__ void outer128_tile(const Prob& P, int bx, int s0, int s1, int base,
+                                              int wd, typename Outer128<T, BF16>::LT* lds) {
   typedef Outer128<T, BF16> O;
   typedef typename O::LT LT;
   constexpr bool F64 = std::is_same<T, double>::value;
-  int bx;
-  const int g = xcd_contiguous(blockIdx.x, gridDim.x);
-  const Prob& P = *probs[sched_member(sc, g, bx)];
-  const int Tb = uniform(P.Np) / TILE - s_end, Tk = (Tb + 1) / 2;
-  if (Tk <= 0 || bx >= Tk * (Tk + 1) / 2) return;
+  const int Tb = uniform(P.Np) / TILE - base, Tk = (Tb + 1) / 2;
   int ti, tj;
-  blocked_tile(bx, Tk, ti, tj);
+  if (wd == 0)
+    blocked_tile(bx, Tk, ti, tj);
+  else
+    column_tile(bx, wd / 2, ti, tj);
   ti = uniform(ti);  // (the square root's)
   tj = uniform(tj);
-  __shared__ __attribute__((aligned(16))) LT lds[4 * O::OP];
   const int64_t ld = uniform(P.Np);
-  const int64_t ri = (int64_t)s_end * TILE + 128 * ti, rj = (int64_t)s_end * TILE + 128 * tj;
+  const int64_t ri = (int64_t)base * TILE + 128 * ti, rj = (int64_t)base * TILE + 128 * tj;
   // an odd last block row: the upper 64 rows of its tile stand in for the
   // missing ones, and the waves they belong to have nothing to do
   const bool fulli = 2 * ti + 1 < Tb, fullj = 2 * tj + 1 < Tb;
@@ -726,7 +753,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_syrk_outer128(Prob* const* prob
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = (T)0;
   const auto A = gbl(uniform((T*)P.L));
-  const int nc = (s_end - s0) * (TILE / O::KC);
+  const int nc = (s1 - s0) * (TILE / O::KC);
 
   // ---- a chunk of both operands: registers, LDS, MFMA steps ----
   typedef double d2 __attribute__((ext_vector_type(2)));
@@ -736,8 +763,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_syrk_outer128(Prob* const* prob
   chunk_t ra[4], rb[4];
   const int mt = F64 ? 2 * l : BF16 ? t >> 1 : t & 127;  // the thread's row of the tile
   const unsigned ma = fulli ? mt : mt & 63, mb = fullj ? mt : mt & 63;
-  const auto p16 = gbl(uniform((const unsigned short*)P.panel16));
-  const unsigned pitch = uniform(P.panel16_pitch);
+  const unsigned pitch = uniform(P.panel16_pitch);  // (BF16: row s1 TILE is the first)
+  const auto p16 = gbl(uniform((const unsigned short*)P.panel16)) +
+                   (int64_t)(base - s1) * TILE * pitch;
   // Parts 0..3 of chunk c into registers, and from there into LDS buffer u.
   auto fetch = [&](int c, int q) {
     if constexpr (F64) {
@@ -889,6 +917,34 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_syrk_outer128(Prob* const* prob
 #pragma unroll
       for (int i = 0; i < 4; ++i) *(gf4)(C + (16 * i + 16 * j * ld) + o) = v[i][j] - acc[i][j];
   }
+}
+
+// The outer update closing a super-step [s0, s_end) (as k_syrk_outer), or
+// (wd > 0) its first wd block columns and, of the triangle right of them, all
+// but the last `rest` tiles.
+__host__ __device__ __forceinline__ int outer_tiles128(int tb, int wd, int rest) {
+  if (wd == 0) return tiles128(tb);
+  const int a = tiles128(tb), t = tiles128(tb - wd);
+  return a - t + (t > rest ? t - rest : 0);
+}
+template <typename T, int BF16>
+__global__ __launch_bounds__(NTHREADS, 2) void k_syrk_outer128(Prob* const* probs, Sched sc,
+                                                               int s0, int s_end, int wd) {
+  __shared__ __attribute__((aligned(16))) typename Outer128<T, BF16>::LT
+      lds[4 * Outer128<T, BF16>::OP];
+  int bx;
+  const int g = xcd_contiguous(blockIdx.x, gridDim.x);
+  const Prob& P = *probs[sched_member(sc, g, bx)];
+  int base = s_end;
+  if (wd > 0) {
+    const int tb = uniform(P.Np) / TILE - s_end, n = tiles128(tb) - tiles128(tb - wd);
+    if (bx >= n) {
+      bx -= n;
+      base += wd;
+      wd = 0;
+    }
+  }
+  outer128_tile<T, BF16>(P, bx, s0, s_end, base, wd, lds);
 }
 
 // Whether an outer update of t128 128-tiles takes them, or the 64-tiles.  Two
@@ -1140,12 +1196,27 @@ constexpr int MAXG = 16;
 // Tickets: the row blocks s0, s0 + 1, ... of the super-step, each for every
 // member that has it, then the rows below, member after member; a workgroup
 // waits only for row blocks of its member above its own, on lower tickets.
+//
+// Outer tiles: with the previous super-step's outer update done only for this
+// one's columns, the rest of it (128-tiles from column s1 on) goes into this
+// launch, where it fills the CUs that the column chain leaves idle.
+// A factor of N = 4096 in FP64: super-steps of 100 us and outer updates of 82
+// on average; with the tiles 124 to 101, and 39 to 24 for the columns before.
+// Evidence and gradient 18.6 -> 16.4 ms; prior draw N = 12288 14.4 -> 13.7;
+// FP32 posterior N = 8192 38.4 -> 35.1 (with tiles handed out by ticket, not
+// in runs per XCD, only 37.6: a tile then took 80 us, not 60).
+constexpr int LOOKB = 64;  // members of a launch with outer tiles
 struct StepSched {
   int32_t count;             // members (sorted by size, descending)
   int32_t s0, s1;            // columns [s0, s1)
   int32_t rlim;              // row blocks [s0, min(nb, rlim))
-  int32_t gbase[MAXG + 1];   // first ticket of row block s0 + g; [s1 - s0]: of the rows below
+  int32_t gbase[MAXG + 1];   // first ticket of row block s0 + g; [s1 - s0]: the end
   int32_t pre[MAXB + 1];     // rows below (i >= s1) of the members before m
+  // the previous super-step's outer update from block column s1 on
+  int32_t p0;                // its columns [p0, s0)
+  int32_t ofirst;            // outer tiles before the rows below
+  int32_t rest;              // at most so many of each member, its last ones
+  int32_t opre[LOOKB + 1];   // outer tiles of the members before m (opre[count] = 0: none)
 };
 
 __device__ __forceinline__ uint32_t* tile_flag(uint32_t* csync, int s0, int i, int c) {
@@ -1207,7 +1278,9 @@ struct StepArena {
   static constexpr int OPER = TILE * (BF16 ? 72 : MmajorF32<T, BF16>::value ? 68 : KP<T>::value);
   static constexpr int all = 2 * TILE * KP<T>::value * (int)sizeof(T) +
                              2 * OPER * (BF16 ? 2 : (int)sizeof(T));
-  static constexpr int bytes = all > FACTOR_LDS ? all : FACTOR_LDS;
+  static constexpr int outer = 4 * Outer128<T, BF16>::OP * (BF16 ? 2 : (int)sizeof(T));
+  static constexpr int step = all > FACTOR_LDS ? all : FACTOR_LDS;
+  static constexpr int bytes = step > outer ? step : outer;
 };
 
 template <typename T, int BF16>
@@ -1215,31 +1288,43 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
                                                         uint32_t* ticket, uint32_t epoch) {
   __shared__ __attribute__((aligned(16))) char arena[StepArena<T, BF16>::bytes];
   __shared__ int s_val;
-  const int t = take_ticket(ticket, &s_val);
-  if ((unsigned)t >= gridDim.x) {  // counter not zero at launch: nothing to take
+  // the outer tiles wait for nothing: no ticket, and a run of tiles per XCD
+  const int s0 = ss.s0, s1 = ss.s1;
+  const int chain = ss.gbase[s1 - s0], rows = chain + ss.pre[ss.count];
+  const int u = (int)blockIdx.x - chain;
+  if (u >= 0 && (u < ss.ofirst || u >= ss.ofirst + rows - chain)) {
+    int o = xcd_contiguous(u < ss.ofirst ? u : u - (rows - chain), gridDim.x - rows);
+    int mo = 0;
+    while (o >= ss.opre[mo + 1]) ++mo;
+    const Prob& P = *uniform(probs[mo]);
+    o += max(0, tiles128(uniform(P.Np) / TILE - s1) - ss.rest) - ss.opre[mo];
+    outer128_tile<T, BF16>(P, o, ss.p0, s0, s1, 0, (typename Outer128<T, BF16>::LT*)arena);
+    return;
+  }
+  const int t = take_ticket(ticket, &s_val, rows);
+  if ((unsigned)t >= (unsigned)rows) {  // counter not zero at launch: nothing to take
     flag_members_stalled(probs, ss.count);
     return;
   }
   // ticket -> (member mi, row block i)
-  const int s0 = ss.s0, s1 = ss.s1;
   int mi, i;
-  if (t < ss.gbase[s1 - s0]) {
+  if (t < chain) {
     int g = 0;
     while (t >= ss.gbase[g + 1]) ++g;
     mi = t - ss.gbase[g];
     i = s0 + g;
   } else {
-    const int u = t - ss.gbase[s1 - s0];
+    const int b = t - chain;
     int lo = 0, hi = ss.count;
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
-      if (ss.pre[mid] <= u)
+      if (ss.pre[mid] <= b)
         lo = mid;
       else
         hi = mid;
     }
     mi = lo;
-    i = s1 + u - ss.pre[lo];
+    i = s1 + b - ss.pre[lo];
   }
   const Prob& P = *uniform(probs[mi]);
   const int nb = uniform(P.Np) / TILE;
@@ -1548,11 +1633,16 @@ struct TuneTable {
   std::mutex mu;
   pgp_tune_entry_t e[3][TUNE_CLASSES];
   TuneTable() {
-    const int G = std::min(16, std::max(1, env_int("PGP_SUPERSTEP", 8)));
     const int cm = env_int("PGP_COLUMN_MAX", 512), fm = env_int("PGP_FUSE_MAX", 512);
     const int mg = std::min(2, std::max(0, env_int("PGP_COLUMN_MERGE", 2)));
     for (int p = 0; p < 3; ++p)
-      for (int c = 0; c < TUNE_CLASSES; ++c) e[p][c] = pgp_tune_entry_t{G, cm, fm, mg};
+      for (int c = 0; c < TUNE_CLASSES; ++c) {
+        // FP64 above the size class: the shorter column chain of six (N = 1537
+        // 6.56 -> 6.07 ms a posterior, N = 4096 19.7 -> 18.6 the evidence and
+        // gradient, N = 12288 14.55 -> 14.66 a prior draw)
+        const int g = env_int("PGP_SUPERSTEP", p == PGP_PREC_FP64 && c == 1 ? 6 : 8);
+        e[p][c] = pgp_tune_entry_t{std::min(16, std::max(1, g)), cm, fm, mg};
+      }
   }
 };
 static TuneTable& tune_table() {
@@ -1682,8 +1772,27 @@ static void rows_launch(const Batch& b, int s0, int s1, bool tpa, hipStream_t s)
       });
 }
 
+// Outer tiles that a super-step's launch takes along, one workgroup a CU, in
+// the CUs that its `chain` workgroups on the column chain and its `rows` rows
+// below leave idle, and how many of them go before the rows (first).  The
+// chain lasts `all` tiles' times (in tenths; FP64 100 us for 6 columns, 60 a
+// tile of K = 384; FP32 175 for 12, 65 of K = 768; BF16 100 for 8, 13 of K =
+// 512; both grow with G).  A row below takes about as long as the chain if it
+// starts with it, waiting most of the time, and less once the chain has got
+// ahead: few rows start with it, many after the first rounds of tiles.  Many
+// FP32 rows, two a CU without outer tiles, take none (N = 16384, 244 rows: 334
+// us with 240 tiles, 194 without and 51 for the tiles).
 template <typename T, int BF16>
-static void superstep_launch(const Batch& b, int s0, int s1, int rlim, bool tpa, hipStream_t s) {
+static int look_tiles(int chain, int rows, int& first) {
+  constexpr int all = sizeof(T) == 8 ? 20 : BF16 ? 80 : 28;
+  constexpr int head = BF16 ? 30 : 10;
+  if (sizeof(T) == 4 && !BF16 && rows > 160) return first = 0;
+  first = rows <= 96 ? 0 : std::max(0, head * (256 - chain) / 10);
+  return first + (all - (first > 0 ? head : 0)) * (256 - chain - rows) / 10;
+}
+template <typename T, int BF16>
+static void superstep_launch(const Batch& b, int s0, int s1, int rlim, int p0, int rest, bool tpa,
+                             hipStream_t s) {
   constexpr double F3 = TILE * TILE * TILE / 3.0;
   constexpr double G64 = 2.0 * TILE * TILE * TILE;
   for (int off = 0; off < b.count; off += MAXB) {
@@ -1709,7 +1818,24 @@ static void superstep_launch(const Batch& b, int s0, int s1, int rlim, bool tpa,
         if (b.np(off + m) / TILE > s0 + g) ++nd;
       ss.gbase[g + 1] = ss.gbase[g] + nd;
     }
-    const int tot = ss.gbase[ncols] + ss.pre[n];
+    ss.p0 = p0;
+    ss.rest = rest;
+    ss.opre[0] = 0;
+    if (p0 >= 0) {
+      for (int m = 0; m < n; ++m) {
+        const int t = std::min(rest, tiles128(b.np(off + m) / TILE - s1));
+        ss.opre[m + 1] = ss.opre[m] + t;
+        fl += 4.0 * t * G64 * (s0 - p0);
+      }
+    } else {
+      ss.opre[std::min(n, LOOKB)] = 0;
+    }
+    const int nouter = ss.opre[std::min(n, LOOKB)];
+    look_tiles<T, BF16>(ss.gbase[ncols], ss.pre[n], ss.ofirst);
+    ss.ofirst = std::min(ss.ofirst, nouter);
+    // with outer tiles one workgroup a CU: a second one would slow the chain's
+    const int lds = nouter > 0 && sizeof(T) == 4 ? 8192 : 0;
+    const int tot = ss.gbase[ncols] + ss.pre[n] + nouter;
     if (tot == 0) continue;
     const uint32_t ep = next_epoch();
     const bool tsu = timer_on(TC_SUPER);
@@ -1722,11 +1848,14 @@ static void superstep_launch(const Batch& b, int s0, int s1, int rlim, bool tpa,
         const int nbm = b.np(off + m) / TILE, nbr = std::min(nbm, rlim);
         for (int j = s0; j < std::min(s1, nbm); ++j)
           by += (double)(nbr - j) * 2.0 * TB * sizeof(T) + TB * 8.0;
+        if (p0 >= 0)
+          by += std::min(rest, tiles128(nbm - s1)) * 8.0 * TB * sizeof(T) +
+                std::max(0, nbm - s1) * TB * (s0 - p0) * (BF16 ? 2.0 : sizeof(T));
       }
       timer_begin(TC_SUPER, s);
     }
-    hipLaunchKernelGGL((k_superstep<T, BF16>), dim3(tot), dim3(NTHREADS), 0, s, b.dprobs + off, ss,
-                       b.ticket, ep);
+    hipLaunchKernelGGL((k_superstep<T, BF16>), dim3(tot), dim3(NTHREADS), lds, s, b.dprobs + off,
+                       ss, b.ticket, ep);
     if (tsu) timer_end(TC_SUPER, s, fl, by);
   }
 }
@@ -1766,11 +1895,9 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
     for (int m = 0; m < b.count; ++m) w += std::max(0, b.np(m) / TILE - s0);
     return w <= column_max;
   };
-  auto outer_launch = [&](int s0, int s_end, bool fuse) {
-    auto outer_tiles = [&](int m) {
-      const int t = std::max(0, b.np(m) / TILE - s_end);
-      return t * (t + 1) / 2;
-    };
+  // rest >= 0: all but the last `rest` 128-tiles of each member's triangle from
+  // the next super-step's end on, which go into that super-step's launch
+  auto outer_launch = [&](int s0, int s_end, bool fuse, int rest) {
     if constexpr (BF16 != 0) {
       // the BF16 copy of the panel rows below the super-step, which the
       // outer update reads instead of converting at every stash
@@ -1780,39 +1907,50 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
             hipLaunchKernelGGL(k_panel_bf16, dim3(n), dim3(NTHREADS), 0, s, dp, sc, s0, s_end);
           });
     }
-    auto outer_tiles128 = [&](int m) {
-      const int t = (std::max(0, b.np(m) / TILE - s_end) + 1) / 2;
-      return t * (t + 1) / 2;
+    const int wd = rest < 0 ? 0 : G;  // its columns, if it has to be split
+    auto tiles128_of = [&](int m) { return outer_tiles128(b.np(m) / TILE - s_end, wd, rest); };
+    auto tiles64_of = [&](int m) {
+      return outer_tiles64(std::max(0, b.np(m) / TILE - s_end), wd > 0 ? wd : nb);
     };
     long long t128 = 0;
-    for (int m = 0; m < b.count; ++m) t128 += outer_tiles128(m);
-    const bool wide = !fuse && outer_wide(t128, BF16 != 0);
-    auto tiles = [&](int m) { return wide ? outer_tiles128(m) : outer_tiles(m); };
+    bool more = false;  // than the columns
+    for (int m = 0; m < b.count; ++m) {
+      t128 += tiles128_of(m);
+      more |= wd > 0 && tiles128(b.np(m) / TILE - s_end - wd) > rest;
+    }
+    const bool wide = more || (!fuse && wd % 2 == 0 && outer_wide(t128, BF16 != 0));
+    auto tiles = [&](int m) { return wide ? tiles128_of(m) : tiles64_of(m); };
     sched_launch(b, tiles, [&](Prob* const* dp, const Sched& sc, int n) {
       if (tsy) timer_begin(TC_SYRK, s);
       if (fuse)
         hipLaunchKernelGGL((k_syrk_outer<T, BF16, 1>), dim3(n), dim3(NTHREADS), 0, s, dp, sc, s0,
-                           s_end);
+                           s_end, nb);
       else if (wide)
         hipLaunchKernelGGL((k_syrk_outer128<T, BF16>), dim3(n), dim3(NTHREADS), 0, s, dp, sc, s0,
-                           s_end);
+                           s_end, wd);
       else
         hipLaunchKernelGGL((k_syrk_outer<T, BF16, 0>), dim3(n), dim3(NTHREADS), 0, s, dp, sc, s0,
-                           s_end);
+                           s_end, wd > 0 ? wd : nb);
       if (tsy) {
         // outer update: an n x n lower triangle (n = 64 T) with rank K = 64 G
-        // counts n (n + 1) K flops; bytes: every lower tile read and written
-        // once, each trailing row block's G panel blocks read once
+        // counts n (n + 1) K flops (a part of it, its tiles' products); bytes:
+        // every tile read and written once, each trailing row block's G panel
+        // blocks read once
         const double es = sizeof(T);
+        auto part = [&](int nbm) {  // 64-tiles of a split update
+          return wide ? 4.0 * outer_tiles128(nbm - s_end, wd, rest)
+                      : (double)outer_tiles64(std::max(0, nbm - s_end), wd);
+        };
         timer_end(TC_SYRK, s, flops(sc, dp,
                                     [&](int nbm) {
                                       const double nn = (double)std::max(0, nbm - s_end) * TILE;
-                                      return nn * (nn + 1) * (double)(TILE * G);
+                                      return wd > 0 ? part(nbm) * G64 * G
+                                                    : nn * (nn + 1) * (double)(TILE * G);
                                     }),
                   flops(sc, dp, [&](int nbm) {
                     // (BF16 factors read the panel from its BF16 copy)
                     const double t = std::max(0, nbm - s_end);
-                    return t * (t + 1) * TILE * TILE * es +
+                    return (wd > 0 ? 2.0 * part(nbm) : t * (t + 1)) * TILE * TILE * es +
                            t * TILE * TILE * G * (BF16 ? 2.0 : es);
                   }));
       }
@@ -1828,22 +1966,40 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
     hipLaunchKernelGGL(k_factor_first<T>, dim3(1, b.count), dim3(NTHREADS), 0, s, b.dprobs);
     if (tpa) timer_end(TC_PANEL, s, b.count * F3, 0.0);
   }
+  auto rows_of = [&](int k) {  // row blocks from k on
+    int w = 0;
+    for (int m = 0; m < b.count; ++m) w += std::max(0, b.np(m) / TILE - k);
+    return w;
+  };
+  int ahead = -1;  // tiles of the last outer update left to the next super-step (-1: none)
   for (int k = 0; k < nb; ++k) {
     const int s0 = k / G * G, s_end = s0 + G;
     const bool outer = (k + 1 == s_end);
     if (col_style(s0)) {
       if (te.column_merge == 2) {
-        // every row block of the super-step's columns in the one launch
-        if (k == s0) superstep_launch<T, BF16>(b, s0, std::min(s_end, nb), nb, tpa, s);
+        // every row block of the super-step's columns in the one launch, with
+        // the rest of the previous super-step's outer update
+        if (k == s0)
+          superstep_launch<T, BF16>(b, s0, std::min(s_end, nb), nb, ahead < 0 ? -1 : s0 - G,
+                                    ahead, tpa, s);
       } else if (te.column_merge == 1) {
         if (k == s0) {
-          superstep_launch<T, BF16>(b, s0, std::min(s_end, nb), s_end, tpa, s);
+          superstep_launch<T, BF16>(b, s0, std::min(s_end, nb), s_end, -1, 0, tpa, s);
           if (s_end < nb) rows_launch<T, BF16>(b, s0, s_end, tpa, s);
         }
       } else {
         column_launch<T, BF16>(b, k, s0, tpa, s);
       }
-      if (outer && s_end < nb) outer_launch(s0, s_end, false);
+      if (outer && s_end < nb) {
+        ahead = -1;
+        int first;
+        if (te.column_merge == 2 && b.count <= LOOKB && s_end + G < nb)
+          ahead = look_tiles<T, BF16>(rows_of(s_end) - rows_of(s_end + G), rows_of(s_end + G),
+                                      first) /
+                  b.count;
+        if (ahead <= 0 || G % 2 != 0) ahead = -1;
+        outer_launch(s0, s_end, false, ahead);
+      }
       continue;
     }
     // U_k (k > s0): left-looking update of column k, factoring block k inside
@@ -1896,7 +2052,7 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
                                         const int t = std::max(0, b.np(m) / TILE - s_end);
                                         return t * (t + 1) / 2;
                                       }) <= fuse_max;
-      outer_launch(s0, s_end, fused);
+      outer_launch(s0, s_end, fused, -1);
       if (!fused && !next_col)
         sched_launch(
             b, [&](int m) { return b.np(m) / TILE > s_end ? 1 : 0; },

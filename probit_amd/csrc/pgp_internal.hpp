@@ -248,12 +248,14 @@ __device__ __forceinline__ double bcast(double v, int lane) {
   return __hiloint2double(hi, lo);
 }
 
-// Ticket of this workgroup in start order (thread 0 takes it; the last
-// ticket resets the counter for the next launch on the stream).
-__device__ __forceinline__ int take_ticket(uint32_t* ticket, int* lds_slot) {
+// Ticket of this workgroup in start order, of `total` that take one (thread 0
+// takes it; the last ticket resets the counter for the next launch on the
+// stream).
+__device__ __forceinline__ int take_ticket(uint32_t* ticket, int* lds_slot,
+                                           uint32_t total = gridDim.x) {
   if (threadIdx.x == 0) {
     const uint32_t t = atomicAdd(ticket, 1u);
-    if (t == gridDim.x - 1) atomicExch(ticket, 0u);
+    if (t == total - 1) atomicExch(ticket, 0u);
     *lds_slot = (int)t;
   }
   __syncthreads();

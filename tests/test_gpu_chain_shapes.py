@@ -108,3 +108,27 @@ def test_outer_update_tilings_agree(mode, count):
                          log_likelihood=P.log_probit_likelihood)
         w, p = gp.approximate_posterior((theta, lp))
         assert torch.equal(w, out[tag].weight) and torch.equal(p, out[tag].precision), tag
+
+
+# super-steps that carry a part of the outer update (odd and even trailing
+# block counts, all of it and a part, before and after the rows below) against
+# the two-launch form, which carries none: the same bits
+@pytest.mark.parametrize("mode,N", [("fp64", 1300), ("fp64", 4450), ("fp64", 7000),
+                                    ("fp32", 4450), ("fp32", 9000), ("bf16", 7000)])
+def test_superstep_with_outer_tiles_agrees(mode, N):
+    import torch
+
+    import probit_amd as P
+    from probit_amd import autotune as at
+    X, y, theta, lp, _ = small_problem(N, N, 2, "probit", "EQ", noise=0.5)
+    saved, out = at.get(mode, 1), []
+    try:
+        for merge in (1, 2):
+            at.set_entry(mode, 1, dict(saved, column_merge=merge))
+            gp = P.LaplaceGP(data=(X, y), prior=make_prior("EQ"), precision_mode=mode,
+                             log_likelihood=P.log_probit_likelihood)
+            out.append(gp.approximate_posterior((theta, lp)))
+    finally:
+        at.set_entry(mode, 1, saved)
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
