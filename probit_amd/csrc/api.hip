@@ -181,12 +181,20 @@ static GradLayout grad_layout(int64_t Np, int prec) {
 // device-side descriptor and pointer-array writes (kernel arguments carry the
 // host values, so no host buffer has to outlive the call)
 // ---------------------------------------------------------------------------
+// reset: of a new state, with the pointer array of the problem alone; 2: and
+// its weight z = 0, latent f = K 0.
 __global__ void k_write_prob(Prob* dst, Prob val, int reset) {
   const uint64_t* src = reinterpret_cast<const uint64_t*>(&val);
   uint64_t* d = reinterpret_cast<uint64_t*>(dst);
   const int nw = (int)(sizeof(Prob) / 8);
   for (int i = threadIdx.x; i < nw; i += blockDim.x) d[i] = src[i];
   if (reset) {
+    if (threadIdx.x == 0) *(Prob**)((char*)dst + OFF_ARR) = dst;
+    if (reset == 2)
+      for (int i = threadIdx.x; i < val.Np; i += blockDim.x) {
+        vslot(val, V_Z)[i] = 0.0;
+        vslot(val, V_F)[i] = 0.0;
+      }
     if (threadIdx.x < 4) val.info[threadIdx.x] = 0;
     if (threadIdx.x < NRED) val.red[threadIdx.x] = 0.0;
     // progress word and ticket counter of the header
@@ -391,6 +399,27 @@ static int check_resident(const Prob& p, unsigned states, const char* who,
 
 constexpr unsigned RS_PREDICT = (1u << RS_LAPLACE) | (1u << RS_VB);
 
+// The header's status words and gathered reductions in one copy: each costs a
+// small fit some 10 us, and every Newton iteration waits for one.
+struct HeadRead {
+  char b[OFF_PROGRESS - OFF_INFO];
+  int info() const {
+    int32_t v;
+    memcpy(&v, b, sizeof v);
+    return v;
+  }
+  double gather(int i) const {
+    double v;
+    memcpy(&v, b + (OFF_GATHER - OFF_INFO) + 8 * i, sizeof v);
+    return v;
+  }
+};
+static int read_head(const char* ws, hipStream_t s, HeadRead& h) {
+  HIP_OK(hipMemcpyAsync(h.b, ws + OFF_INFO, sizeof h.b, hipMemcpyDeviceToHost, s));
+  HIP_OK(hipStreamSynchronize(s));
+  return 0;
+}
+
 // Status bits of the factor and of the solves since the state was formed
 // (a non-positive pivot, an expired bounded wait): after the call's work.
 static int read_info_bits(const char* ws, hipStream_t s, int* bits) {
@@ -408,11 +437,6 @@ static Batch single_batch(char* ws, int Np) {
   b.maxNp = Np;
   b.ticket = (uint32_t*)(ws + OFF_TICKET);
   return b;
-}
-
-static void set_self(char* ws, hipStream_t s) {
-  std::vector<Prob*> v(1, (Prob*)(ws + OFF_PROB));
-  write_ptrs((Prob**)(ws + OFF_ARR), v, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -441,25 +465,26 @@ static void newton_iter(const Batch& all, const Batch* later, const Batch* fac,
                         double* gather, hipStream_t s) {
   // f = K z; at a member's first iteration z = 0 and f was zeroed with it
   if (later && later->count > 0) launch_gemv_sym(*later, V_Z, V_F, 0, s);
-  launch_lik_newton(all, s);
   // the members that re-factor B solve with the new W^1/2; the others keep
   // the one their factor was formed with (a chord step)
-  if (fac && fac->count > 0) launch_vec_op(*fac, OP_SNAP, s);
+  const bool snap = fac && fac->count == all.count;
+  launch_lik_newton(all, snap, s);
+  if (fac && fac->count > 0 && !snap) launch_vec_op(*fac, OP_SNAP, s);
   if (fac32 && fac32->count > 0) launch_vec_op(*fac32, OP_SNAP, s);
   if (fac && fac->count > 0) factor(*fac, prec, 0, s, V_R);
   if (fac32 && fac32->count > 0) factor(*fac32, PGP_PREC_FP32, 0, s, V_R);
   if (nofac && nofac->count > 0) launch_symv_tiles(*nofac, V_R, s);
   launch_symv_reduce(all, V_R, V_T, 1, s);
   solve_B(all, prec, s);
-  launch_vec_op(all, OP_STEP, s);
+  int op = OP_STEP;
   for (int r = 0; r < refine; ++r) {
+    launch_vec_op(all, op, s);
     launch_gemv_sym(all, V_DL, V_Q, 2, s);
     launch_gemv_sym(all, V_Q, V_T, 1, s);
     solve_B(all, prec, s);
-    launch_vec_op(all, OP_IRCORR, s);
+    op = OP_IRCORR;
   }
-  launch_vec_op(all, OP_ZUPD, s);
-  launch_reduce(all, RED_STEP, gather, s);
+  launch_newton_step(all, op, gather, s);
 }
 
 // Final state at the returned weight: f, W, sum log p, and B factored at W.
@@ -476,8 +501,7 @@ static void laplace_finalize(const Batch& all, const Batch* fac, const Batch* fa
   launch_lik_final(all, 0, s);
   if (fac && fac->count > 0) factor(*fac, prec, 0, s);
   if (fac32 && fac32->count > 0) factor(*fac32, PGP_PREC_FP32, 0, s);
-  launch_reduce(all, RED_FINAL, gather, s);
-  launch_vec_op(all, OP_OUT, s);
+  launch_reduce(all, RED_FINAL_OUT, gather, s);
 }
 
 // Status bits of a fit from its device status word, and a NaN objective
@@ -495,6 +519,10 @@ static void fill_result_final(pgp_fit_result_t* r, const double* g4, int info) {
   if (g4[3] > 0) r->status |= PGP_INFO_NEGATIVE_W;
   r->objective = -g4[0] + 0.5 * g4[1] + g4[2];
   apply_info(r, info);
+}
+static void fill_result_final(pgp_fit_result_t* r, const HeadRead& h) {
+  const double g4[4] = {h.gather(0), h.gather(1), h.gather(2), h.gather(3)};
+  fill_result_final(r, g4, h.info());
 }
 
 // Clear only the non-positive-pivot bit of each member's status word (a
@@ -965,12 +993,10 @@ static int laplace_fit_ws(const pgp_problem_t* problem, const pgp_kernel_t* kern
   const int refine = opts->refine >= 0 ? opts->refine : default_refine(prec);
   Prob p = make_prob(problem, kernel, lik, prec, ws);
   p.state = RS_LAPLACE;
-  write_prob(ws, p, 1, s);
-  set_self(ws, s);
+  write_prob(ws, p, 2, s);
   const Batch b = single_batch(ws, p.Np);
   double* gather = (double*)(ws + OFF_GATHER);
   launch_gram_self(b, s);
-  launch_vec_op(b, OP_ZERO_Z, s);
   rc = check_launch();
   if (rc) return rc;
   memset(result, 0, sizeof *result);
@@ -1008,15 +1034,14 @@ static int laplace_fit_ws(const pgp_problem_t* problem, const pgp_kernel_t* kern
     }
     rc = check_launch();
     if (rc) return rc;
-    double h2;
-    int32_t inf0;
-    HIP_OK(hipMemcpyAsync(&h2, gather, sizeof h2, hipMemcpyDeviceToHost, s));
-    HIP_OK(hipMemcpyAsync(&inf0, ws + OFF_INFO, sizeof inf0, hipMemcpyDeviceToHost, s));
-    HIP_OK(hipStreamSynchronize(s));
+    HeadRead head;
+    rc = read_head(ws, s, head);
+    if (rc) return rc;
     hold.release();
-    const double st = sqrt(h2);
+    const int inf0 = head.info();
+    const double st = sqrt(head.gather(0));
     if (cur == PGP_PREC_BF16 && ((inf0 & PGP_INFO_NOT_PD) || !(st == st))) {
-      // the step was not taken (OP_ZUPD); redo the iteration with FP32 updates
+      // the step was not taken (k_newton_step); redo the iteration with FP32 updates
       cur = PGP_PREC_FP32;
       result->status |= PGP_INFO_ESCALATED;
       force_factor = true;
@@ -1043,12 +1068,10 @@ static int laplace_fit_ws(const pgp_problem_t* problem, const pgp_kernel_t* kern
     laplace_finalize(b, gauss ? nullptr : &b, nullptr, cur, gather, s);
   rc = check_launch();
   if (rc) return rc;
-  double g4[4];
-  int32_t info[4];
-  HIP_OK(hipMemcpyAsync(g4, gather, sizeof g4, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipMemcpyAsync(info, ws + OFF_INFO, sizeof info, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipStreamSynchronize(s));
-  fill_result_final(result, g4, info[0]);
+  HeadRead head;
+  rc = read_head(ws, s, head);
+  if (rc) return rc;
+  fill_result_final(result, head);
   return 0;
 }
 
@@ -1158,7 +1181,6 @@ int pgp_vb_map(const pgp_problem_t* problem, const pgp_kernel_t* kernel,
   p.out_latent = nullptr;
   p.state = RS_VBMAP;
   write_prob(ws, p, 1, s);
-  set_self(ws, s);
   const Batch b = single_batch(ws, p.Np);
   launch_gram_self(b, s);
   launch_load_state(b, weight, nullptr, s);
@@ -1189,7 +1211,6 @@ int pgp_laplace_set_state(const pgp_problem_t* problem, const pgp_kernel_t* kern
   Prob p = make_prob(problem, kernel, lik, precision, ws);
   p.state = RS_LAPLACE;
   write_prob(ws, p, 1, s);
-  set_self(ws, s);
   const Batch b = single_batch(ws, p.Np);
   launch_gram_self(b, s);
   // weight -> Z, f = K a, log p at f, then W and S = sqrt(max(W, 0)) from the caller
@@ -1202,14 +1223,12 @@ int pgp_laplace_set_state(const pgp_problem_t* problem, const pgp_kernel_t* kern
   launch_reduce(b, RED_FINAL, gather, s);
   rc = check_launch();
   if (rc) return rc;
-  double g4[4];
-  int32_t info[4];
-  HIP_OK(hipMemcpyAsync(g4, gather, sizeof g4, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipMemcpyAsync(info, ws + OFF_INFO, sizeof info, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipStreamSynchronize(s));
+  HeadRead head;
+  rc = read_head(ws, s, head);
+  if (rc) return rc;
   if (result) {
     memset(result, 0, sizeof *result);
-    fill_result_final(result, g4, info[0]);
+    fill_result_final(result, head);
   }
   launch_vec_op(b, OP_OUT, s);
   return check_launch();
@@ -1344,11 +1363,11 @@ int pgp_laplace_grad(const pgp_kernel_t* kernel, const pgp_likelihood_t* lik, do
   launch_grad_trace(b, (double*)(gw + G.partials), kern_out, s);
   rc = check_launch();
   if (rc) return rc;
-  std::vector<double> hl(1 + PGP_MAX_CUT), hk(grad_npar());
+  std::vector<double> hl(64 + grad_npar());
+  const double* hk = hl.data() + 64;
   HIP_OK(hipMemcpyAsync(hl.data(), lik_out, hl.size() * 8, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipMemcpyAsync(hk.data(), kern_out, hk.size() * 8, hipMemcpyDeviceToHost, s));
   int bits = 0;
-  rc = read_info_bits(ws, s, &bits);  // also waits for the copies
+  rc = read_info_bits(ws, s, &bits);  // also waits for the copy
   if (rc) return rc;
   const int D = p.D, gm = grad_maxd();
   // an invalid factor or an expired wait in the adjoint's solves: NaN
@@ -1437,20 +1456,18 @@ int pgp_vb_grad(const pgp_kernel_t* kernel, const pgp_likelihood_t* lik, double*
   factor(b, prec, 0, s);
   rc = check_launch();
   if (rc) return rc;
-  std::vector<double> hl(1 + PGP_MAX_CUT), hk(grad_npar());
-  double hs[2], g4[4];
+  std::vector<double> hl(128 + 2);
+  const double *hk = hl.data() + 64, *hs = hl.data() + 128;
   HIP_OK(hipMemcpyAsync(hl.data(), lik_out, hl.size() * 8, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipMemcpyAsync(hk.data(), kern_out, hk.size() * 8, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipMemcpyAsync(hs, sig_out, sizeof hs, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipMemcpyAsync(g4, gather, sizeof g4, hipMemcpyDeviceToHost, s));
-  int bits = 0;
-  rc = read_info_bits(ws, s, &bits);  // also waits for the copies
+  HeadRead head;
+  rc = read_head(ws, s, head);  // also waits for the copy
   if (rc) return rc;
+  const int bits = head.info() & (PGP_INFO_NOT_PD | PGP_INFO_STALLED);
   const int D = p.D, gm = grad_maxd();
   const double sigma = p.noise_std;
   // W < 0 somewhere (the probit floor): the Woodbury form does not hold;
   // an invalid factor or an expired wait in the adjoint's solves: NaN too
-  const double bad = (g4[3] > 0 || bits) ? NAN : 0.0;
+  const double bad = (head.gather(3) > 0 || bits) ? NAN : 0.0;
   int o = 0;
   grad_out[o++] = hk[0] + bad;
   for (int d = 0; d < D; ++d) grad_out[o++] = hk[1 + d] + bad;
@@ -1484,13 +1501,11 @@ int pgp_vb_fit(const pgp_problem_t* problem, const pgp_kernel_t* kernel,
   p.S = gw + G.G2;
   p.Mp = p.Np;
   p.state = RS_VB;
-  write_prob(ws, p, 1, s);
-  set_self(ws, s);
+  write_prob(ws, p, 2, s);
   const Batch b = single_batch(ws, p.Np);
   double* gather = (double*)(ws + OFF_GATHER);
   launch_gram_self(b, s);
   factor(b, prec, 1, s);  // A = sigma^2 I + K
-  launch_vec_op(b, OP_ZERO_Z, s);
   rc = check_launch();
   if (rc) return rc;
   memset(result, 0, sizeof *result);
@@ -1509,15 +1524,13 @@ int pgp_vb_fit(const pgp_problem_t* problem, const pgp_kernel_t* kernel,
       launch_trsv(b, prec, 1, V_X3, V_X4, s);
       launch_vec_op(b, OP_VB_IRCORR, s);
     }
-    launch_vec_op(b, OP_VB_STEP, s);
-    launch_vec_op(b, OP_ZUPD, s);
-    launch_reduce(b, RED_STEP, gather, s);
+    launch_newton_step(b, OP_VB_STEP, gather, s);
     rc = check_launch();
     if (rc) return rc;
-    double h2;
-    HIP_OK(hipMemcpyAsync(&h2, gather, sizeof h2, hipMemcpyDeviceToHost, s));
-    HIP_OK(hipStreamSynchronize(s));
-    step = sqrt(h2);
+    HeadRead head;
+    rc = read_head(ws, s, head);
+    if (rc) return rc;
+    step = sqrt(head.gather(0));
     ++it;
     if (!(step == step)) break;
   }
@@ -1538,12 +1551,13 @@ int pgp_vb_fit(const pgp_problem_t* problem, const pgp_kernel_t* kernel,
   launch_vec_op(b, OP_OUT, s);
   rc = check_launch();
   if (rc) return rc;
-  double g4[4], tr[2];
-  int32_t info[4];
-  HIP_OK(hipMemcpyAsync(g4, gather, sizeof g4, hipMemcpyDeviceToHost, s));
+  double tr[2];
   HIP_OK(hipMemcpyAsync(tr, tr_out, sizeof tr, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipMemcpyAsync(info, ws + OFF_INFO, sizeof info, hipMemcpyDeviceToHost, s));
-  HIP_OK(hipStreamSynchronize(s));
+  HeadRead head;
+  rc = read_head(ws, s, head);  // also waits for the copy
+  if (rc) return rc;
+  double g4[4];
+  for (int i = 0; i < 4; ++i) g4[i] = head.gather(i);
   const double sigma = lik->noise_std;
   const double N = (double)problem->N;
   result->sum_log_lik = g4[0];
@@ -1552,7 +1566,7 @@ int pgp_vb_fit(const pgp_problem_t* problem, const pgp_kernel_t* kernel,
   // objective_VB (probit/implicit/VB.py:33-39)
   result->objective = 0.5 * tr[1] + 0.5 * sigma * sigma * tr[0] + 0.5 * g4[1] -
                       N * log(sigma) + g4[2] - 0.5 * N - g4[0];
-  apply_info(result, info[0]);  // NaN objective on a non-positive pivot or an expired wait
+  apply_info(result, head.info());  // NaN objective on a non-positive pivot or an expired wait
   return 0;
 }
 

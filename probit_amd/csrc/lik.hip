@@ -178,7 +178,7 @@ __device__ __forceinline__ LikParams likparams_from_prob(const Prob& P) {
 
 // ---- Newton step: F -> G, W, S, LL, R = G - Z ----
 __global__ __launch_bounds__(NTHREADS) void k_lik_newton(Prob* const* probs, Sched sc,
-                                                         int final_order) {
+                                                         int final_order, int snap) {
   int bx;
   const Prob& P = *probs[sched_member(sc, blockIdx.x, bx)];
   const int i = bx * NTHREADS + threadIdx.x;
@@ -197,24 +197,26 @@ __global__ __launch_bounds__(NTHREADS) void k_lik_newton(Prob* const* probs, Sch
   }
   vslot(P, V_G)[i] = g;
   vslot(P, V_W)[i] = w;
-  vslot(P, V_S)[i] = sqrt(fmax(w, 0.0));
+  const double sq = sqrt(fmax(w, 0.0));
+  vslot(P, V_S)[i] = sq;
+  if (snap) vslot(P, V_SF)[i] = sq;  // B is about to be formed with it (OP_SNAP)
   vslot(P, V_LL)[i] = ll;
   if (final_order == 0) vslot(P, V_R)[i] = g - vslot(P, V_Z)[i];
   if (final_order >= 3) vslot(P, V_D3)[i] = d3;
 }
 
-static void lik_launch(const Batch& b, int order, hipStream_t s) {
+static void lik_launch(const Batch& b, int order, int snap, hipStream_t s) {
   sched_launch(
       b, [&](int m) { return (b.np(m) + NTHREADS - 1) / NTHREADS; },
       [&](Prob* const* dp, const Sched& sc, int n) {
-        hipLaunchKernelGGL(k_lik_newton, dim3(n), dim3(NTHREADS), 0, s, dp, sc, order);
+        hipLaunchKernelGGL(k_lik_newton, dim3(n), dim3(NTHREADS), 0, s, dp, sc, order, snap);
       });
 }
 
-void launch_lik_newton(const Batch& b, hipStream_t s) { lik_launch(b, 0, s); }
+void launch_lik_newton(const Batch& b, int snap, hipStream_t s) { lik_launch(b, 0, snap, s); }
 
 void launch_lik_final(const Batch& b, int order3, hipStream_t s) {
-  lik_launch(b, order3 ? 3 : 2, s);
+  lik_launch(b, order3 ? 3 : 2, 0, s);
 }
 
 // ---- raw elementwise evaluation (kernel-level ABI) ----

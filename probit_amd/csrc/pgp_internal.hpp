@@ -318,7 +318,7 @@ int launch_gram_raw(const pgp_kernel_t* k, int dtype, const double* X, int64_t N
                     const double* Z, int64_t M, void* out, int64_t ld, hipStream_t s);
 
 // lik.hip
-void launch_lik_newton(const Batch& b, hipStream_t s);
+void launch_lik_newton(const Batch& b, int snap, hipStream_t s);  // snap: with OP_SNAP
 void launch_lik_final(const Batch& b, int order3, hipStream_t s);
 int launch_lik_raw(const pgp_likelihood_t* lik, const double* f, const double* y, int64_t N,
                    double* ll, double* d1, double* d2, hipStream_t s);
@@ -367,7 +367,6 @@ int launch_trsm_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const d
 enum VecOp {
   OP_STEP = 0,
   OP_IRCORR = 1,
-  OP_ZUPD = 2,
   OP_ZERO_Z = 3,
   OP_OUT = 4,
   OP_VB_RHS = 5,
@@ -384,7 +383,10 @@ enum VecOp {
   OP_VBG_SHAT = 15,  // X3 = Z - G - sigma W .* X4, X1 = 0, X2 = sigma X4
   OP_SNAP = 16,      // SF = S: the W^1/2 of the factor B is about to be formed with
 };
-enum RedWhat { RED_STEP = 0, RED_FINAL = 1 };
+enum RedWhat { RED_FINAL = 0, RED_FINAL_OUT = 1 };  // _OUT: with OP_OUT
+// A Newton step's end in one launch: OP_STEP, OP_IRCORR or OP_VB_STEP, then
+// z += delta (not from a failed factor) and ||delta||^2 to gather[b]
+void launch_newton_step(const Batch& b, int op, double* gather, hipStream_t s);
 void launch_gemv_sym(const Batch& b, int x_slot, int out_slot, int mode, hipStream_t s);
 // the two halves of launch_gemv_sym's symmetric product (modes < 10)
 void launch_symv_tiles(const Batch& b, int x_slot, hipStream_t s);

@@ -213,9 +213,6 @@ __global__ __launch_bounds__(NTHREADS) void k_vec(Prob* const* probs, Sched sc, 
     case OP_SNAP:
       vslot(P, V_SF)[i] = vslot(P, V_S)[i];
       break;
-    case OP_ZUPD:  // a step from a failed factor is not taken
-      if (!(P.info[0] & PGP_INFO_NOT_PD)) vslot(P, V_Z)[i] += vslot(P, V_DL)[i];
-      break;
     case OP_ZERO_Z:  // the zero weight and its latent f = K 0
       vslot(P, V_Z)[i] = 0.0;
       vslot(P, V_F)[i] = 0.0;
@@ -333,50 +330,77 @@ __device__ double block_sum(double v) {
 
 
 
-__global__ __launch_bounds__(NTHREADS) void k_reduce(Prob* const* probs, int what,
-                                                     double* gather) {
+// One workgroup per member: at N = 16384 a thread has 64 elements, some 10 us;
+// a launch each for the step, the update and the norm cost a small fit as much
+// (N = 20, with the status and the norm read back in one copy: 359 -> 308 us a
+// fit and its predict).
+__global__ __launch_bounds__(NTHREADS) void k_newton_step(Prob* const* probs, int op,
+                                                          double* gather) {
   const Prob& P = *probs[blockIdx.x];
-  if (what == RED_STEP) {
-    const double* d = vslot(P, V_DL);
-    double a = 0.0;
-    for (int i = threadIdx.x; i < P.Np; i += NTHREADS) a += d[i] * d[i];
-    const double s = block_sum(a);
-    if (threadIdx.x == 0) {
-      P.red[R_STEP2] = s;
-      if (gather) gather[blockIdx.x] = s;
-    }
-  } else {
-    const double* ll = vslot(P, V_LL);
-    const double* f = vslot(P, V_F);
-    const double* z = vslot(P, V_Z);
-    const double* w = vslot(P, V_W);
-    double a = 0.0, b = 0.0, c = 0.0, n = 0.0;
-    for (int i = threadIdx.x; i < P.Np; i += NTHREADS) {
-      a += ll[i];
-      b += f[i] * z[i];
-      c += P.logdiag[i];
-      n += (i < P.N && w[i] < 0.0) ? 1.0 : 0.0;
-    }
-    const double sa = block_sum(a);
-    const double sb = block_sum(b);
-    const double sc = block_sum(c);
-    const double sn = block_sum(n);
-    if (threadIdx.x == 0) {
-      P.red[R_SUMLL] = sa;
-      P.red[R_FA] = sb;
-      P.red[R_LOGDET] = sc;
-      P.red[R_NEGW] = sn;
-      if (gather) {
-        gather[8 * blockIdx.x + 0] = sa;
-        gather[8 * blockIdx.x + 1] = sb;
-        gather[8 * blockIdx.x + 2] = sc;
-        gather[8 * blockIdx.x + 3] = sn;
-        gather[8 * blockIdx.x + 4] = (double)P.info[0];
-      }
-    }
+  const int np = uniform(P.Np);
+  const double* vec = uniform(P.vec);
+  const auto slot = [&](int v) { return gbl((double*)vec + (size_t)v * np); };
+  const auto DL = slot(V_DL), Z = slot(V_Z);
+  const auto U = slot(V_U), R = slot(op == OP_IRCORR ? V_Q : V_R), SF = slot(V_SF);
+  const bool take = !(P.info[0] & PGP_INFO_NOT_PD);  // no step from a failed factor
+  double a = 0.0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < np; i += NTHREADS) {
+    const double z = Z[i];
+    double d = op == OP_VB_STEP ? U[i] - z : R[i] - SF[i] * U[i];
+    if (op == OP_IRCORR) d += DL[i];
+    DL[i] = d;
+    if (take) Z[i] = z + d;
+    a += d * d;
+  }
+  const double s = block_sum(a);
+  if (threadIdx.x == 0) {
+    P.red[R_STEP2] = s;
+    if (gather) gather[blockIdx.x] = s;
   }
 }
 
+void launch_newton_step(const Batch& b, int op, double* gather, hipStream_t s) {
+  hipLaunchKernelGGL(k_newton_step, dim3(b.count), dim3(NTHREADS), 0, s, b.dprobs, op, gather);
+}
+
+__global__ __launch_bounds__(NTHREADS) void k_reduce(Prob* const* probs, int what,
+                                                     double* gather) {
+  const Prob& P = *probs[blockIdx.x];
+  const double* ll = vslot(P, V_LL);
+  const double* f = vslot(P, V_F);
+  const double* z = vslot(P, V_Z);
+  const double* w = vslot(P, V_W);
+  double a = 0.0, b = 0.0, c = 0.0, n = 0.0;
+  for (int i = threadIdx.x; i < P.Np; i += NTHREADS) {
+    a += ll[i];
+    b += f[i] * z[i];
+    c += P.logdiag[i];
+    n += (i < P.N && w[i] < 0.0) ? 1.0 : 0.0;
+    if (what == RED_FINAL_OUT && i < P.N) {  // OP_OUT
+      if (P.out_weight) P.out_weight[i] = z[i];
+      if (P.out_prec) P.out_prec[i] = w[i];
+      if (P.out_latent) P.out_latent[i] = f[i];
+    }
+  }
+  const double sa = block_sum(a);
+  const double sb = block_sum(b);
+  const double sc = block_sum(c);
+  const double sn = block_sum(n);
+  if (threadIdx.x == 0) {
+    P.red[R_SUMLL] = sa;
+    P.red[R_FA] = sb;
+    P.red[R_LOGDET] = sc;
+    P.red[R_NEGW] = sn;
+    if (gather) {
+      gather[8 * blockIdx.x + 0] = sa;
+      gather[8 * blockIdx.x + 1] = sb;
+      gather[8 * blockIdx.x + 2] = sc;
+      gather[8 * blockIdx.x + 3] = sn;
+      gather[8 * blockIdx.x + 4] = (double)P.info[0];
+    }
+  }
+}
 void launch_reduce(const Batch& b, int what, double* gather, hipStream_t s) {
   hipLaunchKernelGGL(k_reduce, dim3(b.count), dim3(NTHREADS), 0, s, b.dprobs, what, gather);
 }
