@@ -444,13 +444,11 @@ int launch_trsv_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const d
 }
 
 // ---- TRSM: S <- L^-1 S, S is Np x Mp (ld lds) ----
-// FP64 solves, the transposed solves, and FP32 solves of at most WAVE_NCT
-// column tiles (serving) run as one wavefront launch (k_trsm_rows, below).
-// The others, wider FP32 solves, take a launch per block row (up to TRSM_WIDE
-// column tiles) or per super-step of G block rows: they subtract each block
-// row's (super-step's) product from S in FP32, and a wavefront's one sum over
-// all of them would round differently.  So do solves without a ticket
-// counter, or on a bare matrix.
+// With a ticket counter and up to MAXB block rows a solve is one wavefront
+// launch (k_trsm_rows, below), in FP32 with the roundings of the schedule its
+// width would take without: a launch per block row (up to TRSM_WIDE column
+// tiles) or per super-step of G block rows, which subtract each block row's
+// (super-step's) product from S.
 //
 // Per block row (lagged).
 // Lagged schedule.  Launch k, workgroup (w, ct), row block i = k + w:
@@ -563,9 +561,14 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged_raw(const T* L, int64_
 // 4096: 20.3 ms in 16 launches of 4 column tiles, 2.8 ms (98 TFLOP/s) in one.
 constexpr int WAVE_NCT = 4;
 
-template <typename T>
-__global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sched rows, int nct,
-                                                        int ct0, uint32_t* ticket,
+//
+// GRP: the sum is taken off S_i, in its type, after every 1 << lg blocks but
+// the last whole group before i's own: the roundings of the schedules of one
+// launch per block row (lg = 0) or super-step of TRSM_G (lg = 2), which FP32
+// solves of more than WAVE_NCT column tiles follow without a ticket counter.
+template <typename T, bool GRP>
+__global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 2 : 3) void k_trsm_rows(Prob* const* probs, Sched rows, int nct,
+                                                        int ct0, int lg, uint32_t* ticket,
                                                         uint32_t epoch) {
   constexpr int PP = KP<T>::value;  // A operand: conflict-free MFMA reads
   constexpr int PB = TILE + 1;       // B operand: written transposed, conflict-free stores
@@ -592,8 +595,14 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
   const int cb = uniform((int)(threadIdx.x >> 6));
   // la: the next A operand (L_ij, at last DINV_i), fetched during the
   // product before its own; xb: the next X_j, fetched as early when it is
-  // known to be published, and during the last product S_i.
-  T la[16], xb[16];
+  // known to be published, and (sv) during the last product S_i.
+  T la[16], xb[16], si[GRP ? 16 : 1];
+  T(&sv)[16] = [&]() -> T(&)[16] {
+    if constexpr (GRP)
+      return si;
+    else
+      return xb;
+  }();
   auto fetch_l = [&](int k) {
     auto p = L + (ri + ((int64_t)k * TILE + cb) * ld);
 #pragma unroll
@@ -604,14 +613,14 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
 #pragma unroll
     for (int q = 0; q < 16; ++q) la[q] = (T)D[r + (size_t)(4 * q) * TILE];
   };
-  auto fetch_s = [&]() {  // accumulator layout
+  auto fetch_s = [&](T (&v)[16]) {  // accumulator layout
 #pragma unroll
     for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
       for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          xb[8 * bm + 4 * bn + q] =
+          v[8 * bm + 4 * bn + q] =
               S[(size_t)(ri + acc_row<T>(bm, q)) + (size_t)(n0 + acc_col(bn)) * ld];
   };
   auto fetch_x = [&](int k) {  // published in this launch: coherent loads
@@ -620,11 +629,12 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
     for (int q = 0; q < 16; ++q, p += 4 * ld)
       xb[q] = __hip_atomic_load(p + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
+  if constexpr (GRP) fetch_s(sv);
   if (i > 0) {
     fetch_l(0);
   } else {
     fetch_d();
-    fetch_s();
+    if constexpr (!GRP) fetch_s(sv);
   }
   acc_t acc[2][2];
   zero_acc<T>(acc);
@@ -649,10 +659,21 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
       if (done < ready) fetch_x(done);
     } else {
       fetch_d();
-      fetch_s();
+      if constexpr (!GRP) fetch_s(sv);
     }
     __syncthreads();
     mma64_kmajor<T>(As, PP, Bs, PB, acc);
+    if constexpr (GRP) {
+      if ((done & ((1 << lg) - 1)) == 0 && (done >> lg) < (i >> lg)) {
+#pragma unroll
+        for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+          for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sv[8 * bm + 4 * bn + q] -= acc[bm][bn][q];
+        zero_acc<T>(acc);
+      }
+    }
   }
   // X_i = DINV_i (S_i - acc)
   __syncthreads();
@@ -663,7 +684,7 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows(Prob* const* probs, Sche
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int row = acc_row<T>(bm, q), col = acc_col(bn);
-        Bs[row * PB + col] = xb[8 * bm + 4 * bn + q] - acc[bm][bn][q];
+        Bs[row * PB + col] = sv[8 * bm + 4 * bn + q] - acc[bm][bn][q];
       }
 #pragma unroll
   for (int q = 0; q < 16; ++q) As[(cb + 4 * q) * PP + r] = la[q];
@@ -1044,16 +1065,13 @@ static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, hipStream_t
   }
 }
 
-// FP32, N = 8192, M = 4096: 196 -> 117 us a launch with the addresses from
-// scalar registers (376 vector registers held one workgroup a CU; 152 hold 3).
 // Right-hand sides of at least this many column tiles take the super-step
 // schedule.
 constexpr int TRSM_WIDE = 16;
 
 void launch_trsm(const Batch& bt, int prec, int maxMp, hipStream_t s) {
   const int mt = maxMp / TILE;
-  if (bt.ticket && (prec == PGP_PREC_FP64 || mt <= WAVE_NCT) && bt.maxNp / TILE <= MAXB &&
-      wavefront_trsm()) {
+  if (bt.ticket && bt.maxNp / TILE <= MAXB && wavefront_trsm()) {
     for (int ct0 = 0; ct0 < mt; ct0 += PROGRESS_CT) {
       // row-major schedule: row i holds the members with more than i block
       // rows (a prefix: members are sorted by size), nct workgroups each
@@ -1081,11 +1099,14 @@ void launch_trsm(const Batch& bt, int prec, int maxMp, hipStream_t s) {
       }
       const uint32_t ep = next_epoch();
       if (prec == PGP_PREC_FP64)
-        hipLaunchKernelGGL(k_trsm_rows<double>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                           nct, ct0, bt.ticket, ep);
+        hipLaunchKernelGGL((k_trsm_rows<double, false>), dim3(tot), dim3(NTHREADS), 0, s,
+                           bt.dprobs, rows, nct, ct0, 0, bt.ticket, ep);
+      else if (mt <= WAVE_NCT)
+        hipLaunchKernelGGL((k_trsm_rows<float, false>), dim3(tot), dim3(NTHREADS), 0, s,
+                           bt.dprobs, rows, nct, ct0, 0, bt.ticket, ep);
       else
-        hipLaunchKernelGGL(k_trsm_rows<float>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                           nct, ct0, bt.ticket, ep);
+        hipLaunchKernelGGL((k_trsm_rows<float, true>), dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs,
+                           rows, nct, ct0, mt < TRSM_WIDE ? 0 : 2, bt.ticket, ep);
       if (on) timer_end(TC_TRSM, s, fl, 0.0);
     }
     return;
