@@ -684,10 +684,12 @@ __global__ __launch_bounds__(NTHREADS) void k_syrk_outer(Prob* const* probs, Sch
 // columns through two LDS buffers (one barrier per chunk), a chunk fetched
 // into registers during the product before its own.  The k order inside and
 // across the MFMA steps is the 64-tile's, so both give the same bits.  Bound
-// by the MFMAs (60 TFLOP/s FP64, 121 FP32 at the sizes below), BF16 by C's
-// bytes; per launch, 64- against 128-tiles: FP64, 184 block rows, K = 512:
-// 1570 -> 1188 us; FP32, 244, K = 768: 1946 -> 1569; BF16, 248, K = 512: 622
-// -> 323.  A third of FP32's gain is the addresses: tile indices from a square
+// by the MFMAs and then C's bytes (of N = 12288's 755 us a launch of 3496
+// tiles, K = 384, 704 remain without the loop's fetches and LDS stores: 560 of
+// MFMAs, and C's 180 partly under them); BF16 by C's bytes.  Per launch, 64-
+// against 128-tiles: FP64, 184 block rows, K = 512: 1570 -> 1188 us (60
+// TFLOP/s); FP32, 244, K = 768: 1946 -> 1569 (121); BF16, 248, K = 512: 622 ->
+// 323.  A third of FP32's gain is the addresses: tile indices from a square
 // root and descriptor fields arrive in vector registers, and 80 64-bit vector
 // additions per chunk then hold up the MFMAs (hence uniform()).
 template <typename T, int BF16>
@@ -876,14 +878,26 @@ __device__ __forceinline__ void outer128_tile(const Prob& P, int bx, int s0, int
   if (nc > 1)
 #pragma unroll
     for (int q = 0; q < 4; ++q) fetch(1, q);
+  // (FP32: C arrives during the last chunk's product)
+  typedef __attribute__((address_space(1))) floatx4* gf4;
+  const auto C = A + (ri + wr + (rj + wc) * ld);
+  floatx4 cv[F64 ? 1 : 4][4];
   int c = 0;
   for (; c + 2 < nc; ++c) chunk(c, std::true_type{}, std::true_type{});
   if (c + 1 < nc) chunk(c++, std::true_type{}, std::false_type{});
+  if constexpr (!F64) {
+    if (active) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          cv[i][j] = *(gf4)(C + (16 * i + 16 * j * ld) + (4 * lk + lr * (unsigned)ld));
+    }
+  }
   chunk(c, std::false_type{}, std::false_type{});
   if (!active) return;
   // ---- C -= acc ----
   if constexpr (F64) {
-    const auto C = A + (ri + wr + (rj + wc) * ld);
     const unsigned o = lr + lk * (unsigned)ld;
     double v[2][16];
     auto load = [&](int j) {
@@ -904,18 +918,11 @@ __device__ __forceinline__ void outer128_tile(const Prob& P, int bx, int s0, int
           (C + (16 * i + (16 * j + 4 * r) * ld))[o] = v[j & 1][4 * i + r] - acc[i][j][r];
     }
   } else {
-    typedef __attribute__((address_space(1))) floatx4* gf4;
-    const auto C = A + (ri + wr + (rj + wc) * ld);
     const unsigned o = 4 * lk + lr * (unsigned)ld;
-    floatx4 v[4][4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i][j] = *(gf4)(C + (16 * i + 16 * j * ld) + o);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *(gf4)(C + (16 * i + 16 * j * ld) + o) = v[i][j] - acc[i][j];
+      for (int i = 0; i < 4; ++i) *(gf4)(C + (16 * i + 16 * j * ld) + o) = cv[i][j] - acc[i][j];
   }
 }
 
