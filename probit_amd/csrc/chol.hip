@@ -1278,6 +1278,72 @@ __device__ __forceinline__ void mma_operands(const LT* a, const LT* b,
     mma64_kmajor<T>(a, KP<T>::value, b, KP<T>::value, acc);
 }
 
+// prod += A B over K = 64 for k-major operands with B(k, n) = 0 for k > n (the
+// transposed inverse): each wave 16 rows, block column b up to its k only, 40
+// MFMAs for the 64 of a wave's quadrant of the whole product (the others add
+// zeros, so the result is the same bits).
+template <typename T>
+__device__ __forceinline__ void mma64_upper(const T* As, const T* Bs, int p,
+                                            typename Acc<T>::type (&prod)[4]) {
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const T* a = As + (l >> 4) * p + 16 * w + (l & 15);
+  const T* b = Bs + (l >> 4) * p + (l & 15);
+  T av[2], bv[2][4];
+  auto read = [&](int s) {
+    av[s & 1] = a[4 * s * p];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (4 * c + 3 >= s) bv[s & 1][c] = b[4 * s * p + 16 * c];
+  };
+  read(0);
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    if (s < 15) read(s + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (4 * c + 3 >= s) prod[c] = mfma16(av[s & 1], bv[s & 1][c], prod[c]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// The ten 16 x 16 blocks on and below the diagonal of a 64 x 64 product A A^T
+// (k-major operand), at most three to a wave: block b of wave w.
+__device__ __forceinline__ void lower_block(int w, int b, int& i, int& j) {
+  // w = 0: (3,0) (3,1) (0,0); 1: (3,2) (3,3) (1,0); 2: (2,0) (2,1) (1,1); 3: (2,2)
+  i = (0xa9a7cf >> (6 * w + 2 * b)) & 3;
+  j = (0xa94384 >> (6 * w + 2 * b)) & 3;
+}
+template <typename T>
+__device__ __forceinline__ void mma64_lower(const T* As, int p, typename Acc<T>::type (&acc)[3]) {
+  const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const T *a[3], *c[3];
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    int i, j;
+    lower_block(w, b, i, j);
+    a[b] = As + (l >> 4) * p + 16 * i + (l & 15);
+    c[b] = As + (l >> 4) * p + 16 * j + (l & 15);
+  }
+  T av[2][3], cv[2][3];
+  auto read = [&](int s) {
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      av[s & 1][b] = a[b][4 * s * p];
+      cv[s & 1][b] = c[b][4 * s * p];
+    }
+  };
+  read(0);
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    if (s < 15) read(s + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < 3; ++b) acc[b] = mfma16(av[s & 1][b], cv[s & 1][b], acc[b]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // LDS of the super-step kernel: the panel product's two operands and the
 // updates' two, or the diagonal factor's block.
 template <typename T, int BF16>
@@ -1362,9 +1428,14 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
   auto colk = [&](int64_t r0, int64_t c0) { return A + (r0 + (c0 + operand_k<CK>(kb, 0)) * ld); };
   constexpr int KS = CK ? 1 : 4;
   // acc: update of the current (then the next) tile; accd: of the diagonal tile
-  acc_t acc[2][2], accd[2][2], prod[2][2];
+  constexpr bool F64 = std::is_same<T, double>::value;
+  acc_t acc[2][2], accd[2][2], accl[3], prod[4];
   zero_acc<T>(acc);
   zero_acc<T>(accd);
+#pragma unroll
+  for (int b = 0; b < 3; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) accl[b][r] = (T)0;
   T av[16], ra[2][16], rb[2][16];
   auto load_a = [&](int64_t c0) {
     auto p = col4(ri, c0);
@@ -1439,12 +1510,19 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
       for (int q = 0; q < 16; ++q) bk[(kb + 4 * q) * PP + m] = (T)dv[q];
     }
     __syncthreads();
-    zero_acc<T>(prod);
-    mma64_kmajor<T>(ck, PP, bk, PP, prod);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) prod[b][r] = (T)0;
+    mma64_upper<T>(ck, bk, PP, prod);
     __syncthreads();
     // L_ij through LDS: whole columns per store, and the operand of the
     // following updates
-    to_lds(ck, prod);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        ck[(16 * b + (m & 15)) * PP + 16 * kb + acc_row<T>(0, r) - 32 * (kb >> 1)] = prod[b][r];
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 16; ++q) ra[0][q] = ck[operand_k<CK>(kb, q) * PP + m];
@@ -1463,7 +1541,12 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
       load_a(c0 + TILE);  // the next tile (the diagonal one after the last)
       stash_operand<T, BF16>(sa, ra[0], m, kb);
       __syncthreads();
-      if (diag) mma_operands<T, BF16>(sa, sa, accd);
+      if (diag) {
+        if constexpr (F64)
+          mma64_lower<T>(sa, PP, accl);
+        else
+          mma_operands<T, BF16>(sa, sa, accd);
+      }
     }
     // every wave's stores complete: publish the tile (and read it back as an
     // operand of the next columns)
@@ -1484,6 +1567,18 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
   if (diag) {
     __syncthreads();
     double (*blk)[TILE + 1] = (double (*)[TILE + 1])arena;
+    if constexpr (F64) {
+      // (the blocks above the diagonal ones are not read by the factor)
+#pragma unroll
+      for (int b = 0; b < 3; ++b) {
+        if (kb == 3 && b > 0) break;
+        int bi, bj;
+        lower_block(kb, b, bi, bj);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          blk[16 * bi + acc_row<T>(0, r) - 32 * (kb >> 1)][16 * bj + (m & 15)] = accl[b][r];
+      }
+    } else {
 #pragma unroll
     for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
@@ -1491,6 +1586,7 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           blk[acc_row<T>(bm, r)][acc_col(bn)] = (double)(T)accd[bm][bn][r];
+    }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
