@@ -1278,35 +1278,6 @@ __device__ __forceinline__ void mma_operands(const LT* a, const LT* b,
     mma64_kmajor<T>(a, KP<T>::value, b, KP<T>::value, acc);
 }
 
-// prod += A B over K = 64 for k-major operands with B(k, n) = 0 for k > n (the
-// transposed inverse): each wave 16 rows, block column b up to its k only, 40
-// MFMAs for the 64 of a wave's quadrant of the whole product (the others add
-// zeros, so the result is the same bits).
-template <typename T>
-__device__ __forceinline__ void mma64_upper(const T* As, const T* Bs, int p,
-                                            typename Acc<T>::type (&prod)[4]) {
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const T* a = As + (l >> 4) * p + 16 * w + (l & 15);
-  const T* b = Bs + (l >> 4) * p + (l & 15);
-  T av[2], bv[2][4];
-  auto read = [&](int s) {
-    av[s & 1] = a[4 * s * p];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (4 * c + 3 >= s) bv[s & 1][c] = b[4 * s * p + 16 * c];
-  };
-  read(0);
-#pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    if (s < 15) read(s + 1);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (4 * c + 3 >= s) prod[c] = mfma16(av[s & 1], bv[s & 1][c], prod[c]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
 // The ten 16 x 16 blocks on and below the diagonal of a 64 x 64 product A A^T
 // (k-major operand), at most three to a wave: block b of wave w.
 __device__ __forceinline__ void lower_block(int w, int b, int& i, int& j) {
@@ -1514,7 +1485,7 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
     for (int b = 0; b < 4; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r) prod[b][r] = (T)0;
-    mma64_upper<T>(ck, bk, PP, prod);
+    mma64_tri<T, false, false>(bk, PP, ck, PP, prod);
     __syncthreads();
     // L_ij through LDS: whole columns per store, and the operand of the
     // following updates

@@ -99,6 +99,41 @@ __device__ __forceinline__ void mma64_kmajor(const T* As, int pa, const T* Bs, i
   }
 }
 
+// prod += A B over K = 64 where one operand M is triangular (a diagonal block's
+// inverse), k-major: its block column (row) c of 16 has zeros for k >= 16 (c +
+// 1), or (HI) for k < 16 c.  Each wave takes the 16 rows (columns) 16 w.. of
+// the other operand F, and block c up to (from) its k only: 40 MFMAs for the
+// 64 of a wave's quadrant of the whole product.  The others add zeros, so the
+// result is mma64_kmajor's.  MA: M is A, and prod[c] rows 16 c.., columns 16
+// w..; otherwise M is B, rows 16 w.., columns 16 c...
+template <typename T, bool MA, bool HI>
+__device__ __forceinline__ void mma64_tri(const T* M, int pm, const T* F, int pf,
+                                          typename Acc<T>::type (&prod)[4]) {
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const T* a = F + (l >> 4) * pf + 16 * w + (l & 15);
+  const T* b = M + (l >> 4) * pm + (l & 15);
+  T fv[2], mv[2][4];
+  auto has = [](int c, int s) { return HI ? s >= 4 * c : s <= 4 * c + 3; };
+  auto read = [&](int s) {
+    fv[s & 1] = a[4 * s * pf];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (has(c, s)) mv[s & 1][c] = b[4 * s * pm + 16 * c];
+  };
+  read(0);
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    if (s < 15) read(s + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (has(c, s))
+        prod[c] = MA ? mfma16(mv[s & 1][c], fv[s & 1], prod[c])
+                     : mfma16(fv[s & 1], mv[s & 1][c], prod[c]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // acc += A B^T over K = 64 for float, m-major LDS operands As[m * pa + k],
 // Bs[n * pb + k] (pa, pb multiples of 4; with pa = pb = 4 mod 32 the 16-byte
 // reads of 8 consecutive lanes cover the 32 banks once; the counters still

@@ -557,7 +557,8 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged_raw(const T* L, int64_
 // the hand-off, ~9 us); FP64 at N = 3000, M = 5000: 2400 us as 12 super-step
 // launches, whose solving workgroups run 30 tile products in a row; 1712 in
 // one wavefront launch; 1207 (38 TFLOP/s) with the operands fetched a product
-// ahead.  N = 1537, M = 501: 590 -> 269 us.  Transposed, FP32 at N = 8192, M =
+// ahead; 1110 (41) with DINV's zeros left out and X_i stored by whole columns
+// (256 test points, FP32, a stream of fits: 68.5 -> 65.8 ms).  N = 1537, M = 501: 590 -> 269 us.  Transposed, FP32 at N = 8192, M =
 // 4096: 20.3 ms in 16 launches of 4 column tiles, 2.8 ms (98 TFLOP/s) in one.
 constexpr int WAVE_NCT = 4;
 
@@ -689,16 +690,27 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 2 : 3) void k_trsm_rows(
 #pragma unroll
   for (int q = 0; q < 16; ++q) As[(cb + 4 * q) * PP + r] = la[q];
   __syncthreads();
-  zero_acc<T>(acc);
-  mma64_kmajor<T>(As, PP, Bs, PB, acc);
+  acc_t prod[4];
 #pragma unroll
-  for (int bm = 0; bm < 2; ++bm)
+  for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int bn = 0; bn < 2; ++bn)
+    for (int q = 0; q < 4; ++q) prod[b][q] = (T)0;
+  mma64_tri<T, true, false>(As, PP, Bs, PB, prod);
+  __syncthreads();
+  // X_i through LDS: whole columns per store
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        __hip_atomic_store(&S[(size_t)(ri + acc_row<T>(bm, q)) + (size_t)(n0 + acc_col(bn)) * ld],
-                           (T)acc[bm][bn][q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      Bs[(16 * cb + (r & 15)) * PB + 16 * b + acc_row<T>(0, q) - 32 * (cb >> 1)] = prod[b][q];
+  __syncthreads();
+  {
+    auto p = S + (ri + (n0 + cb) * ld);
+#pragma unroll
+    for (int q = 0; q < 16; ++q, p += 4 * ld)
+      __hip_atomic_store(p + r, Bs[(cb + 4 * q) * PB + r], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
   publish_wait();  // every wave's X_i stores complete ...
   __syncthreads();
   if (threadIdx.x == 0)  // ... before (i + 1, ct) may read them
@@ -822,16 +834,27 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
 #pragma unroll
   for (int q = 0; q < 16; ++q) As[r * PA + cb + 4 * q] = la[q];  // A(m, k) = DINV_i(k, m)
   __syncthreads();
-  zero_acc<T>(acc);
-  mma64_kmajor<T>(As, PA, Bs, PB, acc);
+  acc_t prod[4];
 #pragma unroll
-  for (int bm = 0; bm < 2; ++bm)
+  for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int bn = 0; bn < 2; ++bn)
+    for (int q = 0; q < 4; ++q) prod[b][q] = (T)0;
+  mma64_tri<T, true, true>(As, PA, Bs, PB, prod);
+  __syncthreads();
+  // X_i through LDS: whole columns per store
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        __hip_atomic_store(&S[(size_t)(ri + acc_row<T>(bm, q)) + (size_t)(n0 + acc_col(bn)) * ld],
-                           (T)acc[bm][bn][q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      Bs[(16 * cb + (r & 15)) * PB + 16 * b + acc_row<T>(0, q) - 32 * (cb >> 1)] = prod[b][q];
+  __syncthreads();
+  {
+    auto p = S + (ri + (n0 + cb) * ld);
+#pragma unroll
+    for (int q = 0; q < 16; ++q, p += 4 * ld)
+      __hip_atomic_store(p + r, Bs[(cb + 4 * q) * PB + r], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
   publish_wait();  // every wave's X_i stores complete ...
   __syncthreads();
   if (threadIdx.x == 0)  // ... before step t + 1 may read them
