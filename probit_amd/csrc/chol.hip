@@ -12,12 +12,11 @@
 //          product with the stored inverse of L_kk;
 //   O    : after the super-step's last column, the outer update of every
 //          lower tile right of it with rank 64 G (FP64 / FP32 operands, or
-//          BF16 operands with FP32 accumulation).
+//          BF16 operands with FP32 accumulation); part of it may run in the
+//          next super-step's launch (k_superstep).
 // A diagonal block is factored by one workgroup in FP64 together with its
-// inverse (blocked by 16: each 16-column panel by one wave, one row per
-// lane; the trailing updates and the inverse's off-diagonal blocks on FP64
-// MFMA); the FP64 inverses (DINV) serve the panel products and the
-// triangular solves.
+// inverse (four columns at a time, the updates on FP64 MFMA); the FP64
+// inverses (DINV) serve the panel products and the triangular solves.
 #include <math.h>
 #include <stdlib.h>
 

@@ -7,10 +7,12 @@
 // (probit/approximators.py:177) and the explicit inverses of
 // probit/implicit/VB.py:26-27.
 //
-// Both are blocked by 64: one launch per block step.  The diagonal block is
-// applied as a product with its precomputed FP64 inverse (DINV), so no step
-// has a serial substitution chain; the off-diagonal update is a GEMV / MFMA
-// GEMM.  Vectors are FP64 throughout; TRSM runs in the factor's storage type.
+// Both are blocked by 64 and run as one wavefront launch (k_trsv_seg,
+// k_trsm_rows), or without a ticket counter as a launch per block step.  The
+// diagonal block is applied as a product with its precomputed FP64 inverse
+// (DINV), so no step has a serial substitution chain; the off-diagonal update
+// is a GEMV / MFMA GEMM.  Vectors are FP64 throughout; TRSM runs in the
+// factor's storage type.
 #include <stdlib.h>
 
 #include <algorithm>
