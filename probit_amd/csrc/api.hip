@@ -839,11 +839,12 @@ int64_t pgp_grad_workspace_size(int64_t N, int32_t D) {
 // device descriptor), so one captured graph serves every later iteration with
 // the same key, in this fit and in later fits on the same workspace
 // (optimisation loops, sweeps).  Replays are valid as they are: every
-// wavefront launch of an iteration has its own epoch, a member's progress
-// word is written by at least two of them per iteration (the two triangular
-// sweeps; a factor whose column launches wait on it has two or more of
-// those), so no replay finds its own epoch left from the previous one, and
-// the ticket counters reset themselves at each launch's end.  Capturing and
+// wavefront launch of an iteration has its own epoch, the words that a
+// triangular sweep publishes are all written again by the other sweep (a
+// member's progress word by every column launch that waits on it, two or more
+// a factor), so no replay finds its own epoch left from the previous one, the
+// super-step launches clear their tile flags, and the ticket counters reset
+// themselves at each launch's end.  Capturing and
 // instantiating costs more than launching once, so a key is captured only
 // when it recurs in a later fit; a one-off fit runs its launches directly.
 // Off with PGP_FIT_NO_GRAPH in the options' flags (or PGP_GRAPH=0), and
