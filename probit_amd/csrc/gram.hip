@@ -160,8 +160,8 @@ void launch_gram_self(const Batch& b, hipStream_t s) {
 // the symmetric product K x, x = vector slot rs, in the slots k_symv_reduce
 // adds (row sums of tile (I, J) in part[I][J], column sums in part[J][I];
 // see k_symv_tiles), so the Newton step's K r costs no second read of K.
-// Bound by memory: N = 16384 into FP32 500 -> 366 us (4.4 TB/s), every load of
-// K before the first store.
+// Bound by memory: N = 16384 into FP32 500 -> 366 us with every load of K
+// before the first store, 294 (5.5 TB/s) with column_sums' swaps.
 template <typename T>
 __global__ __launch_bounds__(NTHREADS) void k_form_B(Prob* const* probs, Sched sc, int vb,
                                                      int rs) {
@@ -209,25 +209,13 @@ __global__ __launch_bounds__(NTHREADS) void k_form_B(Prob* const* probs, Sched s
   rpart[jg][il] = rsum;
   double* part = P.symv;
   if (ti != tj) {
-    // column sums of the wave's 16 columns by the transposing butterfly of
-    // k_symv_tiles: lane l ends with column jg * 16 + ((l >> 2) & 15)
+    // column sums of the wave's 16 columns: lane l ends with column jg * 16 +
+    // ((l >> 2) & 15)
     const double xi = x[i];
     double v[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) v[q] = k[q] * xi;
-#pragma unroll
-    for (int h = 8, bit = 32; h >= 1; h >>= 1, bit >>= 1) {
-      const bool up = (il & bit) != 0;
-#pragma unroll
-      for (int q = 0; q < h; ++q) {
-        const double give = up ? v[q] : v[q + h];
-        const double keep = up ? v[q + h] : v[q];
-        v[q] = keep + __shfl_xor(give, bit);
-      }
-    }
-    double cs = v[0];
-    cs += __shfl_xor(cs, 2);
-    cs += __shfl_xor(cs, 1);
+    const double cs = column_sums(v);
     if ((il & 3) == 0) part[((size_t)tj * Tn + ti) * TILE + jg * 16 + ((il >> 2) & 15)] = cs;
   }
   __syncthreads();
@@ -287,22 +275,8 @@ __global__ __launch_bounds__(NTHREADS) void k_cross_prep(Prob* const* probs, Sch
     S[(size_t)i + (size_t)j * P.Np] = (T)(si * v);
     pv[c] = v * a;
   }
-  // sums of v * a over the 64 rows of the tile for the wave's 16 columns, by
-  // a transposing butterfly (fixed order): lane l ends with column
-  // jg * 16 + ((l >> 2) & 15)
-#pragma unroll
-  for (int h = 8, bit = 32; h >= 1; h >>= 1, bit >>= 1) {
-    const bool up = (il & bit) != 0;
-#pragma unroll
-    for (int q = 0; q < h; ++q) {
-      const double give = up ? pv[q] : pv[q + h];
-      const double keep = up ? pv[q + h] : pv[q];
-      pv[q] = keep + __shfl_xor(give, bit);
-    }
-  }
-  double pa = pv[0];
-  pa += __shfl_xor(pa, 2);
-  pa += __shfl_xor(pa, 1);
+  // sums of v * a over the 64 rows of the tile for the wave's 16 columns
+  const double pa = column_sums(pv);
   if ((il & 3) == 0) part[jg][(il >> 2) & 15] = pa;
   __syncthreads();
   if (threadIdx.x < TILE) {

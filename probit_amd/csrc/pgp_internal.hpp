@@ -214,6 +214,43 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T* scalar(con
   return (const __attribute__((address_space(4))) T*)(uintptr_t)p;
 }
 
+// Transposing butterfly of a wave's 16 values per lane: the sums over the lanes
+// of v[q] end in the lanes l with (l >> 2) & 15 = q (each sum in a fixed
+// order).  At lane bits 32 and 16 a pair of registers is exchanged by a half-
+// (quarter-) wave swap, at bits 8 to 1 through LDS shuffles: with shuffles for
+// all of them the LDS pipe, not memory, bounded the passes over K (N = 16384:
+// k_symv_tiles 323 -> 224 us, 4.8 TB/s; k_form_B 363 -> 294).
+__device__ __forceinline__ double fold_swap(double a, double b, bool half) {
+  const unsigned al = (unsigned)__double2loint(a), ah = (unsigned)__double2hiint(a);
+  const unsigned bl = (unsigned)__double2loint(b), bh = (unsigned)__double2hiint(b);
+  const auto lo = half ? __builtin_amdgcn_permlane32_swap(al, bl, false, false)
+                       : __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+  const auto hi = half ? __builtin_amdgcn_permlane32_swap(ah, bh, false, false)
+                       : __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double column_sums(double (&v)[16]) {
+#pragma unroll
+  for (int q = 0; q < 8; ++q) v[q] = fold_swap(v[q], v[q + 8], true);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = fold_swap(v[q], v[q + 4], false);
+  const int l = threadIdx.x & 63;
+#pragma unroll
+  for (int h = 2, bit = 8; h >= 1; h >>= 1, bit >>= 1) {
+    const bool up = (l & bit) != 0;
+#pragma unroll
+    for (int q = 0; q < h; ++q) {
+      const double give = up ? v[q] : v[q + h];
+      const double keep = up ? v[q + h] : v[q];
+      v[q] = keep + __shfl_xor(give, bit);
+    }
+  }
+  double s = v[0];
+  s += __shfl_xor(s, 2);
+  s += __shfl_xor(s, 1);
+  return s;
+}
+
 // Values handed between workgroups of one launch travel only through
 // relaxed agent-scope accesses: the stores write through the XCD's L2 and
 // the loads read past it, so a publication needs no L2 write-back or

@@ -113,25 +113,12 @@ __global__ __launch_bounds__(NTHREADS) void k_symv_tiles(Prob* const* probs, Sch
   rpart[w][r] = rs;
   const auto part = gbl(uniform(P.symv));
   if (ti != tj) {
-    // column sums K_IJ^T x_I of the wave's 16 columns: a transposing
-    // butterfly halves the values per lane at each of lane bits 5..2, then
-    // bits 1, 0 finish the sum; lane l ends with column q = (l >> 2) & 15
+    // column sums K_IJ^T x_I of the wave's 16 columns: lane l ends with column
+    // q = (l >> 2) & 15
     double v[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) v[q] = k[q] * xi;
-#pragma unroll
-    for (int h = 8, bit = 32; h >= 1; h >>= 1, bit >>= 1) {
-      const bool up = (r & bit) != 0;
-#pragma unroll
-      for (int q = 0; q < h; ++q) {
-        const double give = up ? v[q] : v[q + h];
-        const double keep = up ? v[q + h] : v[q];
-        v[q] = keep + __shfl_xor(give, bit);
-      }
-    }
-    double cs = v[0];
-    cs += __shfl_xor(cs, 2);
-    cs += __shfl_xor(cs, 1);
+    const double cs = column_sums(v);
     if ((r & 3) == 0)
       part[((size_t)tj * nb + ti) * TILE + w + 4 * ((r >> 2) & 15)] = cs;
   }
