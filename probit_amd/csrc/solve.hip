@@ -20,6 +20,7 @@
 
 #include "mfma.hpp"
 #include "pgp_internal.hpp"
+#include "solve_schedule.hpp"
 
 namespace pgp {
 
@@ -729,7 +730,7 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 2 : 3) void k_trsm_rows(
 // k_trsm_rows with both L_ji and DINV_i transposed on their way into LDS
 // (rows of the stored tile are the k index, read coalesced along k).
 template <typename T>
-__global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sched rows, int nct,
+__global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, RowSched rows, int nct,
                                                           int ct0, uint32_t* ticket,
                                                           uint32_t epoch) {
   constexpr int PA = TILE + 1;  // A operand, written row by row
@@ -740,11 +741,11 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
   typedef typename Acc<T>::type acc_t;
   const int tk = take_ticket(ticket, &s_val);
   if ((unsigned)tk >= gridDim.x) {  // counter not zero at launch: no block to take
-    flag_members_stalled(probs, (rows.pre[1] - rows.pre[0]) / nct);  // step 0: every member
+    flag_members_stalled(probs, (rows.pre[1] - rows.pre[0]) / nct);  // of the first step
     return;
   }
   int local;
-  const int t = sched_member(rows, uniform(tk), local);
+  const int t = rows.row0 + sched_member(rows, uniform(tk), local);
   const int m = uniform(local / nct), lct = local - m * nct;
   const Prob& P = *probs[m];
   const int nb = uniform(P.Np) / TILE, ct = ct0 + lct;
@@ -796,7 +797,8 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
   }
   acc_t acc[2][2];
   zero_acc<T>(acc);
-  int done = 0, ready = 0;
+  int done = 0, ready = min(rows.row0, t);  // steps known to be published
+  if (ready > 0) fetch_x(0);
   while (done < t) {
     if (done >= ready) {
       __syncthreads();  // everyone has read the previous s_val
@@ -865,22 +867,13 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Sc
 }
 
 // S <- L^-T S for every member's Mp right-hand sides (Mp <= maxMp): one
-// wavefront launch per group of PROGRESS_CT column tiles.
+// wavefront launch per group of PROGRESS_CT column tiles and ROWS_MAX block
+// rows.
 void launch_trsm_t(const Batch& bt, int prec, int maxMp, hipStream_t s) {
   const int nb = bt.maxNp / TILE;
   const int mt = maxMp / TILE;
   for (int ct0 = 0; ct0 < mt; ct0 += PROGRESS_CT) {
     const int nct = std::min(PROGRESS_CT, mt - ct0);
-    Sched rows;
-    rows.count = nb;
-    int tot = 0;
-    for (int t = 0; t < nb; ++t) {
-      rows.pre[t] = tot;
-      for (int m = 0; m < bt.count; ++m)
-        if (bt.np(m) / TILE > t) tot += nct;
-    }
-    rows.pre[nb] = tot;
-    if (tot == 0) return;
     const bool on = timer_on(TC_TRSM);
     double fl = 0.0;
     if (on) {
@@ -890,13 +883,18 @@ void launch_trsm_t(const Batch& bt, int prec, int maxMp, hipStream_t s) {
       }
       timer_begin(TC_TRSM, s);
     }
-    const uint32_t ep = next_epoch();
-    if (prec == PGP_PREC_FP64)
-      hipLaunchKernelGGL(k_trsm_rows_t<double>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                         nct, ct0, bt.ticket, ep);
-    else
-      hipLaunchKernelGGL(k_trsm_rows_t<float>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                         nct, ct0, bt.ticket, ep);
+    for (int row0 = 0; row0 < nb; row0 += ROWS_MAX) {
+      RowSched rows;
+      const int tot = fill_rows(rows, row0, nb, bt.count, [&](int m) { return bt.np(m) / TILE; },
+                                nct);
+      const uint32_t ep = next_epoch();
+      if (prec == PGP_PREC_FP64)
+        hipLaunchKernelGGL(k_trsm_rows_t<double>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs,
+                           rows, nct, ct0, bt.ticket, ep);
+      else
+        hipLaunchKernelGGL(k_trsm_rows_t<float>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
+                           nct, ct0, bt.ticket, ep);
+    }
     if (on) timer_end(TC_TRSM, s, fl, 0.0);
   }
 }
