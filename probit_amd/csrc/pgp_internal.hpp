@@ -144,8 +144,7 @@ struct Sched {
 
 // Member of workgroup `bid` (the largest m with pre[m] <= bid) and the
 // workgroup's index within that member.  Uniform: scalar loads only.
-template <class S>
-__device__ __forceinline__ int sched_member(const S& sc, int bid, int& local) {
+__device__ __forceinline__ int sched_member(const Sched& sc, int bid, int& local) {
   int lo = 0, hi = sc.count;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;

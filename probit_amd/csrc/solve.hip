@@ -447,7 +447,7 @@ int launch_trsv_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const d
 }
 
 // ---- TRSM: S <- L^-1 S, S is Np x Mp (ld lds) ----
-// With a ticket counter and up to MAXB block rows a solve is one wavefront
+// With a ticket counter and up to ROWS_MAX block rows a solve is one wavefront
 // launch (k_trsm_rows, below), in FP32 with the roundings of the schedule its
 // width would take without: a launch per block row (up to TRSM_WIDE column
 // tiles) or per super-step of G block rows, which subtract each block row's
@@ -545,6 +545,68 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged_raw(const T* L, int64_
   trsm_step<T>(L, ld, dinv, k, S, lds, blockIdx.x, blockIdx.y);
 }
 
+// Workgroup tk of a wide solve's launch: block row (in sweep order), member,
+// column tile of the launch.
+__device__ __forceinline__ void solve_unit(const SolveSched& ss, int tk, int& row, int& m,
+                                           int& ct) {
+  auto find = [](const int32_t* pre, int n, int v) {  // the last i < n with pre[i] <= v
+    int lo = 0, hi = n;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (pre[mid] <= v)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    return lo;
+  };
+  const int r = find(ss.rows, ss.count, tk), local = tk - ss.rows[r];
+  row = ss.row0 + r;
+  if (ss.nct > 0) {
+    m = uniform(local / ss.nct);
+    ct = local - m * ss.nct;
+  } else {
+    m = find(ss.tiles, ss.members, local);
+    ct = local - ss.tiles[m];
+  }
+}
+
+// The launches of a wide solve (at most maxMp / 64 column tiles a member):
+// per PROGRESS_CT column tiles, per schedule's members and block rows, each
+// member with its own column tiles (256 requests of 700 to 1024 points, one
+// with 5000 test points and the others with 64, a step of a stream: 14.3 ms in
+// FP32 and 11.9 in FP64 with the widest member's tiles listed for every member,
+// now 8.1 and 9.0).
+// go(dprobs, schedule, first column tile, workgroups, epoch).
+template <class Go>
+static void solve_launches(const Batch& bt, int maxMp, hipStream_t s, Go go) {
+  auto mt_of = [&](int m) { return bt.hm ? (bt.hm[m] + TILE - 1) / TILE : maxMp / TILE; };
+  const bool on = timer_on(TC_TRSM);
+  for (int ct0 = 0; ct0 < maxMp / TILE; ct0 += PROGRESS_CT) {
+    for (int m0 = 0, n = 0; m0 < bt.count; m0 += n) {
+      auto nct_of = [&](int m) {
+        return std::min(PROGRESS_CT, std::max(0, mt_of(m0 + m) - ct0));
+      };
+      auto nb_of = [&](int m) { return bt.np(m0 + m) / TILE; };
+      SolveSched ss;
+      n = fill_tiles(ss, bt.count - m0, nct_of);
+      double fl = 0.0;
+      if (on) {
+        for (int m = 0; m < n; ++m) {
+          const double np = bt.np(m0 + m);
+          fl += np * np * TILE * nct_of(m);
+        }
+        timer_begin(TC_TRSM, s);
+      }
+      for (int row0 = 0; row0 < nb_of(0); row0 += ROWS_MAX) {
+        const int tot = fill_rows(ss, row0, nb_of);
+        if (tot > 0) go(bt.dprobs + m0, ss, ct0, tot, next_epoch());
+      }
+      if (on) timer_end(TC_TRSM, s, fl, 0.0);
+    }
+  }
+}
+
 // Wavefront TRSM for the column tiles [ct0, ct0 + nct) (nct <= PROGRESS_CT),
 // all members in one launch: one workgroup per (block row i, member, column
 // tile ct), numbered row-major so that the wave front moves through every
@@ -563,17 +625,21 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_lagged_raw(const T* L, int64_
 // ahead; 1110 (41) with DINV's zeros left out and X_i stored by whole columns
 // (256 test points, FP32, a stream of fits: 68.5 -> 65.8 ms).  N = 1537, M = 501: 590 -> 269 us.  Transposed, FP32 at N = 8192, M =
 // 4096: 20.3 ms in 16 launches of 4 column tiles, 2.8 ms (98 TFLOP/s) in one.
-constexpr int WAVE_NCT = 4;
-
 //
 // GRP: the sum is taken off S_i, in its type, after every 1 << lg blocks but
 // the last whole group before i's own: the roundings of the schedules of one
 // launch per block row (lg = 0) or super-step of TRSM_G (lg = 2), which FP32
 // solves of more than WAVE_NCT column tiles follow without a ticket counter.
+// lg goes by the member's own column tiles (up to WAVE_NCT: no group is ever
+// whole), so that its results do not depend on the rest of the batch.
+constexpr int WAVE_NCT = 4;
+// Right-hand sides of at least this many column tiles take the super-step
+// schedule.
+constexpr int TRSM_WIDE = 16;
+
 template <typename T, bool GRP>
-__global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 2 : 3) void k_trsm_rows(Prob* const* probs, Sched rows, int nct,
-                                                        int ct0, int lg, uint32_t* ticket,
-                                                        uint32_t epoch) {
+__global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 2 : 3) void k_trsm_rows(
+    Prob* const* probs, SolveSched ss, int ct0, uint32_t* ticket, uint32_t epoch) {
   constexpr int PP = KP<T>::value;  // A operand: conflict-free MFMA reads
   constexpr int PB = TILE + 1;       // B operand: written transposed, conflict-free stores
   __shared__ T As[TILE * PP];
@@ -582,14 +648,16 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 2 : 3) void k_trsm_rows(
   typedef typename Acc<T>::type acc_t;
   const int tk = take_ticket(ticket, &s_val);
   if ((unsigned)tk >= gridDim.x) {  // counter not zero at launch: no block to take
-    flag_members_stalled(probs, (rows.pre[1] - rows.pre[0]) / nct);  // row 0: every member
+    flag_members_stalled(probs, ss.members);
     return;
   }
-  int local;
-  const int i = sched_member(rows, uniform(tk), local);
-  const int m = uniform(local / nct), lct = local - m * nct, ct = ct0 + lct;
+  int i, m, lct;
+  solve_unit(ss, uniform(tk), i, m, lct);
+  const int ct = ct0 + lct;
   const Prob& P = *probs[m];
-  if (ct >= P.Mp / TILE || i >= P.Np / TILE) return;
+  const int mt = uniform(P.Mp) / TILE;
+  if (ct >= mt || i >= P.Np / TILE) return;
+  const int lg = mt <= WAVE_NCT ? 30 : mt < TRSM_WIDE ? 0 : 2;
   uint64_t* prog = P.progress_ct + lct;
   const auto L = gbl(uniform((const T*)P.L));
   const auto S = gbl(uniform((T*)P.S));
@@ -730,7 +798,7 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 2 : 3) void k_trsm_rows(
 // k_trsm_rows with both L_ji and DINV_i transposed on their way into LDS
 // (rows of the stored tile are the k index, read coalesced along k).
 template <typename T>
-__global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, RowSched rows, int nct,
+__global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, SolveSched ss,
                                                           int ct0, uint32_t* ticket,
                                                           uint32_t epoch) {
   constexpr int PA = TILE + 1;  // A operand, written row by row
@@ -741,12 +809,11 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Ro
   typedef typename Acc<T>::type acc_t;
   const int tk = take_ticket(ticket, &s_val);
   if ((unsigned)tk >= gridDim.x) {  // counter not zero at launch: no block to take
-    flag_members_stalled(probs, (rows.pre[1] - rows.pre[0]) / nct);  // of the first step
+    flag_members_stalled(probs, ss.members);
     return;
   }
-  int local;
-  const int t = rows.row0 + sched_member(rows, uniform(tk), local);
-  const int m = uniform(local / nct), lct = local - m * nct;
+  int t, m, lct;
+  solve_unit(ss, uniform(tk), t, m, lct);
   const Prob& P = *probs[m];
   const int nb = uniform(P.Np) / TILE, ct = ct0 + lct;
   if (ct >= P.Mp / TILE || t >= nb) return;
@@ -797,7 +864,7 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Ro
   }
   acc_t acc[2][2];
   zero_acc<T>(acc);
-  int done = 0, ready = min(rows.row0, t);  // steps known to be published
+  int done = 0, ready = min(ss.row0, t);  // steps known to be published
   if (ready > 0) fetch_x(0);
   while (done < t) {
     if (done >= ready) {
@@ -866,37 +933,17 @@ __global__ __launch_bounds__(NTHREADS) void k_trsm_rows_t(Prob* const* probs, Ro
                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// S <- L^-T S for every member's Mp right-hand sides (Mp <= maxMp): one
-// wavefront launch per group of PROGRESS_CT column tiles and ROWS_MAX block
-// rows.
+// S <- L^-T S for every member's Mp right-hand sides (Mp <= maxMp).
 void launch_trsm_t(const Batch& bt, int prec, int maxMp, hipStream_t s) {
-  const int nb = bt.maxNp / TILE;
-  const int mt = maxMp / TILE;
-  for (int ct0 = 0; ct0 < mt; ct0 += PROGRESS_CT) {
-    const int nct = std::min(PROGRESS_CT, mt - ct0);
-    const bool on = timer_on(TC_TRSM);
-    double fl = 0.0;
-    if (on) {
-      for (int m = 0; m < bt.count; ++m) {
-        const double np = bt.np(m);
-        fl += np * np * (double)nct * TILE;
-      }
-      timer_begin(TC_TRSM, s);
-    }
-    for (int row0 = 0; row0 < nb; row0 += ROWS_MAX) {
-      RowSched rows;
-      const int tot = fill_rows(rows, row0, nb, bt.count, [&](int m) { return bt.np(m) / TILE; },
-                                nct);
-      const uint32_t ep = next_epoch();
-      if (prec == PGP_PREC_FP64)
-        hipLaunchKernelGGL(k_trsm_rows_t<double>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs,
-                           rows, nct, ct0, bt.ticket, ep);
-      else
-        hipLaunchKernelGGL(k_trsm_rows_t<float>, dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs, rows,
-                           nct, ct0, bt.ticket, ep);
-    }
-    if (on) timer_end(TC_TRSM, s, fl, 0.0);
-  }
+  solve_launches(bt, maxMp, s, [&](Prob* const* dp, const SolveSched& ss, int ct0, int tot,
+                                   uint32_t ep) {
+    if (prec == PGP_PREC_FP64)
+      hipLaunchKernelGGL(k_trsm_rows_t<double>, dim3(tot), dim3(NTHREADS), 0, s, dp, ss, ct0,
+                         bt.ticket, ep);
+    else
+      hipLaunchKernelGGL(k_trsm_rows_t<float>, dim3(tot), dim3(NTHREADS), 0, s, dp, ss, ct0,
+                         bt.ticket, ep);
+  });
 }
 
 static bool wavefront_trsm() {
@@ -1088,50 +1135,19 @@ static void launch_trsm_lagged(const Batch& bt, int prec, int maxMp, hipStream_t
   }
 }
 
-// Right-hand sides of at least this many column tiles take the super-step
-// schedule.
-constexpr int TRSM_WIDE = 16;
-
 void launch_trsm(const Batch& bt, int prec, int maxMp, hipStream_t s) {
-  const int mt = maxMp / TILE;
-  if (bt.ticket && bt.maxNp / TILE <= MAXB && wavefront_trsm()) {
-    for (int ct0 = 0; ct0 < mt; ct0 += PROGRESS_CT) {
-      // row-major schedule: row i holds the members with more than i block
-      // rows (a prefix: members are sorted by size), nct workgroups each
-      const int nct = std::min(PROGRESS_CT, mt - ct0);
-      const int nb = bt.maxNp / TILE;
-      Sched rows;
-      rows.count = nb;
-      int tot = 0;
-      double fl = 0.0;
-      for (int i = 0; i < nb; ++i) {
-        rows.pre[i] = tot;
-        for (int m = 0; m < bt.count; ++m)
-          if (bt.np(m) / TILE > i) tot += nct;
-      }
-      rows.pre[nb] = tot;
-      if (tot == 0) return;
-      const bool on = timer_on(TC_TRSM);
-      if (on) {
-        for (int m = 0; m < bt.count; ++m) {
-          const double np = bt.np(m);
-          const int mm = bt.hm ? (bt.hm[m] + TILE - 1) / TILE : mt;
-          fl += np * np * TILE * std::max(0, std::min(nct, mm - ct0));
-        }
-        timer_begin(TC_TRSM, s);
-      }
-      const uint32_t ep = next_epoch();
+  if (bt.ticket && bt.maxNp / TILE <= ROWS_MAX && wavefront_trsm()) {
+    const bool narrow = maxMp / TILE <= WAVE_NCT;
+    solve_launches(bt, maxMp, s, [&](Prob* const* dp, const SolveSched& ss, int ct0, int tot,
+                                     uint32_t ep) {
+      const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(tot), dim3(NTHREADS), 0, s, dp, ss, ct0, bt.ticket, ep);
+      };
       if (prec == PGP_PREC_FP64)
-        hipLaunchKernelGGL((k_trsm_rows<double, false>), dim3(tot), dim3(NTHREADS), 0, s,
-                           bt.dprobs, rows, nct, ct0, 0, bt.ticket, ep);
-      else if (mt <= WAVE_NCT)
-        hipLaunchKernelGGL((k_trsm_rows<float, false>), dim3(tot), dim3(NTHREADS), 0, s,
-                           bt.dprobs, rows, nct, ct0, 0, bt.ticket, ep);
+        go(k_trsm_rows<double, false>);
       else
-        hipLaunchKernelGGL((k_trsm_rows<float, true>), dim3(tot), dim3(NTHREADS), 0, s, bt.dprobs,
-                           rows, nct, ct0, mt < TRSM_WIDE ? 0 : 2, bt.ticket, ep);
-      if (on) timer_end(TC_TRSM, s, fl, 0.0);
-    }
+        narrow ? go(k_trsm_rows<float, false>) : go(k_trsm_rows<float, true>);
+    });
     return;
   }
   if (maxMp / TILE < TRSM_WIDE) {

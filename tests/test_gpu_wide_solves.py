@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from oracle import gp_oracle as O
-from tests.helpers import make_prior, oracle_spec, rel_err
+from tests.helpers import make_prior, oracle_spec, rel_err, small_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +38,39 @@ def test_predict_beyond_one_launch_of_block_rows():
         m_ref[j], v_ref[j] = O.predict(spec, X[i], Xt[j], w_ref, np.full(n, noise ** -2.0))
     assert rel_err(mean.cpu().numpy(), m_ref) < 1e-5
     assert rel_err(v.cpu().numpy(), v_ref) < 1e-5
+
+
+# requests with few and many test points in one serving step (1, 5, 18 and 141
+# column tiles: each of FP32's groupings, two launches of column tiles): each
+# as when it is served alone, bit for bit, and as the oracle's
+@pytest.mark.parametrize("mode,tol", [("fp64", 1e-9), ("fp32", 1e-5), ("bf16", None)])
+def test_uneven_test_points_in_one_serving_step(mode, tol):
+    from probit_amd.serving import ServingEngine
+    reqs = []
+    for k, (N, M) in enumerate([(700, 40), (641, 300), (650, 1100), (704, 40), (600, 9000)]):
+        X, y, theta, lp, spec = small_problem(60 + k, N, 2, "gaussian")
+        reqs.append((X, y, theta, lp, spec, np.random.default_rng(70 + k).normal(size=(M, 2))))
+
+    def run(idx):
+        eng = ServingEngine(precision=mode, capacity=8, hbm_budget_bytes=1 << 33)
+        for i in idx:
+            X, y, theta, lp, _, Xt = reqs[i]
+            assert eng.submit(i, X, y, "EQ", theta[0], theta[1], "gaussian", lp[0], None, Xt)
+        out = {}
+        while eng.in_flight:
+            for c in eng.step():
+                out[c.tag] = c
+        eng.close()
+        return out
+
+    mix = run(range(len(reqs)))
+    for i, (X, y, theta, lp, spec, Xt) in enumerate(reqs):
+        alone = run([i])[i]
+        for k in ("mean", "var"):
+            assert np.array_equal(getattr(alone, k).cpu().numpy(),
+                                  getattr(mix[i], k).cpu().numpy()), (i, k)
+        if tol is not None:
+            w_ref = np.linalg.solve(O.gram(spec, X) + lp[0] ** 2 * np.eye(len(X)), y)
+            m_ref, v_ref = O.predict(spec, X, Xt, w_ref, np.full(len(X), lp[0] ** -2.0))
+            assert rel_err(mix[i].mean.cpu().numpy(), m_ref) < tol
+            assert rel_err(mix[i].var.cpu().numpy(), v_ref) < tol
