@@ -181,6 +181,20 @@ static GradLayout grad_layout(int64_t Np, int prec) {
 // device-side descriptor and pointer-array writes (kernel arguments carry the
 // host values, so no host buffer has to outlive the call)
 // ---------------------------------------------------------------------------
+// The words that the launches on a state hand values over by (and its status
+// and reductions), to zero with a new descriptor: a workspace is the caller's
+// memory, whose old contents could pass for flags, progress or published
+// values of a launch.  One workgroup.
+__device__ __forceinline__ void clear_sync(const Prob& v) {
+  if (threadIdx.x < 4) v.info[threadIdx.x] = 0;
+  if (threadIdx.x < NRED) v.red[threadIdx.x] = 0.0;
+  if (threadIdx.x == 0) v.progress[0] = 0;
+  for (int i = threadIdx.x; i < PROGRESS_CT; i += blockDim.x) v.progress_ct[i] = 0;
+  for (int i = threadIdx.x; i < csync_words(v.Np); i += blockDim.x) v.csync[i] = 0;
+  ulonglong2* x = reinterpret_cast<ulonglong2*>(v.xpub);
+  for (int i = threadIdx.x; i < v.Np; i += blockDim.x) x[i] = ulonglong2{0, 0};
+}
+
 // reset: of a new state, with the pointer array of the problem alone; 2: and
 // its weight z = 0, latent f = K 0.
 __global__ void k_write_prob(Prob* dst, Prob val, int reset) {
@@ -195,14 +209,8 @@ __global__ void k_write_prob(Prob* dst, Prob val, int reset) {
         vslot(val, V_Z)[i] = 0.0;
         vslot(val, V_F)[i] = 0.0;
       }
-    if (threadIdx.x < 4) val.info[threadIdx.x] = 0;
-    if (threadIdx.x < NRED) val.red[threadIdx.x] = 0.0;
-    // progress word and ticket counter of the header
-    if (threadIdx.x < 2) reinterpret_cast<uint64_t*>((char*)dst + OFF_PROGRESS)[threadIdx.x] = 0;
-    for (int i = threadIdx.x; i < PROGRESS_CT; i += blockDim.x)
-      reinterpret_cast<uint64_t*>((char*)dst + OFF_PROGRESS_CT)[i] = 0;
-    if (val.csync)
-      for (int64_t w = threadIdx.x; w < csync_words(val.Np); w += blockDim.x) val.csync[w] = 0;
+    if (threadIdx.x == 0) *(uint64_t*)((char*)dst + OFF_TICKET) = 0;
+    clear_sync(val);
   }
 }
 
@@ -227,15 +235,7 @@ __global__ void k_scatter_probs(Prob* const* dst, const Prob* src, int n, int re
   uint64_t* d = reinterpret_cast<uint64_t*>(dst[i]);
   const int nw = (int)(sizeof(Prob) / 8);
   for (int w = threadIdx.x; w < nw; w += blockDim.x) d[w] = sv[w];
-  if (reset) {
-    const Prob& v = src[i];
-    if (threadIdx.x < 4) v.info[threadIdx.x] = 0;
-    if (threadIdx.x < NRED) v.red[threadIdx.x] = 0.0;
-    if (threadIdx.x == 0) v.progress[0] = 0;
-    for (int w = threadIdx.x; w < PROGRESS_CT; w += blockDim.x) v.progress_ct[w] = 0;
-    if (v.csync)
-      for (int64_t w = threadIdx.x; w < csync_words(v.Np); w += blockDim.x) v.csync[w] = 0;
-  }
+  if (reset) clear_sync(src[i]);
 }
 
 static void write_prob(char* ws, const Prob& p, int reset, hipStream_t s) {

@@ -74,3 +74,23 @@ def test_uneven_test_points_in_one_serving_step(mode, tol):
             m_ref, v_ref = O.predict(spec, X, Xt, w_ref, np.full(len(X), lp[0] ** -2.0))
             assert rel_err(mix[i].mean.cpu().numpy(), m_ref) < tol
             assert rel_err(mix[i].var.cpu().numpy(), v_ref) < tol
+
+
+# a state formed in memory with any contents starts with the triangular
+# solves' published values (the last 16 bytes a padded row of an FP64
+# workspace) cleared
+@pytest.mark.parametrize("N", [1, 64, 130, 1000])
+def test_published_values_are_cleared_with_a_new_state(N):
+    import torch
+
+    import probit_amd as P
+    X, y, theta, lp, _ = small_problem(N, max(N, 4), 2, "gaussian")
+    X, y = X[:N], y[:N]
+    gp = P.LaplaceGP(data=(X, y), prior=make_prior("EQ"),
+                     log_likelihood=P.log_gaussian_likelihood)
+    ws = gp._workspace()
+    ws.fill_(0xA5)
+    w = torch.zeros(N, dtype=torch.float64)
+    gp.predict(X, (theta, lp), w, torch.full((N,), lp[0] ** -2.0, dtype=torch.float64))
+    Np = (N + 63) // 64 * 64
+    assert not bool(ws[-16 * Np:].any())
