@@ -163,22 +163,24 @@ __device__ __forceinline__ void factor_block_blocked(double (*A)[TILE + 1], doub
 #pragma unroll
       for (int c = s + 1; c < 4; ++c)
         if (s > 0) R[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(fp[c][r], lp[r], R[c], 0, 0, 0);
-      // (products of column entries are formed beside the reciprocals)
+      // (the quotients l first, never a product of two entries, whose range is
+      // the square of theirs)
       const double r0 = rcp_f64(d[0]);
-      d[1] = fma(-(s10 * s10), r0, d[1]);
-      d[2] = fma(-(s20 * s20), r0, d[2]);
-      d[3] = fma(-(s30 * s30), r0, d[3]);
-      s21 = fma(-(s20 * s10), r0, s21);
-      s31 = fma(-(s30 * s10), r0, s31);
-      s32 = fma(-(s30 * s20), r0, s32);
-      const double r1 = rcp_f64(d[1]);
-      d[2] = fma(-(s21 * s21), r1, d[2]);
-      d[3] = fma(-(s31 * s31), r1, d[3]);
-      s32 = fma(-(s31 * s21), r1, s32);
-      const double r2 = rcp_f64(d[2]);
-      d[3] = fma(-(s32 * s32), r2, d[3]);
       const double l10 = s10 * r0, l20 = s20 * r0, l30 = s30 * r0;
-      const double l21 = s21 * r1, l31 = s31 * r1, l32 = s32 * r2;
+      d[1] = fma(-l10, s10, d[1]);
+      d[2] = fma(-l20, s20, d[2]);
+      d[3] = fma(-l30, s30, d[3]);
+      s21 = fma(-l20, s10, s21);
+      s31 = fma(-l30, s10, s31);
+      s32 = fma(-l30, s20, s32);
+      const double r1 = rcp_f64(d[1]);
+      const double l21 = s21 * r1, l31 = s31 * r1;
+      d[2] = fma(-l21, s21, d[2]);
+      d[3] = fma(-l31, s31, d[3]);
+      s32 = fma(-l31, s21, s32);
+      const double r2 = rcp_f64(d[2]);
+      const double l32 = s32 * r2;
+      d[3] = fma(-l32, s32, d[3]);
       // X = (the four columns) L4^-T = L D, as X^T = L4^-1 (columns)^T: one
       // 4x4x4 MFMA for the four blocks of four rows, whose result is in the
       // operand layout again.  Lane l brings L4^-1(l & 3, l >> 4).
