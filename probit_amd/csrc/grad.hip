@@ -175,29 +175,62 @@ void launch_sym_from_inv(const Batch& b, int prec, int use_scale, hipStream_t s)
     hipLaunchKernelGGL(k_sym_from_inv<float>, g, dim3(NTHREADS), 0, s, b.dprobs, use_scale);
 }
 
-// Sigma_ii = K_ii - (K C K)_ii where W_i < 0 (S_i = 0, so K C K says nothing
-// about W_i): one workgroup per such row, from the lower triangle of C.  The
-// other rows come from (K C)_ii = W_i Sigma_ii (gemv_epilogue's mode 4).
-__global__ __launch_bounds__(NTHREADS) void k_sigma_negative(Prob* const* probs) {
-  const Prob& P = *probs[blockIdx.y];
-  const int i = blockIdx.x;
-  if (i >= P.N || !(vslot(P, V_W)[i] < 0.0)) return;
-  const double* k = P.K + (size_t)i * P.Np;
-  double q = 0.0;
-  for (int c = threadIdx.x >> 6; c < P.N; c += 4) {
-    const double* col = P.C + (size_t)c * P.Np;
-    double a = 0.0;
-    for (int r = c + (threadIdx.x & 63); r < P.N; r += 64) a += (r == c ? 1.0 : 2.0) * col[r] * k[r];
-    q += a * k[c];
-  }
-  __shared__ double red[NTHREADS];
-  red[threadIdx.x] = q;
+// Where W_i is not positive, (K C)_ii = W_i Sigma_ii says nothing about
+// Sigma_ii: there it is K_ii - ||V_:,i||^2, V = L^-1 S K.  A workgroup per row
+// block I and column block J of V, the longest sums first: if one of J's
+// columns has such a W, their norms over I's rows take the place of their row
+// sums of K o C in slot I of J (k_symv_reduce then adds squares).  N^3 flops at
+// worst, as the solve it stands for; none of it where all W > 0.  A gradient at
+// N = 4096 takes 1.8 ms, 2.0 with 40 such W and 3.7 with 3686; with the
+// quadratic form of C by one workgroup per such W 10.2 and 29.3.
+__global__ __launch_bounds__(NTHREADS) void k_sigma_squares(Prob* const* probs) {
+  const Prob& P = *probs[blockIdx.z];
+  const int nb = uniform(P.Np) / TILE, J = blockIdx.y;
+  const int I = nb - 1 - (int)blockIdx.x;
+  if (I < 0 || J >= nb) return;
+  const unsigned m = threadIdx.x & 63;
+  const int kb = uniform((int)(threadIdx.x >> 6));
+  const int64_t ld = uniform(P.Np);
+  const auto W = gbl(vslot(P, V_W)) + J * TILE;
+  const bool mine = J * TILE + (int)m < P.N && !(W[m] > 0.0);
+  const uint64_t which = __builtin_amdgcn_ballot_w64(mine);  // the same in every wave
+  if (which == 0) return;
+  const auto X = gbl(uniform((const double*)P.S));  // L^-1
+  const auto K = gbl(uniform(P.K));
+  const auto S = gbl(vslot(P, V_S));
+  __shared__ GemmLds<double> lds;
+  doublex4 acc[2][2];
+  zero_acc<double>(acc);
+  gemm_tiles<double, false>(
+      0, I + 1,
+      [&](int k, double (&v)[16]) {
+        auto p = X + ((int64_t)I * TILE + ((int64_t)k * TILE + kb) * ld);
+#pragma unroll
+        for (int q = 0; q < 16; ++q, p += 4 * ld) v[q] = p[m];
+      },
+      [&](int k, double (&v)[16]) {
+        const double sk = S[(int64_t)k * TILE + m];
+        auto p = K + ((int64_t)k * TILE + ((int64_t)J * TILE + kb) * ld);
+#pragma unroll
+        for (int q = 0; q < 16; ++q, p += 4 * ld) v[q] = sk * p[m];
+      },
+      lds, acc);
+  constexpr int PB = GemmLds<double>::PB;
+#pragma unroll
+  for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+    for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double v = acc[bm][bn][r];
+        lds.b[acc_row<double>(bm, r) * PB + acc_col(bn)] = v * v;
+      }
   __syncthreads();
-  for (int st = NTHREADS / 2; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-    __syncthreads();
+  if (kb == 0 && mine) {
+    double a = 0.0;
+    for (int r = 0; r < TILE; ++r) a += lds.b[r * PB + m];
+    P.symv[((size_t)J * nb + I) * TILE + m] = a;
   }
-  if (threadIdx.x == 0) vslot(P, V_X1)[i] = k[i] - red[0];
 }
 
 // Right-hand side S_i K_ij of V = L^-1 S K (factors stored in FP32).
@@ -226,19 +259,23 @@ __global__ __launch_bounds__(NTHREADS) void k_sigma_norms(Prob* const* probs) {
 }
 
 // diag Sigma into X1, Sigma = (K^-1 + W)^-1 = K - K C K.  FP64 factors: from C
-// and K alone.  Sigma W = K C, so Sigma_ii = (sum_j K_ij C_ij) / W_i, two N^2
-// passes where the column norms of L^-1 S K take a solve with N right-hand
-// sides (N^3 flops: 3.2 ms at N = 4096, now 0.05).  The terms of the sum
-// carry S_i, so its relative error grows only as max(S) / S_i where W_i is
-// small, and there the third derivative it is multiplied with goes with W_i.
+// and K.  Sigma W = K C, so Sigma_ii = (sum_j K_ij C_ij) / W_i, two N^2 passes
+// where the column norms of L^-1 S K take a solve with N right-hand sides (N^3
+// flops: 3.2 ms at N = 4096, now 0.05), except where W_i <= 0
+// (k_sigma_squares).  The sum cancels as K W grows, like the norms': an entry's
+// error is up to nine times theirs (N = 400, Gaussian noise 1e-3: 9e-8 and 9e-9
+// relative, both with the condition of B), but the gradient, which adds the
+// entries up, is as accurate (noise 1e-3: 6.6e-10 and 5.7e-10; 0.03: 3.6e-13
+// and 2.4e-13; probit noise 0.1, N = 400: 2.9e-12 and 3.3e-12).
 // Factors stored in FP32 keep the column norms: C then carries the factor's
 // FP32 error, which the norms damp (noise gradient of a Gaussian fit at N =
 // 2000: 7e-5 relative error from the norms, 1e-3 from C).
 void launch_sigma_diag(const Batch& b, int prec, hipStream_t s) {
   if (prec == PGP_PREC_FP64) {
+    const int nb = b.maxNp / TILE;
     launch_hadamard_tiles(b, s);
+    hipLaunchKernelGGL(k_sigma_squares, dim3(nb, nb, b.count), dim3(NTHREADS), 0, s, b.dprobs);
     launch_symv_reduce(b, V_X1, V_X1, 4, s);
-    hipLaunchKernelGGL(k_sigma_negative, dim3(b.maxNp, b.count), dim3(NTHREADS), 0, s, b.dprobs);
     return;
   }
   const int64_t n2 = (int64_t)b.maxNp * b.maxNp;

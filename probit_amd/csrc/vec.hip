@@ -25,8 +25,9 @@ __device__ __forceinline__ double wave_sum(double v) {
 // mode 1: out = SF .* Kx              (SF: the W^1/2 of the factored B)
 // mode 2: out = R - DL - S^2 .* Kx     (Laplace residual of (I + W K) d = r, x = DL)
 // mode 3: out = X1 - sigma^2 x - Kx    (VB residual of (sigma^2 I + K) w = rhs, rhs in X1)
-// mode 4: out = Kx / W within [0, K_ii] (K_ii where W = 0): diag of (K^-1 + W)^-1
-//         from the row sums of K o C
+// mode 4: out = Kx / W within [0, K_ii], or K_ii - Kx where W <= 0: diag of
+//         (K^-1 + W)^-1 from the row sums of K o C, or the squares of
+//         k_sigma_squares
 // (modes >= 10: the same with the matrix C in place of K)
 __device__ __forceinline__ void gemv_epilogue(const Prob& P, int i, const double* x, int os,
                                               int mode, double sum) {
@@ -44,8 +45,10 @@ __device__ __forceinline__ void gemv_epilogue(const Prob& P, int i, const double
       break;
     }
     case 4: {
-      const double W = vslot(P, V_W)[i];
-      v = i >= P.N ? 0.0 : W > 0.0 ? fmin(fmax(sum / W, 0.0), P.variance) : P.variance;
+      const double W = vslot(P, V_W)[i], kii = P.variance;
+      v = W > 0.0 ? sum / W : kii - sum;
+      if (W > 0.0) v = v < 0.0 ? 0.0 : v > kii ? kii : v;  // (a NaN stays one)
+      if (i >= P.N) v = 0.0;
       break;
     }
     default: {
