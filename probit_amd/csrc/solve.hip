@@ -1144,7 +1144,7 @@ void launch_trsm(const Batch& bt, int prec, int maxMp, hipStream_t s) {
         hipLaunchKernelGGL(kernel, dim3(tot), dim3(NTHREADS), 0, s, dp, ss, ct0, bt.ticket, ep);
       };
       if (prec == PGP_PREC_FP64)
-        go(k_trsm_rows<double, false>);
+        narrow ? go(k_trsm_rows<double, false>) : go(k_trsm_rows<double, true>);
       else
         narrow ? go(k_trsm_rows<float, false>) : go(k_trsm_rows<float, true>);
     });

@@ -94,3 +94,39 @@ def test_published_values_are_cleared_with_a_new_state(N):
     gp.predict(X, (theta, lp), w, torch.full((N,), lp[0] ** -2.0, dtype=torch.float64))
     Np = (N + 63) // 64 * 64
     assert not bool(ws[-16 * Np:].any())
+
+
+# FP64 solves of 5 to 15 and of 16 and more column tiles in one launch against
+# a launch per block row and per super-step (PGP_TRSM_WAVEFRONT=0), which take
+# the sums off the right-hand side in the same groups: the same bits
+_WIDE_FP64 = """
+import hashlib
+import numpy as np
+import probit_amd as P
+from tests.helpers import make_prior, small_problem
+for N in (64, 300, 1111):
+    X, y, theta, lp, _ = small_problem(N, N, 2, "probit")
+    gp = P.LaplaceGP(data=(X, y), prior=make_prior("EQ"),
+                     log_likelihood=P.log_probit_likelihood)
+    w, p = gp.approximate_posterior((theta, lp))
+    for M in (257, 960, 961, 2000):
+        out = gp.predict(np.random.default_rng(M).normal(size=(M, 2)), (theta, lp), w, p)
+        print("H", N, M, *(hashlib.md5(t.cpu().numpy().tobytes()).hexdigest() for t in out))
+"""
+
+
+def test_wide_fp64_solves_agree_with_the_launch_schedules():
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+    root = Path(__file__).resolve().parent.parent
+    out = []
+    for on in ("0", "1"):
+        r = subprocess.run([sys.executable, "-c", _WIDE_FP64], cwd=root, capture_output=True,
+                           text=True, timeout=100,
+                           env={**os.environ, "PGP_TRSM_WAVEFRONT": on,
+                                "PYTHONPATH": str(root)})
+        assert r.returncode == 0, r.stderr
+        out.append([ln for ln in r.stdout.splitlines() if ln.startswith("H ")])
+    assert len(out[0]) == 12 and out[0] == out[1]
