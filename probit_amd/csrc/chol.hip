@@ -24,6 +24,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "chol_schedule.hpp"
 #include "mfma.hpp"
 #include "pgp_internal.hpp"
 
@@ -651,10 +652,6 @@ __device__ __forceinline__ void column_tile(int t, int w, int& ti, int& tj) {
 // Outer update closing a super-step [s0, s_end): every lower tile (i, j),
 // s_end <= j <= i, j < s_end + wd, gets A_ij -= sum_{c in [s0, s_end)} L_ic
 // L_jc^T.
-__host__ __device__ __forceinline__ int outer_tiles64(int Tk, int wd) {
-  const int w = wd < Tk ? wd : Tk;
-  return w * Tk - w * (w - 1) / 2;
-}
 template <typename T, int BF16, int FUSE>
 __global__ __launch_bounds__(NTHREADS) void k_syrk_outer(Prob* const* probs, Sched sc, int s0,
                                                          int s_end, int wd) {
@@ -714,10 +711,9 @@ struct Outer128<float, 1> {
   static constexpr int OP = 128 * P;
 };
 
-// 128-tiles of a lower triangle of tb block rows
-__host__ __device__ __forceinline__ int tiles128(int tb) {
-  const int t = (tb + 1) / 2;
-  return tb > 0 ? t * (t + 1) / 2 : 0;
+template <typename T, int BF16>
+constexpr OuterOp outer_op() {
+  return std::is_same<T, double>::value ? OUTER_FP64 : BF16 ? OUTER_BF16 : OUTER_FP32;
 }
 
 // Tile bx (blocked_tile's order) of the lower triangle from block row and
@@ -927,14 +923,7 @@ __device__ __forceinline__ void outer128_tile(const Prob& P, int bx, int s0, int
   }
 }
 
-// The outer update closing a super-step [s0, s_end) (as k_syrk_outer), or
-// (wd > 0) its first wd block columns and, of the triangle right of them, all
-// but the last `rest` tiles.
-__host__ __device__ __forceinline__ int outer_tiles128(int tb, int wd, int rest) {
-  if (wd == 0) return tiles128(tb);
-  const int a = tiles128(tb), t = tiles128(tb - wd);
-  return a - t + (t > rest ? t - rest : 0);
-}
+// The outer update closing a super-step [s0, s_end) in outer_tiles128's tiles.
 template <typename T, int BF16>
 __global__ __launch_bounds__(NTHREADS, 2) void k_syrk_outer128(Prob* const* probs, Sched sc,
                                                                int s0, int s_end, int wd) {
@@ -953,21 +942,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_syrk_outer128(Prob* const* prob
     }
   }
   outer128_tile<T, BF16>(P, bx, s0, s_end, base, wd, lds);
-}
-
-// Whether an outer update of t128 128-tiles takes them, or the 64-tiles.  Two
-// workgroups of 128-tiles fit a CU, and a CU given one more than its
-// neighbours keeps the launch waiting for a whole tile (K = 512 FP64: 73 us
-// for one, 133 for two), four times a 64-tile's.  Measured, 128- against
-// 64-tiles: FP64 (K = 512) 210 tiles 79 / 93 us, 300 132 / 121, 406 133 / 164,
-// 528 200 / 207, 1176 335 / 424; FP32 (K = 768) 210 64 / 69, 351 109 / 101,
-// 528 160 / 148, 741 163 / 196; 78 tiles (of 24 block rows) 74 / 50 FP64.
-// BF16 is bound by C's bytes and the operands', not by the tile's MFMAs: 210
-// 15 / 23, 300 24 / 29, 528 34 / 47.
-static bool outer_wide(long long t128, bool bf16) {
-  constexpr int CUS = 256;
-  if (bf16) return t128 >= 3 * CUS / 4;
-  return t128 >= 5 * CUS / 2 || (t128 >= 3 * CUS / 4 && t128 <= CUS);
 }
 
 // BF16 copy of the panel columns [s0, s_end) of the rows below the
@@ -1213,7 +1187,6 @@ constexpr int MAXG = 16;
 // Evidence and gradient 18.6 -> 16.4 ms; prior draw N = 12288 14.4 -> 13.7;
 // FP32 posterior N = 8192 38.4 -> 35.1 (with tiles handed out by ticket, not
 // in runs per XCD, only 37.6: a tile then took 80 us, not 60).
-constexpr int LOOKB = 64;  // members of a launch with outer tiles
 struct StepSched {
   int32_t count;             // members (sorted by size, descending)
   int32_t s0, s1;            // columns [s0, s1)
@@ -1847,24 +1820,6 @@ static void rows_launch(const Batch& b, int s0, int s1, bool tpa, hipStream_t s)
       });
 }
 
-// Outer tiles that a super-step's launch takes along, one workgroup a CU, in
-// the CUs that its `chain` workgroups on the column chain and its `rows` rows
-// below leave idle, and how many of them go before the rows (first).  The
-// chain lasts `all` tiles' times (in tenths; FP64 100 us for 6 columns, 60 a
-// tile of K = 384; FP32 175 for 12, 65 of K = 768; BF16 100 for 8, 13 of K =
-// 512; both grow with G).  A row below takes about as long as the chain if it
-// starts with it, waiting most of the time, and less once the chain has got
-// ahead: few rows start with it, many after the first rounds of tiles.  Many
-// FP32 rows, two a CU without outer tiles, take none (N = 16384, 244 rows: 334
-// us with 240 tiles, 194 without and 51 for the tiles).
-template <typename T, int BF16>
-static int look_tiles(int chain, int rows, int& first) {
-  constexpr int all = sizeof(T) == 8 ? 20 : BF16 ? 80 : 28;
-  constexpr int head = BF16 ? 30 : 10;
-  if (sizeof(T) == 4 && !BF16 && rows > 160) return first = 0;
-  first = rows <= 96 ? 0 : std::max(0, head * (256 - chain) / 10);
-  return first + (all - (first > 0 ? head : 0)) * (256 - chain - rows) / 10;
-}
 template <typename T, int BF16>
 static void superstep_launch(const Batch& b, int s0, int s1, int rlim, int p0, int rest, bool tpa,
                              hipStream_t s) {
@@ -1906,7 +1861,7 @@ static void superstep_launch(const Batch& b, int s0, int s1, int rlim, int p0, i
       ss.opre[std::min(n, LOOKB)] = 0;
     }
     const int nouter = ss.opre[std::min(n, LOOKB)];
-    look_tiles<T, BF16>(ss.gbase[ncols], ss.pre[n], ss.ofirst);
+    look_tiles(outer_op<T, BF16>(), ss.gbase[ncols], ss.pre[n], ss.ofirst);
     ss.ofirst = std::min(ss.ofirst, nouter);
     // with outer tiles one workgroup a CU: a second one would slow the chain's
     const int lds = nouter > 0 && sizeof(T) == 4 ? 8192 : 0;
@@ -1970,6 +1925,7 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
     for (int m = 0; m < b.count; ++m) w += std::max(0, b.np(m) / TILE - s0);
     return w <= column_max;
   };
+  auto nb_of = [&](int m) { return b.np(m) / TILE; };
   // rest >= 0: all but the last `rest` 128-tiles of each member's triangle from
   // the next super-step's end on, which go into that super-step's launch
   auto outer_launch = [&](int s0, int s_end, bool fuse, int rest) {
@@ -1987,13 +1943,8 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
     auto tiles64_of = [&](int m) {
       return outer_tiles64(std::max(0, b.np(m) / TILE - s_end), wd > 0 ? wd : nb);
     };
-    long long t128 = 0;
-    bool more = false;  // than the columns
-    for (int m = 0; m < b.count; ++m) {
-      t128 += tiles128_of(m);
-      more |= wd > 0 && tiles128(b.np(m) / TILE - s_end - wd) > rest;
-    }
-    const bool wide = more || (!fuse && wd % 2 == 0 && outer_wide(t128, BF16 != 0));
+    const bool wide =
+        !fuse && outer_takes_wide(outer_op<T, BF16>(), b.count, nb_of, s_end, wd, rest);
     auto tiles = [&](int m) { return wide ? tiles128_of(m) : tiles64_of(m); };
     sched_launch(b, tiles, [&](Prob* const* dp, const Sched& sc, int n) {
       if (tsy) timer_begin(TC_SYRK, s);
@@ -2041,11 +1992,6 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
     hipLaunchKernelGGL(k_factor_first<T>, dim3(1, b.count), dim3(NTHREADS), 0, s, b.dprobs);
     if (tpa) timer_end(TC_PANEL, s, b.count * F3, 0.0);
   }
-  auto rows_of = [&](int k) {  // row blocks from k on
-    int w = 0;
-    for (int m = 0; m < b.count; ++m) w += std::max(0, b.np(m) / TILE - k);
-    return w;
-  };
   int ahead = -1;  // tiles of the last outer update left to the next super-step (-1: none)
   for (int k = 0; k < nb; ++k) {
     const int s0 = k / G * G, s_end = s0 + G;
@@ -2066,13 +2012,9 @@ static void potrf_steps(const Batch& b, hipStream_t s, const pgp_tune_entry_t& t
         column_launch<T, BF16>(b, k, s0, tpa, s);
       }
       if (outer && s_end < nb) {
-        ahead = -1;
-        int first;
-        if (te.column_merge == 2 && b.count <= LOOKB && s_end + G < nb)
-          ahead = look_tiles<T, BF16>(rows_of(s_end) - rows_of(s_end + G), rows_of(s_end + G),
-                                      first) /
-                  b.count;
-        if (ahead <= 0 || G % 2 != 0) ahead = -1;
+        ahead = te.column_merge == 2
+                    ? outer_ahead(outer_op<T, BF16>(), b.count, nb_of, s_end, G)
+                    : -1;
         outer_launch(s0, s_end, false, ahead);
       }
       continue;
