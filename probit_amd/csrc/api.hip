@@ -445,7 +445,6 @@ static Batch single_batch(char* ws, int Np) {
 static void factor(const Batch& b, int prec, int vb, hipStream_t s, int rs = -1) {
   launch_form_B(b, (prec << 8) | vb, s, rs);
   launch_potrf(b, prec, s);
-  launch_dinv(b, prec, s);
 }
 
 static void solve_B(const Batch& b, int prec, hipStream_t s) {

@@ -527,13 +527,8 @@ __device__ __forceinline__ void syrk_tile_multi(T* A_, int ld_, int kc0, int kc1
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
         const int k = kb + 4 * q;
-        if constexpr (BF16) {
-          da[m * PITCH + k] = f2bf((float)ra[q]);
-          db[m * PITCH + k] = f2bf((float)rb[q]);
-        } else {
-          da[k * PITCH + m] = ra[q];
-          db[k * PITCH + m] = rb[q];
-        }
+        da[k * PITCH + m] = ra[q];
+        db[k * PITCH + m] = rb[q];
       }
     }
   };
@@ -972,20 +967,12 @@ __global__ __launch_bounds__(NTHREADS) void k_panel_bf16(Prob* const* probs, Sch
 // computed as the trailing updates are (T / BF16 operands on MFMA, result
 // rounded to T), then held in LDS as FP64: out[r][c] (kmajor = false) or
 // out[c][r] (kmajor = true).  `arena` holds the operands first.
-// COH: the operand columns were written in this launch by other workgroups
-// (merged column kernel): they are read with coherent loads, and `hook(c)`
-// (called by every thread before column c's operands are fetched) waits
-// for them.  The arithmetic is the same either way.
-struct NoHook {
-  __device__ void operator()(int) const {}
-};
 // SAME: the diagonal tile (ri == rj), whose two operand rows are the same:
 // fetched and staged once.
-template <typename T, int BF16, typename OT, bool SAME = false, bool COH = false,
-          typename Hook = NoHook>
-__device__ __forceinline__ void update_tile_to_lds(const T* A_, int64_t ld, int kc0, int kc1, int64_t ri,
-                                   int64_t rj, char* arena, OT* out, int opitch, bool kmajor,
-                                   Hook hook = Hook()) {
+template <typename T, int BF16, typename OT, bool SAME = false>
+__device__ __forceinline__ void update_tile_to_lds(const T* A_, int64_t ld, int kc0, int kc1,
+                                                   int64_t ri, int64_t rj, char* arena, OT* out,
+                                                   int opitch, bool kmajor) {
   auto A = gbl(A_);
   constexpr bool MM = MmajorF32<T, BF16>::value;
   constexpr int PITCH = BF16 ? 72 : MM ? 68 : KP<T>::value;
@@ -999,18 +986,12 @@ __device__ __forceinline__ void update_tile_to_lds(const T* A_, int64_t ld, int 
   if (kc1 > kc0) {
     T ra[16], rb[16];
     auto fetch = [&](int c) {
-      hook(c);
       const int64_t c0 = (int64_t)c * TILE;
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
         const int k = operand_k<MM>(kb, q);
-        if constexpr (COH) {
-          ra[q] = ld_coh(&A[(size_t)(ri + m) + (size_t)(c0 + k) * ld]);
-          if constexpr (!SAME) rb[q] = ld_coh(&A[(size_t)(rj + m) + (size_t)(c0 + k) * ld]);
-        } else {
-          ra[q] = A[(size_t)(ri + m) + (size_t)(c0 + k) * ld];
-          if constexpr (!SAME) rb[q] = A[(size_t)(rj + m) + (size_t)(c0 + k) * ld];
-        }
+        ra[q] = A[(size_t)(ri + m) + (size_t)(c0 + k) * ld];
+        if constexpr (!SAME) rb[q] = A[(size_t)(rj + m) + (size_t)(c0 + k) * ld];
       }
     };
     fetch(kc0);
@@ -1302,8 +1283,8 @@ struct StepArena {
 };
 
 template <typename T, int BF16>
-__global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(Prob* const* probs, StepSched ss,
-                                                        uint32_t* ticket, uint32_t epoch) {
+__global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
+    Prob* const* probs, StepSched ss, uint32_t* ticket, uint32_t epoch) {
   __shared__ __attribute__((aligned(16))) char arena[StepArena<T, BF16>::bytes];
   __shared__ int s_val;
   // the outer tiles wait for nothing: no ticket, and a run of tiles per XCD
@@ -1525,12 +1506,12 @@ __global__ __launch_bounds__(NTHREADS, sizeof(T) == 8 ? 1 : 2) void k_superstep(
       }
     } else {
 #pragma unroll
-    for (int bm = 0; bm < 2; ++bm)
+      for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
-      for (int bn = 0; bn < 2; ++bn)
+        for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          blk[acc_row<T>(bm, r)][acc_col(bn)] = (double)(T)accd[bm][bn][r];
+          for (int r = 0; r < 4; ++r)
+            blk[acc_row<T>(bm, r)][acc_col(bn)] = (double)(T)accd[bm][bn][r];
     }
     __syncthreads();
 #pragma unroll
@@ -2111,14 +2092,6 @@ void launch_potrf(const Batch& b, int prec, hipStream_t s) {
   if (b.hm) small.hm = b.hm + k;
   potrf_class(big, prec, s);
   potrf_class(small, prec, s);
-}
-
-// The factorisation leaves DINV in place; kept as a no-op entry for callers
-// that re-factor through launch_potrf.
-void launch_dinv(const Batch& b, int prec, hipStream_t s) {
-  (void)b;
-  (void)prec;
-  (void)s;
 }
 
 template <typename T, int BF16>

@@ -261,18 +261,11 @@ __device__ __forceinline__ double column_sums(double (&v)[16]) {
 __device__ __forceinline__ double ld_coherent(const double* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void st_coherent(double* p, double v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // The same for factor values in the storage type (float or double), through
 // the global address space.
 template <typename T>
 __device__ __forceinline__ T ld_coh(const __attribute__((address_space(1))) T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void st_coh(T* p, T v) {
-  __hip_atomic_store(gbl(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // This wave's outstanding global stores (and loads) complete; also a
 // compiler barrier for memory.
@@ -370,7 +363,6 @@ void launch_potrf(const Batch& b, int prec, hipStream_t s);
 int tune_class_of(int np);
 pgp_tune_entry_t tune_get(int prec, int cls);
 void tune_set(int prec, int cls, const pgp_tune_entry_t& v);
-void launch_dinv(const Batch& b, int prec, hipStream_t s);
 int launch_potrf_raw(int prec, void* A, int64_t N, int64_t ld, double* dinv, double* logdiag,
                      int32_t* info, hipStream_t s);
 
