@@ -536,7 +536,8 @@ def main():
 
     # Rooflines over the timed region from the library's HIP-event timers:
     # the dominant kernel (the merged column kernel of the Cholesky,
-    # k_superstep) and the outer trailing update.  achieved = algorithmic
+    # k_superstep) and the outer trailing update (k_syrk_outer, in 64- or
+    # 128-tiles).  achieved = algorithmic
     # flops per launch / average launch duration; traffic = this run's
     # algorithmic bytes per launch x the HBM bytes per algorithmic byte that
     # the committed FETCH_SIZE / WRITE_SIZE runs (copy-calibrated) measured

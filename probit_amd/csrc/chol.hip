@@ -1146,7 +1146,9 @@ __global__ __launch_bounds__(NTHREADS) void k_column(Prob* const* probs, Sched r
 // hand-offs through memory and 33 us (FP64) / 29 us (FP32) of a lone N = 512
 // factor; with one per row block 14.3 us (FP32) and 18 us (FP64, to 29 us in
 // the last columns of 8, where the left-looking products are the longer
-// side): 287 -> 164 us and 217 -> 114 us for the eight columns.
+// side): 287 -> 164 us and 217 -> 114 us for the eight columns.  Super-steps of
+// six, the zeros of the panel product and half the diagonal update left out:
+// 15.8 us a column of an FP64 factor at N = 1537.
 //
 // Member sync words (Prob::csync, zeroed when the descriptor is written with
 // reset): flag (i, c) at csync[(c - s0) MAXG + i - s0] holds the launch's

@@ -448,10 +448,10 @@ int launch_trsv_raw_dinv(int prec, const void* L, int64_t N, int64_t ld, const d
 
 // ---- TRSM: S <- L^-1 S, S is Np x Mp (ld lds) ----
 // With a ticket counter and up to ROWS_MAX block rows a solve is one wavefront
-// launch (k_trsm_rows, below), in FP32 with the roundings of the schedule its
-// width would take without: a launch per block row (up to TRSM_WIDE column
-// tiles) or per super-step of G block rows, which subtract each block row's
-// (super-step's) product from S.
+// launch (k_trsm_rows, below) with the roundings of the schedule its width would
+// take without: a launch per block row (up to TRSM_WIDE column tiles) or per
+// super-step of G block rows, which subtract each block row's (super-step's)
+// product from S.
 //
 // Per block row (lagged).
 // Lagged schedule.  Launch k, workgroup (w, ct), row block i = k + w:
@@ -623,13 +623,17 @@ static void solve_launches(const Batch& bt, int maxMp, hipStream_t s, Go go) {
 // launches, whose solving workgroups run 30 tile products in a row; 1712 in
 // one wavefront launch; 1207 (38 TFLOP/s) with the operands fetched a product
 // ahead; 1110 (41) with DINV's zeros left out and X_i stored by whole columns
-// (256 test points, FP32, a stream of fits: 68.5 -> 65.8 ms).  N = 1537, M = 501: 590 -> 269 us.  Transposed, FP32 at N = 8192, M =
-// 4096: 20.3 ms in 16 launches of 4 column tiles, 2.8 ms (98 TFLOP/s) in one.
+// (256 test points, FP32, a stream of fits: 68.5 -> 65.8 ms); 1061 (43) with
+// the sums taken off in groups and so S_i fetched first.  N = 1537, M = 501: 590
+// -> 269 -> 181 us.  Transposed, FP32 at N = 8192, M = 4096: 20.3 ms in 16
+// launches of 4 column tiles, 2.8 ms (98 TFLOP/s) in one.
 //
 // GRP: the sum is taken off S_i, in its type, after every 1 << lg blocks but
 // the last whole group before i's own: the roundings of the schedules of one
-// launch per block row (lg = 0) or super-step of TRSM_G (lg = 2), which FP32
-// solves of more than WAVE_NCT column tiles follow without a ticket counter.
+// launch per block row (lg = 0) or super-step of TRSM_G (lg = 2), which solves
+// of more than WAVE_NCT column tiles follow without a ticket counter.  A row's
+// whole sum taken off at once is less accurate (FP64, N = 3000, M = 5000:
+// 2.6e-13 from 64-bit references, grouped 1.1e-13).
 // lg goes by the member's own column tiles (up to WAVE_NCT: no group is ever
 // whole), so that its results do not depend on the rest of the batch.
 constexpr int WAVE_NCT = 4;
